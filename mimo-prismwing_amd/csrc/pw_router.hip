@@ -150,6 +150,184 @@ __global__ __launch_bounds__(256) void router_scores_kernel(const TX *__restrict
     }
 }
 
+// The same scores for many rows, in the same declared order, as a contraction on the matrix cores:
+// v_mfma_f32_16x16x1 multiplies 16 rows by 16 experts for one column of each of four column groups
+// and adds the products to four separate accumulators, each with the rounding of one fused
+// multiply-add, so a chain of sixteen of them at hidden 4096 is the partial sums of four column groups
+// of every (row, expert) of the tile. Bound: the kernel above re-reads eight rows per expert from L2
+// (4.7 GB at 2048 rows x 256 experts, 270 us); a 16 x 16 tile reads an eighth of that, and runs within
+// about twice the matrix cores' time for the 2.1 G products (27 us).
+//
+// Work item: 16 rows x 16 experts. Wave v takes the column groups g = 64 v .. 64 v + 63 (its quarter of
+// the declared order) in quads: groups l, l + 1, l + 2, l + 3 of each of the four runs l + {0, 32, 16,
+// 48}, run r in the MFMA's block r, so the first two levels of the halving tree (offsets 32 and 16) are
+// sums of a lane's own accumulators, and the later ones (8, 4, 2, 1) are sums of earlier quads'
+// results that the lane still holds. A quad's columns of one 2048-column pass (64 contiguous bf16
+// bytes per row and run) go straight from global memory into the wave's own LDS, the next step's
+// while this step's are multiplied (no barrier before the end); their 16-byte units are XOR-swizzled
+// by row, so the operand reads (16 rows of one unit) spread over the banks.
+template <typename T>
+struct RsTile {
+    static constexpr uint32_t EPU = 16 / sizeof(T);       // values per 16-byte unit
+    static constexpr uint32_t U = 4 * 8 / EPU;            // units of a quad's 32 columns, per row and run
+    static constexpr uint32_t UNITS = 4 * 16 * U;         // units of a step: four runs, 16 rows
+    static constexpr uint32_t RPC = 64 / U, CPR = 16 / RPC; // rows per 64-lane copy, copies per run
+    static constexpr uint32_t JU = U / 4;                 // units of one group's eight columns
+    __device__ __forceinline__ static uint32_t swizzle(uint32_t row) { return U == 4 ? (row >> 1) & 3 : row & 7; }
+    // the lane's source offsets (values) within the tile's rows; rows past the last reread it
+    __device__ __forceinline__ static void offsets(uint32_t (&off)[CPR], uint32_t row0, uint32_t n_rows, uint32_t K,
+                                                   uint32_t lane)
+    {
+#pragma unroll
+        for (uint32_t c = 0; c < CPR; ++c) {
+            const uint32_t r = RPC * c + lane / U, left = n_rows - 1 - row0;
+            off[c] = (r < left ? r : left) * K + ((lane % U) ^ swizzle(r)) * EPU;
+        }
+    }
+    // a step's columns of the tile's rows (src: the first row at the step's first column) -> LDS
+    // [run][row][unit]
+    __device__ __forceinline__ static void copy(const T *src, const uint32_t (&off)[CPR], uint4 *lds)
+    {
+#pragma unroll
+        for (uint32_t run = 0; run < 4; ++run)
+#pragma unroll
+            for (uint32_t c = 0; c < CPR; ++c)
+                lds_load16(src + off[c] + 8 * (run == 1 ? 32 : run == 2 ? 16 : run == 3 ? 48 : 0),
+                           lds + (run * CPR + c) * 64);
+    }
+    // the units of this lane's row (lane % 16) and run (lane / 16) for group j of the quad
+    __device__ __forceinline__ static void read(const uint4 *lds, uint32_t lane, uint32_t j, uint4 (&q)[JU])
+    {
+        const uint32_t r = lane & 15;
+#pragma unroll
+        for (uint32_t i = 0; i < JU; ++i)
+            q[i] = lds[lane * U + ((JU * j + i) ^ swizzle(r))];
+    }
+    __device__ __forceinline__ static float value(const uint4 (&q)[JU], int c)
+    {
+        const uint4 &u = q[c / EPU];
+        if constexpr (JU == 1) {
+            const uint32_t d[4] = {u.x, u.y, u.z, u.w};
+            return f32_from(c & 1 ? d[c >> 1] & 0xffff0000u : d[c >> 1] << 16);
+        } else {
+            const uint32_t d[4] = {u.x, u.y, u.z, u.w};
+            return f32_from(d[c & 3]);
+        }
+    }
+};
+
+template <typename TX, typename TW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TX) + sizeof(TW) == 4 ? 3 : 2))) void router_scores_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w,
+                                                                 uint32_t rows, uint32_t E, uint32_t K,
+                                                                 float *__restrict__ scores)
+{
+    using X = RsTile<TX>;
+    using W = RsTile<TW>;
+    constexpr uint32_t STEP = X::UNITS + W::UNITS;  // 16-byte units of one step
+    extern __shared__ uint4 lds_rs[];               // per wave one step; then [4][256] wave sums
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t n_et = (E + 15) >> 4, n_rt = (rows + 15) >> 4;
+    // workgroup i runs on XCD i % 8: with eight row tiles or more, an XCD takes whole row tiles, so
+    // each L2 holds the router's weights and its own rows (fewer: row tiles over all XCDs)
+    uint32_t rt, et;
+    if (n_rt >= 8) {
+        const uint32_t j = blockIdx.x >> 3;
+        rt = (blockIdx.x & 7) + 8 * (j / n_et);
+        et = j % n_et;
+    } else {
+        rt = blockIdx.x / n_et;
+        et = blockIdx.x % n_et;
+    }
+    if (rt >= n_rt)
+        return;
+    uint4 *buf = lds_rs + wave * STEP;
+    const uint32_t passes = K >> 11;
+    uint32_t xo[X::CPR], wo[W::CPR];
+    X::offsets(xo, rt * 16, rows, K, lane);
+    W::offsets(wo, et * 16, E, K, lane);
+    const TX *xb = x + (size_t)rt * 16 * K + 512 * wave;
+    const TW *wb = w + (size_t)et * 16 * K + 512 * wave;
+    X::copy(xb, xo, buf);
+    W::copy(wb, wo, buf + X::UNITS);
+    // the halving tree after offsets 32 and 16, group l = 4 quad + j of the sixteen: offset 8 adds
+    // quad 2 to quad 0 and quad 3 to quad 1 (the order they run in), offset 4 the second sum to the
+    // first, offsets 2 and 1 groups within the quad
+    f32x4 part[2][4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t quad = 2 * (k & 1) + (k >> 1), next = 2 * ((k + 1) & 1) + ((k + 1) >> 1);
+        f32x16 acc[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                acc[j][i] = 0.0f;
+        uint32_t p = 0;
+#pragma unroll 1
+        do {
+            // the step's columns are in LDS; its operands into registers, then the next step's copies
+            // overwrite the buffer while this step is multiplied
+            wait_vmcnt<0>();
+            asm volatile("" ::: "memory");
+            uint4 xq[4][X::JU], wq[4][W::JU];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                X::read(buf, lane, j, xq[j]);
+                W::read(buf + X::UNITS, lane, j, wq[j]);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const bool last = p + 1 == passes;
+            if (k < 3 || !last) {
+                const uint32_t col = last ? 32 * next : 32 * quad + 2048 * (p + 1);
+                X::copy(xb + col, xo, buf);
+                W::copy(wb + col, wo, buf + X::UNITS);
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x1f32(X::value(xq[j], c), W::value(wq[j], c), acc[j], 0, 0,
+                                                                  0);
+                __builtin_amdgcn_sched_barrier(0);  // the widened values stay a column at a time
+            }
+        } while (++p < passes);  // K is a positive multiple of 2048
+        // lane: rows 4 (lane / 16) + i, expert lane % 16; acc[j][4 r + i]: run r (offsets 0, 32, 16, 48)
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float v = (acc[j][i] + acc[j][4 + i]) + (acc[j][8 + i] + acc[j][12 + i]);
+                part[k >> 1][j][i] = (k & 1) == 0 ? v : part[k >> 1][j][i] + v;
+            }
+        // formed here: left to itself the compiler keeps all four quads' accumulators (in scratch
+        // memory) and adds them at the end
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+            asm volatile("" : "+v"(part[k >> 1][j]));
+    }
+    f32x4 sum;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            t[j] = part[0][j][i] + part[1][j][i];
+        sum[i] = (t[0] + t[2]) + (t[1] + t[3]);
+    }
+    __syncthreads();  // every wave is done with its steps
+    float *sums = (float *)lds_rs;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        sums[wave * 256 + (4 * (lane >> 4) + i) * 16 + (lane & 15)] = sum[i];
+    __syncthreads();
+    const uint32_t row = rt * 16 + (tid >> 4), e = et * 16 + (tid & 15);
+    if (row < rows && e < E) {
+        const float logit = (sums[tid] + sums[256 + tid]) + (sums[512 + tid] + sums[768 + tid]);
+        scores[(size_t)row * E + e] = sigmoid_pytorch(logit);
+    }
+}
+
 // One wave per row: the row's corrected scores stay in the wave's registers (position p = 64 c +
 // lane in register c), select_route_row runs the top-8 partition on them (pw_select_wave.h), and
 // lane 0 writes the row. A row that fails (non-finite score or bias, a broken top-k, invalid
@@ -187,10 +365,25 @@ __global__ __launch_bounds__(64) void router_select_kernel(const float *__restri
         atomicAdd(tie_rows, 1u);
 }
 
+// The tile kernel runs from this many 16 x 16 tiles on (half the CUs): a tile is a chain of 16 to 32
+// memory round trips (about 15 us at hidden 4096), which fewer tiles do not repay. Scores and
+// selection, us, row kernel / tile kernel: 100 rows x 256 experts 30.8 / 31.1, 128 rows 33.9 / 30.7,
+// 2048 rows 209.5 / 75.6; hidden 2048, 64 experts: 200 rows 18.6 / 17.9, 512 rows 23.9 / 20.4.
+constexpr uint32_t ROUTER_TILES = 128;
+
 template <typename TX, typename TW>
 static void launch_scores_xw(const TX *x, const TW *w, uint32_t rows, uint32_t E, uint32_t K, float *scores,
                              hipStream_t stream)
 {
+    const uint32_t n_et = (E + 15) / 16, n_rt = (rows + 15) / 16;
+    if (K % 2048 == 0 && n_et * n_rt >= ROUTER_TILES) {
+        const uint32_t tiles = n_rt >= 8 ? 8 * ((n_rt + 7) / 8) * n_et : n_rt * n_et;
+        constexpr size_t lds = (size_t)4 * (RsTile<TX>::UNITS + RsTile<TW>::UNITS) * 16;
+        static_assert(lds <= 65536, "the default LDS limit");
+        hipLaunchKernelGGL((router_scores_tile_kernel<TX, TW>), dim3(tiles), dim3(256), lds, stream, x, w, rows, E, K,
+                           scores);
+        return;
+    }
     const dim3 grid(E, (rows + 7) / 8), block(256);
     if (rows == 1) hipLaunchKernelGGL((router_scores_kernel<TX, TW, 1>), grid, block, 0, stream, x, w, rows, E, K, scores);
     else if (rows == 2) hipLaunchKernelGGL((router_scores_kernel<TX, TW, 2>), grid, block, 0, stream, x, w, rows, E, K, scores);

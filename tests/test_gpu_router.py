@@ -368,3 +368,30 @@ def test_routed_layer_rejects_zero_route_weights(rt):
         assert (fi == experts).all() and (ti == experts).all()
         assert not np.any(fw) and not np.any(tw)
         assert not np.any(fo.view(np.uint32)) and not np.any(to.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,experts,hidden,x_f32,w_f32", [
+    (128, 256, 4096, False, False), (129, 250, 2048, False, True), (257, 113, 6144, True, False),
+    (500, 64, 2048, True, True), (2050, 9, 4096, False, False)])
+def test_device_scores_tiles_bit_exact(rt, rows, experts, hidden, x_f32, w_f32):
+    """The 16 x 16 tile form of the scores (from 128 tiles on): partial last row and expert tiles, one,
+    two and three 2048-column passes, every input type, a subnormal and a huge row; the declared order
+    bit for bit."""
+    import torch
+    rng = np.random.default_rng(rows + experts)
+    x = rng.standard_normal((rows, hidden)).astype(np.float32)
+    x[1] *= 1e-39
+    x[2] *= 1e30
+    rw = (rng.standard_normal((experts, hidden)) * 0.02).astype(np.float32)
+    if not x_f32:
+        x = WL.bf16_round_np(x)
+    if not w_f32:
+        rw = WL.bf16_round_np(rw)
+    bias = rng.uniform(-0.01, 0.01, experts).astype(np.float32)
+    ids, wts, scores, ties, flags = _device_route(rt, torch, x, rw, bias, x_f32=x_f32, w_f32=w_f32)
+    _, ref_scores, ref_sel, ref_w, ref_ties = O.route(x, rw, bias)
+    assert flags == 0
+    assert np.array_equal(scores.view(np.uint32), ref_scores.view(np.uint32))
+    assert np.array_equal(ids, ref_sel)
+    assert np.array_equal(wts.view(np.uint32), ref_w.view(np.uint32))
+    assert ties == ref_ties
