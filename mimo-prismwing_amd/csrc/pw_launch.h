@@ -63,8 +63,8 @@ struct MoeBuffers {
     uint16_t *x_planes;        // [3][rows][H]        mode A f32 activations as bf16 planes
     float *y;                  // [rows * 8 * H]
     ActiveExpert *active;      // [E]   per routed expert: weights, placement slots
-    ActiveExpert *pieces;      // [rows * 8] decode batches (<= 8 rows): the routed experts' slots
-                               // in pieces of at most four rows, for the projections
+    ActiveExpert *pieces;      // [rows * 8] decode batches: the routed experts' slots in entries of
+                               // at most moe_piece_rows rows, for the projections
     float *partial;            // split-K partial sums of the mode A projections
     uint8_t *xq;               // [rows * H]      mode B activation codes
     float *xs;                 // [rows * H/128]  mode B activation scales
@@ -190,9 +190,9 @@ struct MoeBArgs {
     uint32_t *flags;
     RouteJob job;                // gate/up only: run in ROUTE_JOB_WGS extra workgroups
 };
-// Whether both launches below take hidden H, intermediate I and `cap` rows per expert: K a
-// multiple of 1024 with K/1024 a power of two (gate/up: up to 4; down: up to 16, more than 4
-// only for a lone expert), R a multiple of 16, at most 16 rows per expert whose codes fit LDS.
+// Whether the gate/up launch below (a lone expert: both launches) takes hidden H, intermediate I
+// and `cap` rows per expert: K a multiple of 1024 with K/1024 a power of two (gate/up: up to 4;
+// down: up to 16), R a multiple of 16, at most 16 rows per expert whose codes fit LDS.
 bool moe_b_fused_shapes(uint32_t H, uint32_t I, uint32_t cap, bool single);
 bool launch_moe_b_gateup_fused(const MoeBArgs &args, uint32_t max_active, hipStream_t stream);
 // Returns the K shares it launched with (0: nothing launched). One share: the rounded expert outputs
@@ -261,8 +261,11 @@ struct QuantJob {
 // false: the caller launches both itself. With `quantised` non-null, a decode batch's one-wave
 // schedule also quantises `quant` (in other workgroups of its launch); *quantised tells whether
 // `quant` was done by either path.
+// piece_rows: the batch's projections take mb.pieces, entries of at most that many slots
+// (moe_piece_rows of the layer that follows; 0: no pieces; batches of at most 128 rows).
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows);
 bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const float *weights,
-                         uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb,
+                         uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb, uint32_t piece_rows,
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles = nullptr,
                          const QuantJob *quant = nullptr, bool *quantised = nullptr);
 // expert_offsets [E + 1]: expert e's placement slots are [off[e], off[e + 1]) (after a schedule).
@@ -299,7 +302,8 @@ void launch_router_select(const float *scores, const float *bias, uint32_t rows,
 // (launch_moe_layer's job) or as launch_route_weights.
 bool launch_route_set_schedule(const float *scores, const float *bias, const ExpertPtrs *bank, uint32_t rows,
                                uint32_t E, uint32_t max_active, uint32_t *set_ids, const MoeBuffers &mb,
-                               uint32_t *flags, hipStream_t stream, const QuantJob *quant = nullptr);
+                               uint32_t piece_rows, uint32_t *flags, hipStream_t stream,
+                               const QuantJob *quant = nullptr);
 void launch_route_weights(const RouteJob &job, hipStream_t stream);
 // The expert sets alone (row_expert_set: one wave per row) into set_ids [rows][8], rows <= 8.
 void launch_route_set(const float *scores, const float *bias, uint32_t rows, uint32_t E, uint32_t *set_ids,

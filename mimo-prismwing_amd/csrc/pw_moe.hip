@@ -93,12 +93,31 @@ __device__ __forceinline__ void place_route_row(const RouteRow &rr, uint32_t p, 
     }
 }
 
+// The schedule of a decode batch also cuts every routed expert's slots into entries of at most this many
+// rows, with their token rows, for the projections (see launch_a_moe and launch_b_fused).
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows)
+{
+    if (mode != 0)
+        return rows <= 8 ? 4u : 8u;  // mode B takes pieces for experts of more than 16 rows only
+    return x_f32 ? 3u : 4u;
+}
+constexpr uint32_t PIECE_MAX_ROWS = 8;
+
+// At most this many entries of piece_rows rows: one per routed expert and one for every further
+// piece_rows of its slots.
+static uint32_t piece_bound(uint32_t rows, uint32_t max_active, uint32_t piece_rows)
+{
+    const uint32_t P = rows * 8, U = max_active < P ? max_active : P;
+    return U + (P - U) / piece_rows;
+}
+
 __global__ __launch_bounds__(1024) void moe_schedule_kernel(
     const ExpertPtrs *__restrict__ bank, const uint32_t *__restrict__ ids,
     const float *__restrict__ weights, uint32_t rows, uint32_t E, uint32_t max_active, uint32_t with_prefix,
     MoePlan *plan, uint32_t *__restrict__ active_expert, uint32_t *__restrict__ active_offset,
     ActiveExpert *__restrict__ active, uint32_t *__restrict__ placement_pos, float *__restrict__ placement_w,
-    uint32_t *__restrict__ row_slots, uint32_t *flags)
+    uint32_t *__restrict__ row_slots, ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t piece_rows,
+    uint32_t *flags)
 {
     extern __shared__ uint32_t lds[];
     const uint32_t words = (rows + 31) >> 5;
@@ -185,6 +204,41 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
     }
     if (tid == 0)
         active_offset[n_active] = total;
+    if (max_pieces) {  // (uniform) the projections' entries of at most piece_rows slots
+        const uint32_t np = (c + piece_rows - 1) / piece_rows;
+        uint32_t n_pieces;
+        const uint32_t pbase = block_exclusive_scan(np, s_scan, &n_pieces);
+        uint32_t w = 0, bits = np ? mask[e * words] : 0u;
+        for (uint32_t i = 0; i < np; ++i) {
+            uint32_t tw[PIECE_MAX_ROWS / 2] = {};
+#pragma unroll
+            for (uint32_t k = 0; k < PIECE_MAX_ROWS; ++k) {
+                if (k < piece_rows) {
+                    while (!bits && w + 1 < words)
+                        bits = mask[e * words + ++w];
+                    const uint32_t t = bits ? w * 32 + __builtin_ctz(bits) : 0u;
+                    tw[k >> 1] |= t << (16 * (k & 1));
+                    bits &= bits - 1;
+                }
+            }
+            if (pbase + i < max_pieces) {
+                const uint32_t left = c - i * piece_rows;
+                u32x4 *dst = (u32x4 *)(pieces + pbase + i);
+                dst[0] = ep0;
+                dst[1] = ep1;
+                dst[2] = ep2;
+                dst[3] = u32x4{off + i * piece_rows, left < piece_rows ? left : piece_rows, tw[0], tw[1]};
+                dst[4] = u32x4{tw[2], tw[3], 0u, 0u};
+                dst[5] = u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+        for (uint32_t a = n_pieces + tid; a < max_pieces; a += nthr) {
+            u32x4 *dst = (u32x4 *)(pieces + a);
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+                dst[i] = u32x4{0u, 0u, 0u, 0u};
+        }
+    }
     // entries past the last routed expert: cnt = 0, the projection workgroups exit at once
     for (uint32_t a = n_active + tid; a < max_active; a += nthr) {
         uint4 *dst = (uint4 *)(active + a);
@@ -516,9 +570,6 @@ void launch_expert_offsets(const MoeBuffers &mb, uint32_t E, uint32_t *expert_of
                        mb.active_expert, mb.active_offset, E, expert_offsets);
 }
 
-// Rows per projection entry when the one-wave schedule cuts experts into pieces.
-constexpr uint32_t PIECE_ROWS = 4;
-
 // The schedule of a decode batch runs in one wave (moe_schedule_wave_kernel) under these bounds.
 static bool wave_schedule(uint32_t rows, uint32_t E, uint32_t max_active)
 {
@@ -559,7 +610,7 @@ __device__ __forceinline__ void schedule_wave_body(
     uint32_t id, float w, uint32_t rows, uint32_t E, uint32_t max_active, const u32x4 *lds_bank, SchedWaveLds &lds,
     MoePlan *plan, uint32_t *__restrict__ active_expert, uint32_t *__restrict__ active_offset,
     ActiveExpert *__restrict__ active, uint32_t *__restrict__ placement_pos, float *__restrict__ placement_w,
-    uint32_t *__restrict__ row_slots, ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t *flags)
+    uint32_t *__restrict__ row_slots, ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t piece_rows, uint32_t *flags)
 {
     uint32_t *bitmap = lds.bitmap, *expert_of = lds.expert_of, *rows_of = lds.rows_of;
     uint16_t *tok_of = lds.tok_of;
@@ -643,22 +694,22 @@ __device__ __forceinline__ void schedule_wave_body(
     }
     if (lane == 0)
         active_offset[U] = total;
-    // the projections' entries: each routed expert's slots in pieces of at most PIECE_ROWS, so
-    // their LDS stages are sized for that many rows (see launch_a_moe); a piece carries its slots'
-    // token rows (slots 0..15 of an expert: PIECE_ROWS * pieces <= 16 here)
-    const uint32_t np = (c_a + PIECE_ROWS - 1) / PIECE_ROWS;  // 0 past the routed experts
+    // the projections' entries: each routed expert's slots in pieces of at most piece_rows (up to
+    // four here), so their LDS stages are sized for that many rows (see launch_a_moe); a piece
+    // carries its slots' token rows (of an expert's at most eight)
+    const uint32_t np = (c_a + piece_rows - 1) / piece_rows;  // 0 past the routed experts
     const uint32_t pincl = wave_inclusive_scan(np);
     const uint32_t pbase = pincl - np, npieces = __builtin_amdgcn_readlane(pincl, 63);
     for (uint32_t i = 0; i < np; ++i) {
         if (pbase + i < max_pieces) {
-            const uint32_t left = c_a - i * PIECE_ROWS;
-            const uint32_t pc = left < PIECE_ROWS ? left : PIECE_ROWS;
-            const uint16_t *tk = tok_of + a * 16 + i * PIECE_ROWS;
+            const uint32_t left = c_a - i * piece_rows;
+            const uint32_t pc = left < piece_rows ? left : piece_rows;
+            const uint16_t *tk = tok_of + a * 16 + i * piece_rows;
             u32x4 *dst = (u32x4 *)(pieces + pbase + i);
             dst[0] = ep0;
             dst[1] = ep1;
             dst[2] = ep2;
-            dst[3] = u32x4{off_a + i * PIECE_ROWS, pc, (uint32_t)tk[0] | ((uint32_t)tk[1] << 16),
+            dst[3] = u32x4{off_a + i * piece_rows, pc, (uint32_t)tk[0] | ((uint32_t)tk[1] << 16),
                            (uint32_t)tk[2] | ((uint32_t)tk[3] << 16)};
             dst[4] = u32x4{0u, 0u, 0u, 0u};
             dst[5] = u32x4{0u, 0u, 0u, 0u};
@@ -698,7 +749,7 @@ __global__ __launch_bounds__(64) void moe_schedule_wave_kernel(
     uint32_t rows, uint32_t E, uint32_t max_active, MoePlan *plan, uint32_t *__restrict__ active_expert,
     uint32_t *__restrict__ active_offset, ActiveExpert *__restrict__ active, uint32_t *__restrict__ placement_pos,
     float *__restrict__ placement_w, uint32_t *__restrict__ row_slots, ActiveExpert *__restrict__ pieces,
-    uint32_t max_pieces, uint32_t *flags, const QuantJob qj)
+    uint32_t max_pieces, uint32_t piece_rows, uint32_t *flags, const QuantJob qj)
 {
     extern __shared__ u32x4 lds_bank[];  // the bank's ExpertPtrs table, E x 48 bytes
     __shared__ SchedWaveLds sl;
@@ -729,7 +780,7 @@ __global__ __launch_bounds__(64) void moe_schedule_wave_kernel(
             lds_load16((const u32x4 *)bank + u0 + lane, lds_bank + u0);
     __builtin_amdgcn_s_waitcnt(0);  // the table copy has landed in LDS (and the routes are in)
     schedule_wave_body(id, w, rows, E, max_active, lds_bank, sl, plan, active_expert, active_offset, active,
-                       placement_pos, placement_w, row_slots, pieces, max_pieces, flags);
+                       placement_pos, placement_w, row_slots, pieces, max_pieces, piece_rows, flags);
 }
 
 // Row p's eight experts into ids[0..7] by one wave: fast_top8_set (ascending ids), or where that
@@ -783,7 +834,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     uint32_t rows, uint32_t E, uint32_t max_active, uint32_t *__restrict__ set_ids, MoePlan *plan,
     uint32_t *__restrict__ active_expert, uint32_t *__restrict__ active_offset, ActiveExpert *__restrict__ active,
     uint32_t *__restrict__ placement_pos, float *__restrict__ placement_w, uint32_t *__restrict__ row_slots,
-    ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t *flags, const QuantJob qj)
+    ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t piece_rows, uint32_t *flags, const QuantJob qj)
 {
     extern __shared__ u32x4 lds_bank[];  // the bank's ExpertPtrs table, E x 48 bytes
     __shared__ TopkEntry pairs[8][64 * NC];
@@ -817,12 +868,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     if (lane < P)
         set_ids[lane] = id;
     schedule_wave_body(id, 0.0f, rows, E, max_active, lds_bank, sl, plan, active_expert, active_offset, active,
-                       placement_pos, placement_w, row_slots, pieces, max_pieces, flags);
+                       placement_pos, placement_w, row_slots, pieces, max_pieces, piece_rows, flags);
 }
 
 bool launch_route_set_schedule(const float *scores, const float *bias, const ExpertPtrs *bank, uint32_t rows,
                                uint32_t E, uint32_t max_active, uint32_t *set_ids, const MoeBuffers &mb,
-                               uint32_t *flags, hipStream_t stream, const QuantJob *quant)
+                               uint32_t piece_rows, uint32_t *flags, hipStream_t stream, const QuantJob *quant)
 {
     if (rows < 1 || rows > 8 || E < 9 || E > 256 || max_active > 64)
         return false;
@@ -833,7 +884,8 @@ bool launch_route_set_schedule(const float *scores, const float *bias, const Exp
 #define PW_RSS(NC)                                                                                                 \
     hipLaunchKernelGGL(route_set_schedule_kernel<NC>, dim3(1 + quant_wgs), dim3(512), table, stream, scores, bias,  \
                        bank, rows, E, max_active, set_ids, mb.plan, mb.active_expert, mb.active_offset, mb.active,  \
-                       mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, rows * 8, flags, qj)
+                       mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, piece_bound(rows, max_active, piece_rows),         \
+                       piece_rows, flags, qj)
     if (E <= 64) PW_RSS(1);
     else if (E <= 128) PW_RSS(2);
     else PW_RSS(4);
@@ -857,29 +909,6 @@ void launch_route_weights(const RouteJob &job, hipStream_t stream)
     if (job.E <= 64) hipLaunchKernelGGL(route_weights_kernel<1>, dim3(job.rows), dim3(64), 0, stream, job);
     else if (job.E <= 128) hipLaunchKernelGGL(route_weights_kernel<2>, dim3(job.rows), dim3(64), 0, stream, job);
     else hipLaunchKernelGGL(route_weights_kernel<4>, dim3(job.rows), dim3(64), 0, stream, job);
-}
-
-// --------------------------------------------------------------- shared tile preamble
-struct ExpertTile {
-    ExpertPtrs ep;
-    uint32_t off;    // first placement slot of this expert
-    uint32_t cnt;    // placements of this expert
-    bool live;
-};
-
-__device__ __forceinline__ ExpertTile expert_tile(const MoePlan *plan, const uint32_t *active_expert,
-                                                  const uint32_t *active_offset, const ExpertPtrs *bank,
-                                                  uint32_t a)
-{
-    ExpertTile t;
-    t.live = a < plan->n_active;
-    if (!t.live)
-        return t;
-    const uint32_t e = active_expert[a];
-    t.off = active_offset[a];
-    t.cnt = active_offset[a + 1] - t.off;
-    t.ep = bank[e];
-    return t;
 }
 
 // Deterministic cross-wave sum (wave order 0..KSPLIT-1) of NT x f32x4 per lane, result in wave 0.
@@ -910,9 +939,7 @@ __device__ __forceinline__ void reduce_waves(f32x4 (*red)[NT][64], f32x4 *v, int
 // (kernels/block_fp8_gemv.metal:139-160, :935-1046; fused twin :1048-1186).
 template <int KSPLIT, int NT>
 __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
-    const ExpertPtrs *__restrict__ bank, const MoePlan *__restrict__ plan,
-    const uint32_t *__restrict__ active_expert, const uint32_t *__restrict__ active_offset,
-    const uint32_t *__restrict__ placement_pos, const uint8_t *__restrict__ xq,
+    const ActiveExpert *__restrict__ entries, const uint32_t *__restrict__ placement_pos, const uint8_t *__restrict__ xq,
     const float *__restrict__ xs, uint32_t rows, uint32_t H, uint32_t I, float *__restrict__ hidden,
     uint32_t *flags)
 {
@@ -924,8 +951,8 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
     // XCD x (workgroup i runs on XCD i % 8) takes a contiguous eighth of each expert's row tiles
     const uint32_t a = blockIdx.x / tiles_per_expert, lt = blockIdx.x % tiles_per_expert;
     const uint32_t rt = tiles_per_expert % 8 == 0 ? (lt % 8) * (tiles_per_expert / 8) + lt / 8 : lt;
-    const ExpertTile et = expert_tile(plan, active_expert, active_offset, bank, a);
-    if (!et.live)
+    const ActiveExpert et = load_entry(entries, a);
+    if (et.cnt == 0)
         return;
     if (et.cnt > 16u * NT) {
         if (threadIdx.x == 0)
@@ -1011,9 +1038,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
 // ------------------------------------------------------------------ mode B, down projection
 template <int KSPLIT, int NT>
 __global__ __launch_bounds__(64 * KSPLIT) void moe_b_down_kernel(
-    const ExpertPtrs *__restrict__ bank, const MoePlan *__restrict__ plan,
-    const uint32_t *__restrict__ active_expert, const uint32_t *__restrict__ active_offset,
-    const uint8_t *__restrict__ hq, const float *__restrict__ hs, uint32_t H, uint32_t I,
+    const ActiveExpert *__restrict__ entries, const uint8_t *__restrict__ hq, const float *__restrict__ hs, uint32_t H, uint32_t I,
     float *__restrict__ y, uint32_t *flags)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1021,8 +1046,8 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_down_kernel(
     __shared__ f32x4 red[KSPLIT][NT][64];
     const uint32_t tiles_per_expert = H >> 4;
     const uint32_t a = blockIdx.x / tiles_per_expert, rt = blockIdx.x % tiles_per_expert;
-    const ExpertTile et = expert_tile(plan, active_expert, active_offset, bank, a);
-    if (!et.live || et.cnt > 16u * NT)
+    const ActiveExpert et = load_entry(entries, a);
+    if (et.cnt == 0 || et.cnt > 16u * NT)
         return;
     const uint32_t row0 = rt << 4;
     const uint32_t blocks = I >> 7;
@@ -1223,10 +1248,11 @@ __global__ __launch_bounds__(256) void round_output_kernel(const float *__restri
 
 // ------------------------------------------------------------------------------- launchers
 bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const float *weights,
-                         uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb,
+                         uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb, uint32_t piece_rows,
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles, const QuantJob *quant,
                          bool *quantised)
 {
+    const uint32_t max_pieces = piece_rows ? piece_bound(rows, max_active, piece_rows) : 0u;
     bool long_batch = false;
     if (quantised)
         *quantised = false;
@@ -1250,14 +1276,16 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
         const uint32_t quant_wgs = (qj.rows * (qj.K >> 7) + 3) / 4;
         hipLaunchKernelGGL(moe_schedule_wave_kernel, dim3(1 + quant_wgs), dim3(64), table, stream, bank, ids, weights,
                            rows, E, max_active, mb.plan, mb.active_expert, mb.active_offset, mb.active,
-                           mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, rows * 8, flags, qj);
+                           mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces,
+                           piece_rows ? piece_rows : 1u, flags, qj);
         if (quant_wgs)
             *quantised = true;
     }
     else if (rows <= SCHED_WG_MAX_ROWS)
         hipLaunchKernelGGL(moe_schedule_kernel, dim3(1), dim3(1024), lds, stream, bank, ids, weights, rows,
                            E, max_active, with_prefix, mb.plan, mb.active_expert, mb.active_offset, mb.active,
-                           mb.placement_pos, mb.placement_w, mb.row_slots, flags);
+                           mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces,
+                           piece_rows ? piece_rows : 1u, flags);
     else {
         // rows <= 4096 (SCHED_MAX_WORDS words) and E <= 1024 (one plan thread per expert)
         const SchedScratch ss = sched_carve(mb.sched, rows, E, nullptr);
@@ -1295,15 +1323,27 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
                               const OneTokenRoutes *routes = nullptr, const RouteJob *job = nullptr,
                               bool *job_done = nullptr)
 {
-    const int nt = max_count > 16 ? 2 : 1;
-    const uint32_t cnt = max_count < 16u * nt ? max_count : 16u * nt;
+    // A routed batch runs both projections on the schedule's pieces of each expert's slots, so their
+    // LDS stages hold piece_rows rows instead of as many as the batch could send one expert (an
+    // expert with more rows reads its weights once per piece, from the caches; every slot's
+    // arithmetic is unchanged). Uniform and skewed routes give most experts one to three rows. The
+    // down's stage of four rows (25 KB at hidden 4096) leaves its 98 VGPRs to set its occupancy,
+    // four workgroups per CU (width 8: 90 -> 83 us); the fused gate/up fits two workgroups per CU
+    // with four bf16 rows or three f32 ones (three planes each). 19 f32 rows with skewed routes: the
+    // layer 542 -> 388 us against stages of 19 rows (split-K gate/up with partials through memory,
+    // down in four K splits).
+    const uint32_t piece_rows = moe_piece_rows(0, x_f32, rows);
+    const bool pieces = !one && max_count > piece_rows;
+    const uint32_t entries = pieces ? piece_bound(rows, max_active, piece_rows) : max_active;
+    const int nt = !pieces && max_count > 16 ? 2 : 1;
+    const uint32_t cnt = pieces ? piece_rows : (max_count < 16u * nt ? max_count : 16u * nt);
     const uint16_t *xp = (const uint16_t *)x;
     if (x_f32) {
         launch_split_planes((const float *)x, rows * H, mb.x_planes, stream);
         xp = mb.x_planes;
     }
     SplitArgs ga{};
-    ga.active = mb.active;
+    ga.active = pieces ? mb.pieces : mb.active;
     ga.placement_pos = mb.placement_pos;
     ga.x = xp;
     ga.x_plane = (size_t)rows * H;
@@ -1327,26 +1367,16 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     const SplitPlan gp = plan_split(H, 2, x_f32 ? 3 : 1, cnt);
     ga.KS = gp.ks;
     int t = timer_begin(K_MOE_GATEUP, stream);
-    // the one-wave schedule also cut every routed expert's slots into entries of at most
-    // PIECE_ROWS rows (with their token rows): a decode batch gives most experts one to three
-    // rows, and LDS stages sized for four rows let more workgroups share a CU (an expert with more
-    // rows reads its weights once per piece; every slot's arithmetic is unchanged)
-    const bool pieces = !one && cnt > PIECE_ROWS && wave_schedule(rows, mb.experts, max_active);
     SplitArgs gp_args = ga;
-    if (pieces && !x_f32) {
-        gp_args.active = mb.pieces;
-        gp_args.cap = PIECE_ROWS;
-    }
     // the route weights (job) ride in extra workgroups of a launch that runs anyway: the split-K
     // down's (about 1 us there against about 4 us in the gate/up launch, whose workgroups are
     // longer), or the fused gate/up's where the down is the one-token down+combine
     const bool job_in_down = job && !direct;
     if (job && !job_in_down)
         gp_args.job = *job;
-    const bool fused = nt == 1 && launch_moe_a_gateup_fused(x_f32 ? 3 : 1, gp_args, pieces && !x_f32 ? placements
-                                                            : max_active, mb.hidden_planes, stream);
+    const bool fused = nt == 1 && launch_moe_a_gateup_fused(x_f32 ? 3 : 1, gp_args, entries, mb.hidden_planes, stream);
     if (!fused)
-        launch_moe_a_split(2, x_f32 ? 3 : 1, nt, ga, gp, max_active, stream);
+        launch_moe_a_split(2, x_f32 ? 3 : 1, nt, ga, gp, entries, stream);
     timer_end(t, stream);
     if (!fused) {
         t = timer_begin(K_MOE_SWIGLU, stream);
@@ -1366,13 +1396,6 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     da.K = I;
     da.R = H;
     da.rows = placements;
-    // down in pieces: a four-row LDS stage (25 KB at hidden 4096) leaves the kernel's 98 VGPRs
-    // (four waves per SIMD) to set its occupancy, four workgroups per CU instead of three at eight
-    // rows
-    if (pieces) {
-        da.active = mb.pieces;
-        da.cap = PIECE_ROWS;
-    }
     t = timer_begin(K_MOE_DOWN, stream);
     // one expert: the whole-K down writes the rounded output rows itself; a one-token batch: down
     // and combine in one launch
@@ -1382,13 +1405,13 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
         timer_end(t, stream);
         return ExpertOut{nullptr, 0, 0};
     }
-    const SplitPlan dp = plan_split(I, 1, 3, pieces ? PIECE_ROWS : cnt);
+    const SplitPlan dp = plan_split(I, 1, 3, cnt);
     da.KS = dp.ks;
-    if (job_in_down && dp.bpw == 8 && (pieces || nt == 1)) {  // the instantiation compiled with a job
+    if (job_in_down && dp.bpw == 8 && nt == 1) {  // the instantiation compiled with a job
         da.job = *job;
         *job_done = true;
     }
-    launch_moe_a_split(1, 3, pieces ? 1 : nt, da, dp, pieces ? placements : max_active, stream);
+    launch_moe_a_split(1, 3, nt, da, dp, entries, stream);
     if (job_in_down && !*job_done) {  // another down shape: the weights on their own, before the combine
         launch_route_weights(*job, stream);
         *job_done = true;
@@ -1401,16 +1424,15 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
 // activations were quantised into mb.xq / mb.xs: from the schedule's entries, or for the one expert
 // `one` on token rows 0..rows-1. The down writes each expert output rounded to bf16 into y (a lone
 // expert: the output rows, y_bf16 too). False, with nothing launched, when the shapes do not fit.
-static bool launch_b_fused(const ExpertPtrs *bank, const MoeBuffers &mb, const ActiveExpert *one, uint32_t rows,
-                           uint32_t placements,
-                           uint32_t max_active, uint32_t max_count, uint32_t H, uint32_t I, float *y,
+static bool launch_b_fused(const MoeBuffers &mb, const ActiveExpert *entries, const ActiveExpert *one, uint32_t rows,
+                           uint32_t placements, uint32_t max_active, uint32_t max_count, uint32_t H, uint32_t I, float *y,
                            uint16_t *y_bf16, uint32_t *flags, hipStream_t stream, const RouteJob *job = nullptr,
                            bool *job_done = nullptr)
 {
-    if (!moe_b_fused_shapes(H, I, max_count, one != nullptr))  // both launches take the shapes, or neither runs
+    if (!moe_b_fused_shapes(H, I, max_count, one != nullptr))
         return false;
     MoeBArgs ga{};
-    ga.active = mb.active;
+    ga.active = entries;
     ga.codes = mb.xq;
     ga.scales = mb.xs;
     ga.K = H;
@@ -1449,8 +1471,8 @@ static bool launch_b_fused(const ExpertPtrs *bank, const MoeBuffers &mb, const A
     if (one)
         ks = launch_moe_b_down_fused(da, max_active, stream);
     else
-        hipLaunchKernelGGL((moe_b_down_kernel<4, 1>), dim3(max_active * (H >> 4)), dim3(256), 0, stream, bank, mb.plan,
-                           mb.active_expert, mb.active_offset, mb.hq, mb.hs, H, I, mb.y, flags);
+        hipLaunchKernelGGL((moe_b_down_kernel<4, 1>), dim3(max_active * (H >> 4)), dim3(256), 0, stream, entries,
+                           mb.hq, mb.hs, H, I, mb.y, flags);
     timer_end(t, stream);
     if (ks > 1) {
         // the share sums added in share order and rounded (mode B's output is the rounded expert
@@ -1463,20 +1485,18 @@ static bool launch_b_fused(const ExpertPtrs *bank, const MoeBuffers &mb, const A
 }
 
 template <int KS, int NT>
-static void launch_b_moe(const ExpertPtrs *bank, const MoeBuffers &mb, uint32_t rows, uint32_t placements,
+static void launch_b_moe(const MoeBuffers &mb, const ActiveExpert *entries, uint32_t rows, uint32_t placements,
                          uint32_t max_active, uint32_t H, uint32_t I, uint32_t *flags, hipStream_t stream)
 {
     const dim3 g1(max_active * (I >> 4)), g2(max_active * (H >> 4)), blk(64 * KS);
     int t = timer_begin(K_MOE_GATEUP, stream);
-    hipLaunchKernelGGL((moe_b_gateup_kernel<KS, NT>), g1, blk, 0, stream, bank, mb.plan,
-                       mb.active_expert, mb.active_offset, mb.placement_pos, mb.xq, mb.xs, rows, H, I,
-                       mb.hidden, flags);
+    hipLaunchKernelGGL((moe_b_gateup_kernel<KS, NT>), g1, blk, 0, stream, entries, mb.placement_pos, mb.xq, mb.xs,
+                       rows, H, I, mb.hidden, flags);
     timer_end(t, stream);
     // re-quantise the bf16-staged hidden activations per (placement, 128 group)
     launch_quant_group128(mb.hidden, true, placements, I, mb.hq, mb.hs, flags, stream);
     t = timer_begin(K_MOE_DOWN, stream);
-    hipLaunchKernelGGL((moe_b_down_kernel<KS, NT>), g2, blk, 0, stream, bank, mb.plan,
-                       mb.active_expert, mb.active_offset, mb.hq, mb.hs, H, I, mb.y, flags);
+    hipLaunchKernelGGL((moe_b_down_kernel<KS, NT>), g2, blk, 0, stream, entries, mb.hq, mb.hs, H, I, mb.y, flags);
     timer_end(t, stream);
 }
 
@@ -1486,17 +1506,25 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
                                 const DirectOut *direct = nullptr, const OneTokenRoutes *routes = nullptr,
                                 bool x_quantised = false, const RouteJob *job = nullptr, bool *job_done = nullptr)
 {
-    const bool wide = max_count > 16;
     if (mode == 0)
         return launch_a_moe(mb, x, x_f32, rows, placements, max_active, max_count, H, I, flags, stream, nullptr,
                             direct, bank, routes, job, job_done);
     if (!x_quantised)
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
-    if (!wide && launch_b_fused(bank, mb, nullptr, rows, placements, max_active, max_count, H, I, mb.y, nullptr, flags,
-                                stream, job, job_done))
+    // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces; a lone
+    // expert (the one-expert forward) on 32 tokens per workgroup
+    const uint32_t piece_rows = moe_piece_rows(1, x_f32, rows);
+    const bool lone = placements == rows, pieces = !lone && max_count > 16;
+    const ActiveExpert *entries = pieces ? mb.pieces : mb.active;
+    if (pieces) {
+        max_active = piece_bound(rows, max_active, piece_rows);
+        max_count = piece_rows;
+    }
+    if (max_count <= 16 && launch_b_fused(mb, entries, nullptr, rows, placements, max_active, max_count, H, I, mb.y,
+                                          nullptr, flags, stream, job, job_done))
         return ExpertOut{mb.y, 1, 0};
-    if (wide) launch_b_moe<4, 2>(bank, mb, rows, placements, max_active, H, I, flags, stream);
-    else launch_b_moe<4, 1>(bank, mb, rows, placements, max_active, H, I, flags, stream);
+    if (max_count > 16) launch_b_moe<4, 2>(mb, entries, rows, placements, max_active, H, I, flags, stream);
+    else launch_b_moe<4, 1>(mb, entries, rows, placements, max_active, H, I, flags, stream);
     return ExpertOut{mb.y, 1, 0};
 }
 
@@ -1564,7 +1592,7 @@ void launch_expert_forward(uint32_t mode, const ExpertPtrs *bank, const ExpertPt
             for (uint32_t k = 0; k < 16; ++k)
                 one.tok[k] = (uint16_t)k;
             launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
-            if (launch_b_fused(bank, mb, &one, rows, rows, 1, rows, H, I, out_f32, out_bf16, flags, stream))
+            if (launch_b_fused(mb, nullptr, &one, rows, rows, 1, rows, H, I, out_f32, out_bf16, flags, stream))
                 return;
         }
         hipLaunchKernelGGL(moe_single_plan_kernel, dim3(1), dim3(256), 0, stream, bank, expert, rows, mb.plan,

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
 }
 
 // Gate/up over the whole K in one workgroup, SwiGLU fused: the decode fast path when the expert's
-// routed rows fit LDS (NS * cnt <= 8). Work item: (routed expert, 16 weight rows of gate and of
+// routed rows fit LDS (NS * cnt <= 9). Work item: (routed expert, 16 weight rows of gate and of
 // up). Eight waves split K (wave w: blocks [w * BPW, (w + 1) * BPW)), each issuing all of its
 // weight loads at once (the same per-lane stream as the split kernel); the expert's routed
 // activation rows for the whole K go straight into LDS; the eight partial sums meet in LDS and
@@ -440,7 +440,8 @@ bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_activ
                                hipStream_t stream)
 {
     // four 128-column blocks per wave and split (the split kernel's gate/up stream), eight splits
-    if (args.K != 8 * 4 * 128 || args.R % 16 != 0 || (uint32_t)ns * args.cap > 8)
+    // (up to eight bf16 rows or three f32 ones, 74 KB: two workgroups per CU)
+    if (args.K != 8 * 4 * 128 || args.R % 16 != 0 || (uint32_t)ns * args.cap > 9)
         return false;
     const size_t lds = fused_lds(ns, args.cap, args.K);
     // a lone expert (the one-expert forward) and one-row experts (a one-token batch) take 8 + 8-row

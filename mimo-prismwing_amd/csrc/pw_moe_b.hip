@@ -385,7 +385,7 @@ static bool down_fits(uint32_t K, uint32_t R, uint32_t cap, bool single)
 
 bool moe_b_fused_shapes(uint32_t H, uint32_t I, uint32_t cap, bool single)
 {
-    return gateup_fits(H, I, cap) && down_fits(I, H, cap, single);
+    return gateup_fits(H, I, cap) && (!single || down_fits(I, H, cap, single));
 }
 
 bool launch_moe_b_gateup_fused(const MoeBArgs &args, uint32_t max_active, hipStream_t stream)

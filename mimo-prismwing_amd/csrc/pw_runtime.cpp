@@ -1189,7 +1189,8 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
     bool quantised = false;
     pw::launch_moe_schedule((const ExpertPtrs *)rt->bank_table.p, (const uint32_t *)rt->route_ids.p,
                             (const float *)rt->route_w.p, rows, n_experts,
-                            std::min<uint32_t>(n_experts, rows * 8), rt->mb, rt->d_flags, rt->stream, nullptr,
+                            std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, rows),
+                            rt->d_flags, rt->stream, nullptr,
                             mode == PW_MODE_B ? &qj : nullptr, mode == PW_MODE_B ? &quantised : nullptr);
     pw::launch_moe_layer(mode, (const ExpertPtrs *)rt->bank_table.p, rt->mb, rt->in.p, x_f32, rows,
                          std::min<uint32_t>(n_experts, rows * 8), max_count, H, I,
@@ -1328,7 +1329,8 @@ static void launch_routed_layer(const MoeBuffers &mb, const pw_expert_bank *bank
     // mode B: a decode batch's schedule launch also quantises the activations
     const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, mb.xq, mb.xs};
     bool quantised = false;
-    pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E, max_active, mb, flags, s, nullptr,
+    pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E, max_active, mb,
+                            pw::moe_piece_rows(mode, x_f32, rows), flags, s, nullptr,
                             mode == PW_MODE_B ? &qj : nullptr, mode == PW_MODE_B ? &quantised : nullptr);
     pw::launch_moe_layer(mode, bank->table, mb, x, x_f32, rows, max_active, rows, H, I, out_f32, out_bf16, raw, flags,
                          s, nullptr, quantised);
@@ -1395,7 +1397,8 @@ int pw_moe_layer_routed_device(pw_runtime *rt, const pw_expert_bank *bank, uint3
     // mode B: the schedule launch also quantises the activations
     const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
     if (!direct && pw::launch_route_set_schedule(scores, bias, bank->table, rows, E, max_active,
-                                                 (uint32_t *)rt->set_ids.p, rt->mb, rt->d_flags, s,
+                                                 (uint32_t *)rt->set_ids.p, rt->mb,
+                                                 pw::moe_piece_rows(mode, x_f32, rows), rt->d_flags, s,
                                                  mode == PW_MODE_B ? &qj : nullptr)) {
         // the expert sets are scheduled; the routes' order and weights (a serial partition per row)
         // run in extra workgroups of an expert launch (mode A: the down, mode B: the gate/up) while
@@ -1523,7 +1526,7 @@ int pw_moe_prefill_device(pw_runtime *rt, const pw_expert_bank *bank, const void
     const pw::PfTileTable tt{pb.tiles, pb.n_tiles, max_tiles};
     const pw::QuantJob qj{x, x_dtype == PW_DTYPE_F32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
     const bool scheduled_long = pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E,
-                                                        std::min<uint32_t>(E, P), rt->mb, rt->d_flags, s, &tt, &qj);
+                                                        std::min<uint32_t>(E, P), rt->mb, 0, rt->d_flags, s, &tt, &qj);
     pw::launch_moe_prefill(bank->table, rt->mb, pb, x, x_dtype == PW_DTYPE_F32, rows, E, H, I,
                            out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
                            out_dtype == PW_DTYPE_BF16 ? (uint16_t *)output : nullptr,
@@ -1551,7 +1554,7 @@ int pw_moe_schedule_device(pw_runtime *rt, const pw_expert_bank *bank, const uin
     PW_TRY(ensure_sched(rt, rows, E));
     const size_t P = (size_t)rows * 8;
     pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E, std::min<uint32_t>(E, (uint32_t)P),
-                            rt->mb, rt->d_flags, s);
+                            rt->mb, 0, rt->d_flags, s);
     pw::launch_expert_offsets(rt->mb, E, expert_offsets, s);
     PW_HIP(hipMemcpyAsync(positions, rt->mb.placement_pos, P * 4, hipMemcpyDeviceToDevice, s));
     PW_HIP(hipMemcpyAsync(weights, rt->mb.placement_w, P * 4, hipMemcpyDeviceToDevice, s));

@@ -320,6 +320,41 @@ def test_pieces_match_one_workgroup_schedule(rt, full_bank, width):
     check_mode_a(outs[0], ref_raw, moe_condition(x[:width], experts, sel[:width], w[:width]), raw=True)
 
 
+@pytest.mark.parametrize("mode,x_f32", [(P.MODE_A, False), (P.MODE_A, True), (P.MODE_B, False)])
+@pytest.mark.parametrize("rows", [9, 17, 32])
+def test_wide_batch_pieces_equal_small_batches(rt, full_bank, mode, x_f32, rows):
+    """A batch of 9 to 32 rows runs the experts on pieces of their slots (three or four rows in mode A;
+    eight in mode B, for more than sixteen rows). Experts with every row (full pieces and a
+    remainder), with some rows and with one: each row equals, bit for bit, its result in a two-row
+    batch, whose experts need no pieces."""
+    import torch
+    stream = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(rows)
+    x = WL.activations(rows, WL.SEED_BASE + 150 + rows)
+    sel = np.empty((rows, 8), np.uint32)
+    for p in range(rows):
+        rest = rng.permutation(np.arange(16, 256))[:4]
+        sel[p] = rng.permutation(np.concatenate([[3, 9], [0 if p % 2 else 1, 4 + p % 3], rest]))
+    w = rng.uniform(0.01, 0.3, (rows, 8)).astype(np.float32)
+
+    def layer(at):
+        n = len(at)
+        xt = (torch.from_numpy(np.ascontiguousarray(x[at])).cuda() if x_f32
+              else torch.from_numpy(WL.bf16_bits_np(x[at]).view(np.int16)).cuda())
+        ids, wts = torch.from_numpy(sel[at].astype(np.int32)).cuda(), torch.from_numpy(w[at]).cuda()
+        raw = torch.empty((n, 4096), dtype=torch.float32, device="cuda")
+        rt.moe_layer_device(full_bank.bank, xt, n, ids, wts, raw, mode=mode,
+                            x_dtype=P.DTYPE_F32 if x_f32 else P.DTYPE_BF16, out_dtype=P.DTYPE_F32_RAW, stream=stream)
+        torch.cuda.synchronize()
+        assert rt.take_flags() == 0
+        return raw.cpu().numpy()
+
+    whole = layer(np.arange(rows))
+    for p in range(0, rows - 1, 3):
+        at = np.array([p, p + 1])
+        assert np.array_equal(layer(at).view(np.uint32), whole[at].view(np.uint32)), (p, rows)
+
+
 @pytest.mark.parametrize("x_f32", [False, True])
 def test_one_token_equals_two_copies(rt, full_bank, x_f32):
     """Each token's result depends only on its own row and routes: a two-row batch holding the
