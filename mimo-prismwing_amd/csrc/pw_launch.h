@@ -210,20 +210,13 @@ inline void timer_end(int slot, hipStream_t s)
         tl_timer->end(slot, s);
 }
 
-// x: `planes` bf16 planes [planes][W][K] (1: bf16 activations, 3: f32 split by launch_split_planes)
-void launch_linear_a(const ProjTile *tiles, uint32_t n_tiles, const uint16_t *x, int planes,
-                     uint32_t W, uint32_t K, float *y32, uint16_t *y16, uint32_t N,
-                     uint32_t round_f32, hipStream_t stream);
+// f32 [n] -> three bf16 planes [3][n]
 void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream_t stream);
-// Mode A on f32 activation rows [W][K]: one row is split into its planes inside the projection's
-// staging; more rows (or a split whose stage would not fit) go through launch_split_planes into
-// `scratch` ([3][W][K] bf16) first.
-void launch_linear_a_f32(const ProjTile *tiles, uint32_t n_tiles, const float *xf, uint16_t *scratch, uint32_t W,
-                         uint32_t K, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32,
-                         hipStream_t stream);
-void launch_linear_b(const ProjTile *tiles, uint32_t n_tiles, const uint8_t *codes,
-                     const float *scales, uint32_t W, uint32_t K, float *y32, uint16_t *y16,
-                     uint32_t N, uint32_t round_f32, hipStream_t stream);
+// Block-FP8 projection (pw_linear.hip): x [W][K] 16-byte aligned, bf16 or f32 (mode A) or e4m3 codes
+// with x_scales [W][K / 128] (mode B).
+enum WideX : int { WX_BF16 = 0, WX_F32 = 1, WX_CODES = 2 };
+void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
+                   uint32_t K, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream);
 void launch_quant_group128(const void *x, bool x_f32, uint32_t rows, uint32_t K, uint8_t *codes,
                            float *scales, uint32_t *flags, hipStream_t stream);
 

@@ -825,23 +825,22 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
                           hipStream_t stream)
 {
     if (mode == PW_MODE_A) {
-        if (x_f32) {
-            const size_t n = (size_t)rows * p->columns;
-            PW_HIP(rt->lin_planes.ensure(3 * n * 2));
-            pw::launch_linear_a_f32(p->tiles, p->n_tiles, (const float *)x, (uint16_t *)rt->lin_planes.p, rows,
-                                    p->columns, y32, y16, p->rows, round_f32, stream);
-        } else {
-            pw::launch_linear_a(p->tiles, p->n_tiles, (const uint16_t *)x, 1, rows, p->columns, y32, y16,
-                                p->rows, round_f32, stream);
+        if ((uintptr_t)x & 15) {
+            // rows off 16 bytes (a caller's slice): the projection's copies take an aligned one
+            const size_t bytes = (size_t)rows * p->columns * (x_f32 ? 4 : 2);
+            PW_HIP(rt->lin_planes.ensure(bytes));
+            PW_HIP(hipMemcpyAsync(rt->lin_planes.p, x, bytes, hipMemcpyDeviceToDevice, stream));
+            x = rt->lin_planes.p;
         }
+        pw::launch_linear(x_f32 ? pw::WX_F32 : pw::WX_BF16, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, y32,
+                          y16, p->rows, round_f32, stream);
     } else if (mode == PW_MODE_B) {
         PW_HIP(rt->codes.ensure((size_t)rows * p->columns));
         PW_HIP(rt->scales.ensure((size_t)rows * (p->columns / 128) * 4));
         pw::launch_quant_group128(x, x_f32, rows, p->columns, (uint8_t *)rt->codes.p,
                                   (float *)rt->scales.p, rt->d_flags, stream);
-        pw::launch_linear_b(p->tiles, p->n_tiles, (const uint8_t *)rt->codes.p,
-                            (const float *)rt->scales.p, rows, p->columns, y32, y16, p->rows,
-                            round_f32, stream);
+        pw::launch_linear(pw::WX_CODES, p->tiles, p->n_tiles, rt->codes.p, (const float *)rt->scales.p, rows,
+                          p->columns, y32, y16, p->rows, round_f32, stream);
     } else {
         return fail(PW_ERR_ARGUMENT, "unknown mode %u", mode);
     }

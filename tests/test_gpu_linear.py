@@ -118,6 +118,57 @@ def test_mode_a_f32_row_split_in_staging(rt, n, k):
     assert normwise(one, O.gemm_mode_a(w, s, x)) <= (2e-6 if k <= 512 else 1e-5)
 
 
+@pytest.mark.parametrize("n", [24, 4104, 8200, 12296])
+@pytest.mark.parametrize("k", [128, 1152, 3328])
+def test_projection_tile_and_step_edges(rt, n, k):
+    """Every staged-row count (4, 8, 16, 24, 32 rows and one off each), workgroups of one, two and
+    four 16-row tiles with a partial last tile and a partial last workgroup, and waves with no, one,
+    two, three and four steps (1, 9 and 26 blocks over eight waves). Mode A against 64 bits: exact
+    products added in f32 in chains of at most 48 roundings (2e-6). Mode B on integers whose sums are
+    exact in f32 (weights up to 2, codes up to 8 with one 448 a group, so activation scales are 1,
+    block scales powers of two): equal."""
+    rng = np.random.default_rng(n + k)
+    s = log_uniform_scales(rng, n, k)
+    w = fp8_weight(rng, n, k, s)
+    proj = rt.bind_projection(w, s)
+    wd = dequant(w, s).astype(np.float64)
+    xf = rng.standard_normal((32, k)).astype(np.float32)
+    xb = bf16_round(xf)
+    si = np.exp2(rng.integers(-1, 2, s.shape)).astype(np.float32)
+    wi = encode_e4m3(rng.integers(-2, 3, (n, k)).astype(np.float32))
+    xi = rng.integers(-8, 9, (32, k)).astype(np.float32)
+    xi[:, rng.integers(0, 128) :: 128] = 448.0
+    proj_i = rt.bind_projection(wi, si)
+    ref_f, ref_b = xf.astype(np.float64) @ wd.T, xb.astype(np.float64) @ wd.T
+    ref_i = (xi.astype(np.float64) @ dequant(wi, si).astype(np.float64).T).astype(np.float32)
+    for rows in (1, 4, 5, 8, 9, 16, 17, 24, 25, 32):
+        for dt, x, ref in ((P.DTYPE_F32, xf, ref_f), (P.DTYPE_BF16, xb, ref_b)):
+            assert rel_l2(run_device(rt, proj, x[:rows], x_dtype=dt), ref[:rows]) <= 2e-6, (rows, dt)
+        assert np.array_equal(run_device(rt, proj_i, xi[:rows], mode=P.MODE_B, x_dtype=P.DTYPE_F32), ref_i[:rows]), rows
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_mode_a_rows_off_16_bytes(rt, kind):
+    """Activation rows that start off 16 bytes give the bits of aligned ones."""
+    torch = _torch()
+    rng = np.random.default_rng(77)
+    n, k, rows = 200, 512, 5
+    s = log_uniform_scales(rng, n, k)
+    proj = rt.bind_projection(fp8_weight(rng, n, k, s), s)
+    dt, pt = (torch.float32, P.DTYPE_F32) if kind == "f32" else (torch.bfloat16, P.DTYPE_BF16)
+    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).to(dt).cuda()
+    off = torch.empty(rows * k + 1, dtype=dt, device="cuda")[1:].view(rows, k)
+    off.copy_(x)
+    outs = []
+    for t in (x, off):
+        out = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+        rt.fp8_linear_device(proj, t, rows, out, mode=P.MODE_A, x_dtype=pt, out_dtype=P.DTYPE_F32_RAW,
+                             stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
 def test_real_checkpoint_gemv_fixture(rt, golden_dir):
     with open(os.path.join(golden_dir, "mtp-gate-fp8-gemv.json")) as f:
         fx = json.load(f)
