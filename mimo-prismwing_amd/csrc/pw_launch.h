@@ -105,8 +105,6 @@ struct SplitArgs {
     uint32_t cap;                   // routed rows per expert the LDS stage holds
     float *partial;                 // [KS][MATS][P][R]
     uint32_t *flags;
-    uint32_t single;                // 1: one expert on rows 0..rows-1, its entry is `one` (no schedule)
-    ActiveExpert one;
     // One token's routes with no schedule (route_ids non-null): work item a is the token's route a,
     // expert route_ids[a] of the bank's E, on placement slot a (see moe_a_one_token_direct)
     const ExpertPtrs *bank;
@@ -132,8 +130,8 @@ struct SplitPlan {
 // K split of a mode A expert projection (`mats` weight matrices sharing the activations) with K
 // columns, NS activation planes and up to max_cnt routed rows per expert.
 SplitPlan plan_split(uint32_t K, int mats, int ns, uint32_t max_cnt);
-void launch_moe_a_split(int mats, int ns, int nt, const SplitArgs &args, const SplitPlan &sp,
-                        uint32_t max_active, hipStream_t stream);
+void launch_moe_a_split(int mats, int ns, const SplitArgs &args, const SplitPlan &sp, uint32_t max_active,
+                        hipStream_t stream);
 // gate/up split sums -> SwiGLU -> hidden as three bf16 planes [3][P][I]
 // BF16 wide linear (pw_bf16.hip): w bf16 [R][K] (K a multiple of 128), x bf16 planes [NS][W][K],
 // split-K partials [KS][W][R] f32 summed in split order by the reduce kernel.
@@ -153,9 +151,6 @@ void launch_bf16_linear(const Bf16Args &a, int planes, int bpw, float *y32, uint
 
 // Gate/up with the SwiGLU fused and no split partials (pw_moe_a.hip), when the routed rows fit the
 // LDS stage; returns false (nothing launched) otherwise.
-// The one-expert forward's whole-K down projection with the output rounding fused (K = I of 1024
-// or 2048, at most eight rows); false when the shape does not fit it.
-bool launch_moe_a_down_out(const SplitArgs &args, float *out_f32, uint16_t *out_bf16, bool raw, hipStream_t stream);
 // Down and combine of a one-token decode batch in one launch (mode A, I = 2048, eight routed
 // experts; args are the down projection's, whose rows are the eight placement slots): the same
 // arithmetic as the split-K down followed by the combine; false when the batch does not fit it.
@@ -172,33 +167,23 @@ bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_activ
 void launch_moe_a_swiglu(const float *partial, uint32_t ks, uint32_t P, uint32_t I, uint16_t *hidden_planes,
                          uint32_t *flags, hipStream_t stream);
 
-// Mode B whole-K projections of routed experts (pw_moe_b.hip): e4m3 activation codes with per
-// (row, 128-column) scales against the block-FP8 weights. Gate/up reads token rows ae.tok[t] of
-// the codes and writes the bf16-staged SwiGLU to hidden [slots][R]; down reads slot rows
-// ae.off + t and writes each expert output rounded to bf16 at its slot row.
+// Mode B whole-K gate/up of routed experts (pw_moe_b.hip): e4m3 activation codes with per
+// (row, 128-column) scales against the block-FP8 weights; token rows ae.tok[t] of the codes, the
+// bf16-staged SwiGLU to hidden [slots][R].
 struct MoeBArgs {
-    const ActiveExpert *active;  // schedule entries (unused when single)
+    const ActiveExpert *active;  // schedule entries
     const uint8_t *codes;        // activation codes [rows][K]
     const float *scales;         // activation scales [rows][K/128]
     uint32_t K, R, rows, cap;    // columns, weight rows, activation rows, routed rows per expert at most
-    uint32_t single;             // 1: one expert, entry `one` (no schedule)
-    ActiveExpert one;
-    float *out;                  // gate/up: hidden; down: expert outputs (single: the output rows)
-    uint16_t *out_bf16;          // down, single: bf16 output rows (or null)
-    uint32_t KS;                 // down: K shares (set by the launcher)
-    float *partial;              // down with KS > 1: share sums [KS][rows][R]
+    float *out;                  // hidden [slots][R]
     uint32_t *flags;
-    RouteJob job;                // gate/up only: run in ROUTE_JOB_WGS extra workgroups
+    RouteJob job;                // run in ROUTE_JOB_WGS extra workgroups
 };
-// Whether the gate/up launch below (a lone expert: both launches) takes hidden H, intermediate I
-// and `cap` rows per expert: K a multiple of 1024 with K/1024 a power of two (gate/up: up to 4;
-// down: up to 16), R a multiple of 16, at most 16 rows per expert whose codes fit LDS.
-bool moe_b_fused_shapes(uint32_t H, uint32_t I, uint32_t cap, bool single);
+// Whether the launch below takes hidden H, intermediate I and `cap` rows per expert: H a multiple of
+// 1024 with H/1024 a power of two up to 4, I a multiple of 16, at most 16 rows per expert whose codes
+// fit LDS.
+bool moe_b_fused_shapes(uint32_t H, uint32_t I, uint32_t cap);
 bool launch_moe_b_gateup_fused(const MoeBArgs &args, uint32_t max_active, hipStream_t stream);
-// Returns the K shares it launched with (0: nothing launched). One share: the rounded expert outputs
-// are in args.out / args.out_bf16. KS > 1 (a lone expert): the share sums are in args.partial,
-// args.rows * R floats apart, for the output rounding to add in share order.
-uint32_t launch_moe_b_down_fused(const MoeBArgs &args, uint32_t max_active, hipStream_t stream);
 
 // The runtime points this at its timer for the duration of one ABI call (calls on a runtime are
 // serialised by the caller, and each thread has its own pointer).
@@ -217,6 +202,15 @@ void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream
 enum WideX : int { WX_BF16 = 0, WX_F32 = 1, WX_CODES = 2 };
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
                    uint32_t K, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream);
+// One expert on W rows (pw_expert.hip). Gate/up with the SwiGLU: x [W][H] e4m3 codes with x_scales
+// (mode B, hidden bf16-staged), f32 or bf16 (mode A) -> hidden [W][I] f32. Down: x [W][I] codes or f32
+// -> the output rows [W][H] (raw: f32 sums unrounded), or with the K shares it returns above one the
+// share sums partial [KS][W][H] (KS <= 8) for the caller to add in order and round.
+void launch_expert_gateup(const ExpertPtrs &ep, bool codes, bool x_f32, const void *x, const float *x_scales, uint32_t W,
+                          uint32_t H, uint32_t I, float *hidden, uint32_t *flags, hipStream_t stream);
+uint32_t launch_expert_down(const ExpertPtrs &ep, bool codes, const void *x, const float *x_scales, uint32_t W, uint32_t H,
+                            uint32_t I, float *partial, float *out_f32, uint16_t *out_bf16, bool raw, uint32_t *flags,
+                            hipStream_t stream);
 void launch_quant_group128(const void *x, bool x_f32, uint32_t rows, uint32_t K, uint8_t *codes,
                            float *scales, uint32_t *flags, hipStream_t stream);
 
@@ -321,10 +315,9 @@ void launch_moe_prefill(const ExpertPtrs *bank, const MoeBuffers &mb, const Pref
                         bool x_f32, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, float *out_f32,
                         uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream, bool scheduled_long);
 
-void launch_expert_forward(uint32_t mode, const ExpertPtrs *bank, const ExpertPtrs &ep, uint32_t expert,
-                           const MoeBuffers &mb,
-                           const void *x, bool x_f32, uint32_t rows, uint32_t H, uint32_t I,
-                           float *out_f32, uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream);
+void launch_expert_forward(uint32_t mode, const ExpertPtrs &ep, const MoeBuffers &mb, const void *x, bool x_f32,
+                           uint32_t rows, uint32_t H, uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw,
+                           uint32_t *flags, hipStream_t stream);
 
 // Seeded synthetic data for benchmarks and tests (counter-based, reproducible on one device).
 void launch_synth_fp8(uint8_t *w, const float *scales, uint64_t rows, uint64_t cols, uint64_t seed,

@@ -15,363 +15,13 @@
 // the f32 block partial in registers: total += scale * partial. MFMA is used because f32 VALU FMA
 // (no packed math) cannot reach 8 TB/s x 8 rows x 2 FLOP/B.
 //
-// What bounds it: the weights' bytes once, and beside them the activations, which every workgroup
-// reads again from L2. A workgroup of 16 weight rows reads W rows of activations for its 16 rows of
-// weights: at 13 f32 rows 52 bytes a column (78 as three bf16 planes) against 16. Here a workgroup
-// takes 16 RT weight rows over the whole K (pick_rt), its eight waves split K, and each wave streams
-// its blocks two steps deep with no barrier: the step's activation columns go by coalesced
-// direct-to-LDS copies to the wave's own LDS region, the step's weights to registers, and step
-// j + 2 is issued as soon as step j is computed. f32 rows are read as f32 and split in registers,
-// once per step for all RT tiles. The split sums meet in LDS and are added in split order 0..7, so
-// results are deterministic.
 //
-// Measured against one 16-row tile per workgroup with the activations read inside the MFMA loop (us,
-// weights in the memory-side cache): 13800 x 4096 (56.5 MB) with 13 f32 rows, mode A, 46.8 -> 15.7
-// (3.6 TB/s); 13568 x 4096, mode B with its quantiser launch, 8 f32 rows 19.2 -> 14.7; mode A, f32
-// rows, width 1 / 8 / 32 18.7 / 42.2 / 99.4 -> 16.3 / 16.1 / 22.1, bf16 rows 14.5 / 15.4 / 41.8 ->
-// 13.7 / 13.7 / 16.5.
-#include <type_traits>
-
+// The kernel and what bounds it: pw_wide.h.
 #include "pw_device.h"
 #include "pw_launch.h"
+#include "pw_wide.h"
 
 namespace pw {
-
-// ------------------------------------------------------------------------------- projections
-template <int XT>
-struct WideXBytes {
-    static constexpr int value = XT == WX_F32 ? 4 : XT == WX_BF16 ? 2 : 1;
-};
-
-// Columns per step: a block, or half a block where two steps of eight waves would not fit in LDS
-// with whole blocks of f32 rows (24 rows: 196 KB; half blocks 98 KB).
-template <int XT, int XR>
-struct WideStep {
-    static constexpr int value = XT == WX_F32 && XR > 16 ? 64 : 128;
-};
-
-struct WideArgs {
-    const ProjTile *tiles;
-    uint32_t n_tiles;
-    const void *x;         // activations [W][K]: bf16, f32 or e4m3 codes
-    const float *x_scales; // codes: [W][K / 128]
-    uint32_t W, K, N;
-    float *y_f32;
-    uint16_t *y_bf16;
-    uint32_t round_f32;
-};
-
-// Two f32 -> one dword each of their three bf16 planes, by truncation: every remainder is exact, the
-// last has at most eight significant bits, so hi + mid + lo == x as with rounded planes.
-__device__ __forceinline__ void split3_pair(float x0, float x1, uint32_t &hi, uint32_t &mid, uint32_t &lo)
-{
-    const uint32_t b0 = f32_bits(x0), b1 = f32_bits(x1);
-    const float r0 = x0 - f32_from(b0 & 0xffff0000u), r1 = x1 - f32_from(b1 & 0xffff0000u);
-    const uint32_t c0 = f32_bits(r0), c1 = f32_bits(r1);
-    const float s0 = r0 - f32_from(c0 & 0xffff0000u), s1 = r1 - f32_from(c1 & 0xffff0000u);
-    hi = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-    mid = __builtin_amdgcn_perm(c1, c0, 0x07060302u);
-    lo = __builtin_amdgcn_perm(f32_bits(s1), f32_bits(s0), 0x07060302u);
-}
-
-// 16-byte LDS reads of a step slot, waited for in the same block. Written out because the compiler
-// cannot tell the two slots apart: ahead of a plain read of one slot it waits for the direct-to-LDS
-// copies of the other, and with them for every weight load of the next step (vmcnt 0).
-__device__ __forceinline__ uint32_t lds_at(const uint4 *p)
-{
-    return (uint32_t)(size_t)(const __attribute__((address_space(3))) uint4 *)p;
-}
-__device__ __forceinline__ void lds_read(const uint32_t (&a)[1], u32x4 (&v)[1])
-{
-    asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(v[0]) : "v"(a[0]) : "memory");
-}
-__device__ __forceinline__ void lds_read(const uint32_t (&a)[2], u32x4 (&v)[2])
-{
-    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(v[0]), "=&v"(v[1])
-                 : "v"(a[0]), "v"(a[1])
-                 : "memory");
-}
-__device__ __forceinline__ void lds_read(const uint32_t (&a)[4], u32x4 (&v)[4])
-{
-    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
-                 : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3])
-                 : "memory");
-}
-
-template <int XT, int XR, int RT>
-struct WideStream {
-    static constexpr int SC = WideStep<XT, XR>::value;
-    static constexpr int XB = WideXBytes<XT>::value;
-    static constexpr int NT = (XR + 15) / 16;             // 16-token tiles
-    static constexpr int UPR = SC * XB / 16;              // 16-byte units per staged row
-    static constexpr int XC = XR * UPR / 64;              // activation copies per step
-    static constexpr int WL = SC / 64;                    // weight loads per tile and step
-    static constexpr int SLOT = XR * UPR;                 // units per step slot
-    static constexpr int RED = 8 * RT * NT * 64;          // split partials, in the slots' place
-    static constexpr int LDS = 16 * SLOT > RED ? 16 * SLOT : RED;
-    static_assert(XR * UPR % 64 == 0, "whole copies");
-    static_assert(LDS * 16 <= 160 * 1024, "a workgroup's LDS");
-
-    // step columns [col, col + SC) of the activation rows -> LDS (row r's unit u at r * UPR + (u ^ (r & 7)))
-    static __device__ __forceinline__ void copy_x(const char *x, uint32_t W, uint32_t K, uint32_t col, uint4 *slot,
-                                                  int lane)
-    {
-#pragma unroll
-        for (int c = 0; c < XC; ++c) {
-            const uint32_t p = c * 64 + lane, row = p / UPR, u = (p % UPR) ^ (row & 7);
-            const uint32_t r = row < W ? row : W - 1;  // rows past the batch repeat its last row
-            lds_load16(x + ((size_t)r * K + col) * XB + u * 16, slot + c * 64);
-        }
-    }
-
-    // the row of tile nt that lane r16 reads (a tile of fewer than sixteen staged rows repeats them)
-    static __device__ __forceinline__ uint32_t x_row(int nt, int r16)
-    {
-        const int rows = XR - nt * 16 < 16 ? XR - nt * 16 : 16;
-        return nt * 16 + (r16 & (rows - 1));
-    }
-};
-
-template <int XT, int XR, int RT>
-__global__ __launch_bounds__(512, 2) void linear_wide_kernel(const WideArgs args)
-{
-    using S = WideStream<XT, XR, RT>;
-    constexpr int NT = S::NT, SC = S::SC, WL = S::WL, XC = S::XC;
-    __shared__ uint4 lds_w[S::LDS];  // per wave two step slots; then the split partials [8][RT * NT][64]
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int q = lane >> 4, r16 = lane & 15;
-    const uint32_t K = args.K, W = args.W, blocks = K >> 7;
-    const char *x = (const char *)args.x;
-    uint4 *slots = lds_w + (size_t)wave * 2 * S::SLOT;
-
-    // the tiles' descriptors in one round trip: all of them are taken before any address is formed
-    const uint8_t *wt[RT], *wrow[RT];
-    const float *ws[RT];
-    uint32_t valid[RT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r) {
-        const uint32_t t = blockIdx.x * RT + r;
-        const ProjTile *tile = args.tiles + (t < args.n_tiles ? t : args.n_tiles - 1);
-        wt[r] = tile->w;
-        ws[r] = tile->s;
-        valid[r] = tile->valid;
-    }
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-        asm volatile("" ::"s"(wt[r]), "s"(ws[r]), "s"(valid[r]));
-#pragma unroll
-    for (int r = 0; r < RT; ++r)  // rows past the tile repeat its last row (never stored)
-        wrow[r] = wt[r] + (size_t)((uint32_t)r16 < valid[r] ? (uint32_t)r16 : valid[r] - 1) * K +
-                  q * (XT == WX_CODES ? 32 : 16);
-    // this wave's blocks, and its steps
-    const uint32_t b0 = (uint32_t)wave * blocks / 8, b1 = ((uint32_t)wave + 1) * blocks / 8;
-    const uint32_t steps = (b1 - b0) * (128 / SC);
-
-    f32x4 total[RT][NT], acc[RT][NT];
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            total[r][nt] = acc[r][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    u32x4 wv[2][RT][WL];
-    float sw[2][RT], sa[2][NT];
-    // step st into slot s: scales, activation copies, then the weights, in this order in the memory
-    // counter (so the youngest XC + RT * WL loads are the copies and weights of the last step issued)
-    auto issue = [&](auto s_, uint32_t st) __attribute__((always_inline)) {
-        constexpr int s = decltype(s_)::value;
-        const uint32_t col = (b0 << 7) + st * SC, b = col >> 7;
-        if constexpr (XT == WX_CODES) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const uint32_t row = nt * 16 + r16;
-                sa[s][nt] = load_g(args.x_scales + (size_t)(row < W ? row : W - 1) * blocks + b);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-            sw[s][r] = load_g(ws[r] + b);
-        asm volatile("" ::: "memory");
-        S::copy_x(x, W, K, col, slots + s * S::SLOT, lane);
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-            for (int h = 0; h < WL; ++h)
-                wv[s][r][h] = *(global_u32x4 *)(wrow[r] + col + h * (XT == WX_CODES ? 16 : 64));
-        asm volatile("" ::: "memory");
-    };
-    // N loads issued after step s's own may be outstanding
-    auto compute = [&](auto s_, auto n_) __attribute__((always_inline)) {
-        constexpr int s = decltype(s_)::value;
-        wait_vmcnt<decltype(n_)::value>();
-        asm volatile("" ::: "memory");
-#pragma unroll
-        for (int r = 0; r < RT; ++r)  // the weights' conversions stay behind this wait
-#pragma unroll
-            for (int h = 0; h < WL; ++h)
-                asm volatile("" : "+v"(wv[s][r][h]));
-        const uint32_t slot = lds_at(slots + s * S::SLOT);
-        if constexpr (XT == WX_CODES) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const uint32_t row = S::x_row(nt, r16), at = slot + row * S::UPR * 16;
-                const uint32_t ad[2] = {at + ((q * 2) ^ (row & 7)) * 16, at + ((q * 2 + 1) ^ (row & 7)) * 16};
-                u32x4 c[2];
-                lds_read(ad, c);
-                const i32x8 xb = {(int)c[0][0], (int)c[0][1], (int)c[0][2], (int)c[0][3],
-                                  (int)c[1][0], (int)c[1][1], (int)c[1][2], (int)c[1][3]};
-#pragma unroll
-                for (int r = 0; r < RT; ++r) {
-                    const u32x4 w0 = wv[s][r][0], w1 = wv[s][r][WL - 1];
-                    const i32x8 wa = {(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3],
-                                      (int)w1[0], (int)w1[1], (int)w1[2], (int)w1[3]};
-                    const f32x4 p = mfma_fp8_16x16x128(wa, xb, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        total[r][nt][i] = __builtin_fmaf(p[i] * sw[s][r], sa[s][nt], total[r][nt][i]);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int h = 0; h < WL; ++h) {
-                bf16x8 a[RT][2];
-#pragma unroll
-                for (int r = 0; r < RT; ++r) {
-                    a[r][0] = fp8x8_to_bf16x8(wv[s][r][h][0], wv[s][r][h][1]);
-                    a[r][1] = fp8x8_to_bf16x8(wv[s][r][h][2], wv[s][r][h][3]);
-                }
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const uint32_t row = S::x_row(nt, r16), at = slot + row * S::UPR * 16;
-                    constexpr int NP = XT == WX_F32 ? 3 : 1;
-                    u32x4 pl[NP][2];  // the planes of this lane's sixteen columns
-                    if constexpr (XT == WX_BF16) {
-                        const uint32_t ad[2] = {at + ((h * 8 + q * 2) ^ (row & 7)) * 16,
-                                                at + ((h * 8 + q * 2 + 1) ^ (row & 7)) * 16};
-                        lds_read(ad, pl[0]);
-                    } else {
-                        // Of fewer than sixteen staged rows, each is read by G = 16 / XR lanes of a
-                        // DPP row: each splits its share of the sixteen columns, and the first of
-                        // them, whose column of the product is the one stored, takes the others' by
-                        // row shifts (one row of 1000 x 8192: 11.1 -> 9.8 us).
-                        constexpr int G = XR < 16 ? 16 / XR : 1, UG = 4 / G;
-                        uint32_t ad[UG];
-                        u32x4 u[UG];
-#pragma unroll
-                        for (int i = 0; i < UG; ++i)
-                            ad[i] = at + ((h * 16 + q * 4 + (G > 1 ? (r16 / XR) * UG : 0) + i) ^ (row & 7)) * 16;
-                        lds_read(ad, u);
-                        uint32_t own[3][2 * UG];
-#pragma unroll
-                        for (int i = 0; i < 2 * UG; ++i)
-                            split3_pair(f32_from(u[i / 2][(i % 2) * 2]), f32_from(u[i / 2][(i % 2) * 2 + 1]), own[0][i],
-                                        own[1][i], own[2][i]);
-#pragma unroll
-                        for (int p = 0; p < NP; ++p)
-#pragma unroll
-                            for (int i = 0; i < 2 * UG; ++i) {
-                                pl[p][i / 4][i % 4] = own[p][i];
-                                if constexpr (G >= 2)
-                                    pl[p][(2 * UG + i) / 4][(2 * UG + i) % 4] = dpp_u32<0x100 + XR % 16, 0xf>(own[p][i]);
-                                if constexpr (G == 4) {
-                                    pl[p][1][i % 4] = dpp_u32<0x100 + 2 * XR % 16, 0xf>(own[p][i]);
-                                    pl[p][1][(2 + i) % 4] = dpp_u32<0x100 + 3 * XR % 16, 0xf>(own[p][i]);
-                                }
-                            }
-                    }
-#pragma unroll
-                    for (int p = 0; p < NP; ++p) {
-                        const bf16x8 x0 = __builtin_bit_cast(bf16x8, pl[p][0]), x1 = __builtin_bit_cast(bf16x8, pl[p][1]);
-#pragma unroll
-                        for (int r = 0; r < RT; ++r) {
-                            acc[r][nt] = mfma_bf16_16x16x32(a[r][0], x0, acc[r][nt]);
-                            acc[r][nt] = mfma_bf16_16x16x32(a[r][1], x1, acc[r][nt]);
-                        }
-                    }
-                }
-            }
-            if constexpr (SC == 128 || s == 1) {  // a block is complete
-#pragma unroll
-                for (int r = 0; r < RT; ++r)
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            total[r][nt][i] = __builtin_fmaf(sw[s][r], acc[r][nt][i], total[r][nt][i]);
-                        acc[r][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    }
-            }
-        }
-        asm volatile("" ::: "memory");  // the slot's reads stay ahead of its next copies
-    };
-    // two steps in flight; no issue inside a condition, so the wait for one step's weights never
-    // has to assume that the next step's were not issued
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using Next = std::integral_constant<int, XC + RT * WL>;
-    if (steps >= 2) {
-        issue(I0{}, 0);
-        issue(I1{}, 1);
-        uint32_t st = 0;
-        for (; st + 4 <= steps; st += 2) {
-            compute(I0{}, Next{});
-            issue(I0{}, st + 2);
-            compute(I1{}, Next{});
-            issue(I1{}, st + 3);
-        }
-        compute(I0{}, Next{});
-        if (SC == 128 && st + 3 == steps) {
-            issue(I0{}, st + 2);
-            compute(I1{}, Next{});
-            compute(I0{}, I0{});
-        } else {
-            compute(I1{}, I0{});
-        }
-    } else if (steps == 1) {
-        issue(I0{}, 0);
-        compute(I0{}, I0{});
-    }
-
-    // the split partials in LDS over the slots (every wave is past its reads), summed in split order
-    __syncthreads();
-    f32x4 *red = (f32x4 *)lds_w;
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            red[(wave * RT * NT + r * NT + nt) * 64 + lane] = total[r][nt];
-    __syncthreads();
-    if (wave >= RT * NT)
-        return;
-    const uint32_t t = blockIdx.x * RT + wave / NT, token = (wave % NT) * 16 + r16;
-    if (t >= args.n_tiles || token >= W)
-        return;
-    f32x4 sum = red[wave * 64 + lane];
-#pragma unroll
-    for (int w = 1; w < 8; ++w) {
-        const f32x4 o = red[(w * RT * NT + wave) * 64 + lane];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            sum[i] += o[i];
-    }
-    const ProjTile tile = args.tiles[t];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t row = q * 4 + i;
-        if (row >= tile.valid)
-            continue;
-        const size_t at = (size_t)token * args.N + tile.out_row + row;
-        if (args.y_f32)
-            args.y_f32[at] = args.round_f32 ? round_bf16(sum[i]) : sum[i];
-        if (args.y_bf16)
-            args.y_bf16[at] = bf16_bits(sum[i]);
-    }
-}
 
 // ------------------------------------------------------------------ dynamic FP8 quantiser
 // dynamic_fp8_quantized_group128 (kernels/block_fp8_gemv.metal:84-137) and its CPU authority
@@ -410,67 +60,28 @@ void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream
     hipLaunchKernelGGL(split_planes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, x, n, planes);
 }
 
-template <int XT, int XR, int RT>
-static void launch_wide(const WideArgs &args, hipStream_t stream)
-{
-    hipLaunchKernelGGL((linear_wide_kernel<XT, XR, RT>), dim3((args.n_tiles + RT - 1) / RT), dim3(512), 0, stream, args);
-}
-
-// Tiles per workgroup. One generation of workgroups over the 256 CUs reads the activations least and
-// has no second start: one tile up to 256 tiles, two up to 512, then four. Where a row's activations
-// are few bytes beside the weights, several small workgroups per CU beat half a chip of larger ones:
-// up to four rows of bf16 or codes keep one tile up to 768 tiles, eight rows from 513 to 768 (us,
-// K = 4096, one / two / four tiles: bf16 width 1, 257 tiles 7.0 / 8.3 / 12.5, 532 tiles
-// 10.9 / 12.6 / 12.7, 848 tiles 14.8 / 14.3 / 13.7; f32 width 16, 257 tiles 14.8 / 11.2 / 15.4, 512
-// tiles 17.4 / 12.2 / 16.8, 532 tiles 23.5 / 20.4 / 16.7).
-static int pick_rt(int xt, uint32_t W, uint32_t n_tiles)
-{
-    const bool light = xt != WX_F32 && W <= 4, medium = xt != WX_F32 && W <= 8;
-    if (n_tiles <= 256 || (light && n_tiles <= 512) || (medium && n_tiles > 512 && n_tiles <= 768))
-        return 1;
-    return n_tiles <= 512 ? 2 : 4;
-}
-
-template <int XT, int XR>
-static void launch_wide_rt(const WideArgs &args, hipStream_t stream)
-{
-    const int rt = pick_rt(XT, args.W, args.n_tiles);
-    if (rt == 4)
-        launch_wide<XT, XR, 4>(args, stream);
-    else if (rt == 2)
-        launch_wide<XT, XR, 2>(args, stream);
-    else
-        launch_wide<XT, XR, 1>(args, stream);
-}
-
-// Staged rows: the batch's, rounded up to 4 (not for codes, whose eight rows are one copy), 8, 16,
-// 24 (f32) or 32.
-template <int XT>
-static void launch_wide_rows(const WideArgs &args, hipStream_t stream)
-{
-    if (XT != WX_CODES && args.W <= 4)
-        launch_wide_rt<XT, XT != WX_CODES ? 4 : 8>(args, stream);
-    else if (args.W <= 8)
-        launch_wide_rt<XT, 8>(args, stream);
-    else if (args.W <= 16)
-        launch_wide_rt<XT, 16>(args, stream);
-    else if (XT == WX_F32 && args.W <= 24)
-        launch_wide_rt<XT, XT == WX_F32 ? 24 : 32>(args, stream);
-    else
-        launch_wide_rt<XT, 32>(args, stream);
-}
-
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
                    uint32_t K, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
 {
-    const WideArgs args{tiles, n_tiles, x, x_scales, W, K, N, y32, y16, round_f32};
+    WideArgs args{};
+    args.tiles = tiles;
+    args.n_tiles = n_tiles;
+    args.x = x;
+    args.x_scales = x_scales;
+    args.W = W;
+    args.K = K;
+    args.N = N;
+    args.y_f32 = y32;
+    args.y_bf16 = y16;
+    args.round_f32 = round_f32;
+    const int rt = pick_rt(xt, W, n_tiles);
     const int t = timer_begin(xt == WX_CODES ? K_LINEAR_B : K_LINEAR_A, stream);
     if (xt == WX_F32)
-        launch_wide_rows<WX_F32>(args, stream);
+        launch_wide<WK_PROJ, WX_F32>(args, rt, stream);
     else if (xt == WX_BF16)
-        launch_wide_rows<WX_BF16>(args, stream);
+        launch_wide<WK_PROJ, WX_BF16>(args, rt, stream);
     else
-        launch_wide_rows<WX_CODES>(args, stream);
+        launch_wide<WK_PROJ, WX_CODES>(args, rt, stream);
     timer_end(t, stream);
 }
 

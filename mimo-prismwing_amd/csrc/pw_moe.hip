@@ -911,33 +911,26 @@ void launch_route_weights(const RouteJob &job, hipStream_t stream)
     else hipLaunchKernelGGL(route_weights_kernel<4>, dim3(job.rows), dim3(64), 0, stream, job);
 }
 
-// Deterministic cross-wave sum (wave order 0..KSPLIT-1) of NT x f32x4 per lane, result in wave 0.
-template <int KSPLIT, int NT>
-__device__ __forceinline__ void reduce_waves(f32x4 (*red)[NT][64], f32x4 *v, int wave, int lane)
+// Deterministic cross-wave sum (wave order 0..KSPLIT-1) of an f32x4 per lane, result in wave 0.
+template <int KSPLIT>
+__device__ __forceinline__ f32x4 reduce_waves(f32x4 (*red)[64], f32x4 v, int wave, int lane)
 {
-    if constexpr (KSPLIT > 1) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            red[wave][nt][lane] = v[nt];
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                f32x4 s = red[0][nt][lane];
-                for (int w = 1; w < KSPLIT; ++w) {
-                    const f32x4 o = red[w][nt][lane];
-                    s[0] += o[0]; s[1] += o[1]; s[2] += o[2]; s[3] += o[3];
-                }
-                v[nt] = s;
-            }
+    red[wave][lane] = v;
+    __syncthreads();
+    if (wave == 0) {
+        v = red[0][lane];
+        for (int w = 1; w < KSPLIT; ++w) {
+            const f32x4 o = red[w][lane];
+            v[0] += o[0]; v[1] += o[1]; v[2] += o[2]; v[3] += o[3];
         }
     }
+    return v;
 }
 
 // ------------------------------------------------------------- mode B, gate/up + SwiGLU
 // block_fp8_gemm{count}_sglang_blockscaled gate and up, then bf16_staged_swiglu
 // (kernels/block_fp8_gemv.metal:139-160, :935-1046; fused twin :1048-1186).
-template <int KSPLIT, int NT>
+template <int KSPLIT>
 __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
     const ActiveExpert *__restrict__ entries, const uint32_t *__restrict__ placement_pos, const uint8_t *__restrict__ xq,
     const float *__restrict__ xs, uint32_t rows, uint32_t H, uint32_t I, float *__restrict__ hidden,
@@ -945,8 +938,8 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int q = lane >> 4, r16 = lane & 15;
-    __shared__ f32x4 red_g[KSPLIT][NT][64];
-    __shared__ f32x4 red_u[KSPLIT][NT][64];
+    __shared__ f32x4 red_g[KSPLIT][64];
+    __shared__ f32x4 red_u[KSPLIT][64];
     const uint32_t tiles_per_expert = I >> 4;
     // XCD x (workgroup i runs on XCD i % 8) takes a contiguous eighth of each expert's row tiles
     const uint32_t a = blockIdx.x / tiles_per_expert, lt = blockIdx.x % tiles_per_expert;
@@ -954,7 +947,7 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
     const ActiveExpert et = load_entry(entries, a);
     if (et.cnt == 0)
         return;
-    if (et.cnt > 16u * NT) {
+    if (et.cnt > 16u) {
         if (threadIdx.x == 0)
             raise_flag(flags, FLAG_SCHEDULE);
         return;
@@ -965,21 +958,10 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
     const uint8_t *urow = et.ep.up_w + (size_t)(row0 + r16) * H;
     const float *gs = et.ep.gate_s + (row0 >> 7) * blocks;
     const float *us = et.ep.up_s + (row0 >> 7) * blocks;
-    uint32_t pos[NT];
-    bool tok_ok[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t t = nt * 16 + r16;
-        tok_ok[nt] = t < et.cnt;
-        pos[nt] = tok_ok[nt] ? placement_pos[et.off + t] : 0;
-        pos[nt] = pos[nt] < rows ? pos[nt] : rows - 1;
-    }
-    f32x4 tg[NT], tu[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        tg[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        tu[nt] = tg[nt];
-    }
+    const bool tok_ok = (uint32_t)r16 < et.cnt;
+    uint32_t pos = tok_ok ? placement_pos[et.off + r16] : 0;
+    pos = pos < rows ? pos : rows - 1;
+    f32x4 tg = f32x4{0.f, 0.f, 0.f, 0.f}, tu = tg;
     const uint32_t b_begin = wave * blocks / KSPLIT, b_end = (wave + 1) * blocks / KSPLIT;
     for (uint32_t b = b_begin; b < b_end; ++b) {
         const uint32_t col = (b << 7) + q * 32;
@@ -990,81 +972,65 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_gateup_kernel(
         const i32x8 ga = {(int)g0.x, (int)g0.y, (int)g0.z, (int)g0.w, (int)g1.x, (int)g1.y, (int)g1.z, (int)g1.w};
         const i32x8 ua = {(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
         const float sg = gs[b], su = us[b];
+        uint4 c0 = make_uint4(0, 0, 0, 0), c1 = c0;
+        float sa = 0.f;
+        if (tok_ok) {
+            const uint4 *cp = (const uint4 *)(xq + (size_t)pos * H + col);
+            c0 = cp[0];
+            c1 = cp[1];
+            sa = xs[(size_t)pos * blocks + b];
+        }
+        const i32x8 xb = {(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
+        const f32x4 pg = mfma_fp8_16x16x128(ga, xb, f32x4{0.f, 0.f, 0.f, 0.f});
+        const f32x4 pu = mfma_fp8_16x16x128(ua, xb, f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            uint4 c0 = make_uint4(0, 0, 0, 0), c1 = c0;
-            float sa = 0.f;
-            if (tok_ok[nt]) {
-                const uint4 *cp = (const uint4 *)(xq + (size_t)pos[nt] * H + col);
-                c0 = cp[0];
-                c1 = cp[1];
-                sa = xs[(size_t)pos[nt] * blocks + b];
-            }
-            const i32x8 xb = {(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
-            const f32x4 pg = mfma_fp8_16x16x128(ga, xb, f32x4{0.f, 0.f, 0.f, 0.f});
-            const f32x4 pu = mfma_fp8_16x16x128(ua, xb, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                tg[nt][i] = __builtin_fmaf(pg[i] * sg, sa, tg[nt][i]);
-                tu[nt][i] = __builtin_fmaf(pu[i] * su, sa, tu[nt][i]);
-            }
+        for (int i = 0; i < 4; ++i) {
+            tg[i] = __builtin_fmaf(pg[i] * sg, sa, tg[i]);
+            tu[i] = __builtin_fmaf(pu[i] * su, sa, tu[i]);
         }
     }
-    reduce_waves<KSPLIT, NT>(red_g, tg, wave, lane);
-    reduce_waves<KSPLIT, NT>(red_u, tu, wave, lane);
+    tg = reduce_waves<KSPLIT>(red_g, tg, wave, lane);
+    tu = reduce_waves<KSPLIT>(red_u, tu, wave, lane);
     if (wave != 0)
         return;
     bool bad = false;
+    if (!tok_ok)
+        return;
+    float4 out;
+    float *o = (float *)&out;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        if (!tok_ok[nt])
-            continue;
-        const uint32_t t = nt * 16 + r16;
-        float4 out;
-        float *o = (float *)&out;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float g = round_bf16(tg[nt][i]);
-            const float u = round_bf16(tu[nt][i]);
-            o[i] = round_bf16(silu_bf16_staged(g) * u);
-            bad |= !finite_f32(g) || !finite_f32(u) || !finite_f32(o[i]);
-        }
-        *(float4 *)(hidden + (size_t)(et.off + t) * I + row0 + q * 4) = out;
+    for (int i = 0; i < 4; ++i) {
+        const float g = round_bf16(tg[i]);
+        const float u = round_bf16(tu[i]);
+        o[i] = round_bf16(silu_bf16_staged(g) * u);
+        bad |= !finite_f32(g) || !finite_f32(u) || !finite_f32(o[i]);
     }
+    *(float4 *)(hidden + (size_t)(et.off + r16) * I + row0 + q * 4) = out;
     if (bad)
         raise_flag(flags, FLAG_SWIGLU_NONFINITE);
 }
 
 // ------------------------------------------------------------------ mode B, down projection
-template <int KSPLIT, int NT>
+template <int KSPLIT>
 __global__ __launch_bounds__(64 * KSPLIT) void moe_b_down_kernel(
     const ActiveExpert *__restrict__ entries, const uint8_t *__restrict__ hq, const float *__restrict__ hs, uint32_t H, uint32_t I,
     float *__restrict__ y, uint32_t *flags)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int q = lane >> 4, r16 = lane & 15;
-    __shared__ f32x4 red[KSPLIT][NT][64];
+    __shared__ f32x4 red[KSPLIT][64];
     const uint32_t tiles_per_expert = H >> 4;
     const uint32_t a = blockIdx.x / tiles_per_expert, rt = blockIdx.x % tiles_per_expert;
     const ActiveExpert et = load_entry(entries, a);
-    if (et.cnt == 0 || et.cnt > 16u * NT)
+    if (et.cnt == 0 || et.cnt > 16u)
         return;
     const uint32_t row0 = rt << 4;
     const uint32_t blocks = I >> 7;
     const uint8_t *drow = et.ep.down_w + (size_t)(row0 + r16) * I;
     const float *ds = et.ep.down_s + (row0 >> 7) * blocks;
-    uint32_t slot[NT];
-    bool tok_ok[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t t = nt * 16 + r16;
-        tok_ok[nt] = t < et.cnt;
-        slot[nt] = et.off + (tok_ok[nt] ? t : 0);
-    }
-    f32x4 tot[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-        tot[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bool tok_ok = (uint32_t)r16 < et.cnt;
+    const uint32_t slot = et.off + (tok_ok ? r16 : 0);
+    f32x4 tot = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint32_t b_begin = wave * blocks / KSPLIT, b_end = (wave + 1) * blocks / KSPLIT;
     for (uint32_t b = b_begin; b < b_end; ++b) {
         const uint32_t col = (b << 7) + q * 32;
@@ -1072,35 +1038,29 @@ __global__ __launch_bounds__(64 * KSPLIT) void moe_b_down_kernel(
         const uint4 d1 = load_global16(drow + col + 16);
         const i32x8 da = {(int)d0.x, (int)d0.y, (int)d0.z, (int)d0.w, (int)d1.x, (int)d1.y, (int)d1.z, (int)d1.w};
         const float sd = ds[b];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            uint4 c0 = make_uint4(0, 0, 0, 0), c1 = c0;
-            float sa = 0.f;
-            if (tok_ok[nt]) {
-                const uint4 *cp = (const uint4 *)(hq + (size_t)slot[nt] * I + col);
-                c0 = cp[0];
-                c1 = cp[1];
-                sa = hs[(size_t)slot[nt] * blocks + b];
-            }
-            const i32x8 xb = {(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
-            const f32x4 p = mfma_fp8_16x16x128(da, xb, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                tot[nt][i] = __builtin_fmaf(p[i] * sd, sa, tot[nt][i]);
+        uint4 c0 = make_uint4(0, 0, 0, 0), c1 = c0;
+        float sa = 0.f;
+        if (tok_ok) {
+            const uint4 *cp = (const uint4 *)(hq + (size_t)slot * I + col);
+            c0 = cp[0];
+            c1 = cp[1];
+            sa = hs[(size_t)slot * blocks + b];
         }
+        const i32x8 xb = {(int)c0.x, (int)c0.y, (int)c0.z, (int)c0.w, (int)c1.x, (int)c1.y, (int)c1.z, (int)c1.w};
+        const f32x4 p = mfma_fp8_16x16x128(da, xb, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            tot[i] = __builtin_fmaf(p[i] * sd, sa, tot[i]);
     }
-    reduce_waves<KSPLIT, NT>(red, tot, wave, lane);
+    tot = reduce_waves<KSPLIT>(red, tot, wave, lane);
     if (wave != 0)
         return;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        if (!tok_ok[nt])
-            continue;
-        // bf16_round_in_place of the expert output (src/wide_metal_moe.rs:1236-1251)
-        *(float4 *)(y + (size_t)slot[nt] * H + row0 + q * 4) =
-            make_float4(round_bf16(tot[nt][0]), round_bf16(tot[nt][1]), round_bf16(tot[nt][2]),
-                        round_bf16(tot[nt][3]));
-    }
+    if (!tok_ok)
+        return;
+    // bf16_round_in_place of the expert output (src/wide_metal_moe.rs:1236-1251)
+    *(float4 *)(y + (size_t)slot * H + row0 + q * 4) =
+        make_float4(round_bf16(tot[0]), round_bf16(tot[1]), round_bf16(tot[2]),
+                    round_bf16(tot[3]));
 }
 
 // ------------------------------------------------------------------------------- combine
@@ -1192,38 +1152,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
         raise_flag(flags, FLAG_ROUND_NONFINITE);
 }
 
-// ------------------------------------------------------------------- single-expert plan
-// One expert applied to rows 0..rows-1 (the reference's complete-expert measurement,
-// src/lib.rs:4008-6590 "L3" harness): the plan has one active expert whose placements are the
-// rows themselves, so the same gate/up and down kernels run unchanged.
-__global__ void moe_single_plan_kernel(const ExpertPtrs *bank, uint32_t expert, uint32_t rows,
-                                       MoePlan *plan, uint32_t *active_expert,
-                                       uint32_t *active_offset, ActiveExpert *active,
-                                       uint32_t *placement_pos, float *placement_w)
-{
-    const uint32_t i = threadIdx.x;
-    if (i == 0) {
-        plan->n_active = 1;
-        plan->n_placements = rows;
-        plan->max_count = rows;
-        plan->rejected = 0u;
-        active_expert[0] = expert;
-        active_offset[0] = 0;
-        active_offset[1] = rows;
-        ActiveExpert ae{};
-        ae.ep = bank[expert];
-        ae.off = 0;
-        ae.cnt = rows;
-        for (uint32_t k = 0; k < 16; ++k)
-            ae.tok[k] = (uint16_t)k;
-        active[0] = ae;
-    }
-    if (i < rows) {
-        placement_pos[i] = i;
-        placement_w[i] = 1.0f;
-    }
-}
-
 // y [rows x H] f32 -> output (bf16-rounded f32 or bf16 bits).
 __global__ __launch_bounds__(256) void round_output_kernel(const float *__restrict__ y, uint32_t ks,
                                                            size_t split_stride, uint32_t n,
@@ -1309,7 +1237,7 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
 }
 
 // Mode A: gate/up (+SwiGLU) then down, both as split-K expert projections (pw_moe_a.hip).
-// Where the one-expert forward's rounded output goes when its down projection writes it directly.
+// Where a one-token batch's combined output goes when its down projection writes it directly.
 struct DirectOut {
     float *f32;
     uint16_t *bf16;
@@ -1318,8 +1246,8 @@ struct DirectOut {
 
 static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, uint32_t rows,
                               uint32_t placements, uint32_t max_active, uint32_t max_count, uint32_t H,
-                              uint32_t I, uint32_t *flags, hipStream_t stream, const ActiveExpert *one = nullptr,
-                              const DirectOut *direct = nullptr, const ExpertPtrs *bank = nullptr,
+                              uint32_t I, uint32_t *flags, hipStream_t stream, const DirectOut *direct = nullptr,
+                              const ExpertPtrs *bank = nullptr,
                               const OneTokenRoutes *routes = nullptr, const RouteJob *job = nullptr,
                               bool *job_done = nullptr)
 {
@@ -1333,10 +1261,9 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     // layer 542 -> 388 us against stages of 19 rows (split-K gate/up with partials through memory,
     // down in four K splits).
     const uint32_t piece_rows = moe_piece_rows(0, x_f32, rows);
-    const bool pieces = !one && max_count > piece_rows;
+    const bool pieces = max_count > piece_rows;
     const uint32_t entries = pieces ? piece_bound(rows, max_active, piece_rows) : max_active;
-    const int nt = !pieces && max_count > 16 ? 2 : 1;
-    const uint32_t cnt = pieces ? piece_rows : (max_count < 16u * nt ? max_count : 16u * nt);
+    const uint32_t cnt = pieces ? piece_rows : max_count;
     const uint16_t *xp = (const uint16_t *)x;
     if (x_f32) {
         launch_split_planes((const float *)x, rows * H, mb.x_planes, stream);
@@ -1354,10 +1281,6 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     ga.partial = mb.partial;
     ga.flags = flags;
     ga.cap = cnt;
-    if (one) {
-        ga.single = 1;
-        ga.one = *one;
-    }
     if (routes) {  // the fused gate/up and the one-token down+combine read the routes themselves
         ga.bank = bank;
         ga.route_ids = routes->ids;
@@ -1374,9 +1297,9 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     const bool job_in_down = job && !direct;
     if (job && !job_in_down)
         gp_args.job = *job;
-    const bool fused = nt == 1 && launch_moe_a_gateup_fused(x_f32 ? 3 : 1, gp_args, entries, mb.hidden_planes, stream);
+    const bool fused = launch_moe_a_gateup_fused(x_f32 ? 3 : 1, gp_args, entries, mb.hidden_planes, stream);
     if (!fused)
-        launch_moe_a_split(2, x_f32 ? 3 : 1, nt, ga, gp, entries, stream);
+        launch_moe_a_split(2, x_f32 ? 3 : 1, ga, gp, entries, stream);
     timer_end(t, stream);
     if (!fused) {
         t = timer_begin(K_MOE_SWIGLU, stream);
@@ -1397,21 +1320,19 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     da.R = H;
     da.rows = placements;
     t = timer_begin(K_MOE_DOWN, stream);
-    // one expert: the whole-K down writes the rounded output rows itself; a one-token batch: down
-    // and combine in one launch
-    if (direct && (one ? launch_moe_a_down_out(da, direct->f32, direct->bf16, direct->raw, stream)
-                       : launch_moe_a_down_combine1(da, mb.plan, mb.placement_w, direct->f32, direct->bf16,
-                                                    direct->raw, stream))) {
+    // a one-token batch: down and combine in one launch
+    if (direct && launch_moe_a_down_combine1(da, mb.plan, mb.placement_w, direct->f32, direct->bf16, direct->raw,
+                                             stream)) {
         timer_end(t, stream);
         return ExpertOut{nullptr, 0, 0};
     }
     const SplitPlan dp = plan_split(I, 1, 3, cnt);
     da.KS = dp.ks;
-    if (job_in_down && dp.bpw == 8 && nt == 1) {  // the instantiation compiled with a job
+    if (job_in_down && dp.bpw == 8) {  // the instantiation compiled with a job
         da.job = *job;
         *job_done = true;
     }
-    launch_moe_a_split(1, 3, nt, da, dp, entries, stream);
+    launch_moe_a_split(1, 3, da, dp, entries, stream);
     if (job_in_down && !*job_done) {  // another down shape: the weights on their own, before the combine
         launch_route_weights(*job, stream);
         *job_done = true;
@@ -1420,16 +1341,14 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     return ExpertOut{mb.partial, dp.ks, (size_t)placements * H};
 }
 
-// Mode B gate/up, hidden re-quantisation and down as whole-K workgroups (pw_moe_b.hip), after the
-// activations were quantised into mb.xq / mb.xs: from the schedule's entries, or for the one expert
-// `one` on token rows 0..rows-1. The down writes each expert output rounded to bf16 into y (a lone
-// expert: the output rows, y_bf16 too). False, with nothing launched, when the shapes do not fit.
-static bool launch_b_fused(const MoeBuffers &mb, const ActiveExpert *entries, const ActiveExpert *one, uint32_t rows,
-                           uint32_t placements, uint32_t max_active, uint32_t max_count, uint32_t H, uint32_t I, float *y,
-                           uint16_t *y_bf16, uint32_t *flags, hipStream_t stream, const RouteJob *job = nullptr,
-                           bool *job_done = nullptr)
+// Mode B gate/up as whole-K workgroups (pw_moe_b.hip), hidden re-quantisation and down, after the
+// activations were quantised into mb.xq / mb.xs. The down writes each expert output rounded to bf16
+// into mb.y. False, with nothing launched, when the shapes do not fit.
+static bool launch_b_fused(const MoeBuffers &mb, const ActiveExpert *entries, uint32_t rows, uint32_t placements,
+                           uint32_t max_active, uint32_t max_count, uint32_t H, uint32_t I, uint32_t *flags,
+                           hipStream_t stream, const RouteJob *job, bool *job_done)
 {
-    if (!moe_b_fused_shapes(H, I, max_count, one != nullptr))
+    if (!moe_b_fused_shapes(H, I, max_count))
         return false;
     MoeBArgs ga{};
     ga.active = entries;
@@ -1439,64 +1358,39 @@ static bool launch_b_fused(const MoeBuffers &mb, const ActiveExpert *entries, co
     ga.R = I;
     ga.rows = rows;
     ga.cap = max_count;
-    if (one) {
-        ga.single = 1;
-        ga.one = *one;
-    }
     ga.out = mb.hidden;
     ga.flags = flags;
-    MoeBArgs da = ga;
     if (job) {  // the gate/up launch carries the route weights (in extra workgroups)
         ga.job = *job;
         *job_done = true;
     }
-    da.codes = mb.hq;
-    da.scales = mb.hs;
-    da.K = I;
-    da.R = H;
-    da.rows = placements;
-    da.out = y;
-    da.out_bf16 = y_bf16;
-    da.partial = mb.y;  // a lone expert's share sums: [KS][rows][H] within y's [8 rows][H]
     int t = timer_begin(K_MOE_GATEUP, stream);
     (void)launch_moe_b_gateup_fused(ga, max_active, stream);
     timer_end(t, stream);
     // re-quantise the bf16-staged hidden activations per (placement, 128 group)
     launch_quant_group128(mb.hidden, true, placements, I, mb.hq, mb.hs, flags, stream);
     t = timer_begin(K_MOE_DOWN, stream);
-    // a lone expert: whole-K down workgroups that write the output rows; routed experts: the
-    // split-K down (16 rows per workgroup, four waves of four blocks each), which measured faster
-    // there than whole-K workgroups of 16 rows (81 against 98 us at width 8)
-    uint32_t ks = 1;
-    if (one)
-        ks = launch_moe_b_down_fused(da, max_active, stream);
-    else
-        hipLaunchKernelGGL((moe_b_down_kernel<4, 1>), dim3(max_active * (H >> 4)), dim3(256), 0, stream, entries,
-                           mb.hq, mb.hs, H, I, mb.y, flags);
+    // the split-K down (16 rows per workgroup, four waves of four blocks each) measured faster than
+    // whole-K workgroups of 16 rows (81 against 98 us at width 8)
+    hipLaunchKernelGGL(moe_b_down_kernel<4>, dim3(max_active * (H >> 4)), dim3(256), 0, stream, entries, mb.hq, mb.hs, H,
+                       I, mb.y, flags);
     timer_end(t, stream);
-    if (ks > 1) {
-        // the share sums added in share order and rounded (mode B's output is the rounded expert
-        // output, also as F32_RAW)
-        const uint32_t n = rows * H;
-        hipLaunchKernelGGL(round_output_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, mb.y, ks, (size_t)n, n,
-                           y, y_bf16, 0u, flags);
-    }
     return true;
 }
 
-template <int KS, int NT>
+template <int KS>
 static void launch_b_moe(const MoeBuffers &mb, const ActiveExpert *entries, uint32_t rows, uint32_t placements,
                          uint32_t max_active, uint32_t H, uint32_t I, uint32_t *flags, hipStream_t stream)
 {
     const dim3 g1(max_active * (I >> 4)), g2(max_active * (H >> 4)), blk(64 * KS);
     int t = timer_begin(K_MOE_GATEUP, stream);
-    hipLaunchKernelGGL((moe_b_gateup_kernel<KS, NT>), g1, blk, 0, stream, entries, mb.placement_pos, mb.xq, mb.xs,
+    hipLaunchKernelGGL((moe_b_gateup_kernel<KS>), g1, blk, 0, stream, entries, mb.placement_pos, mb.xq, mb.xs,
                        rows, H, I, mb.hidden, flags);
     timer_end(t, stream);
     // re-quantise the bf16-staged hidden activations per (placement, 128 group)
     launch_quant_group128(mb.hidden, true, placements, I, mb.hq, mb.hs, flags, stream);
     t = timer_begin(K_MOE_DOWN, stream);
-    hipLaunchKernelGGL((moe_b_down_kernel<KS, NT>), g2, blk, 0, stream, entries, mb.hq, mb.hs, H, I, mb.y, flags);
+    hipLaunchKernelGGL((moe_b_down_kernel<KS>), g2, blk, 0, stream, entries, mb.hq, mb.hs, H, I, mb.y, flags);
     timer_end(t, stream);
 }
 
@@ -1507,24 +1401,20 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
                                 bool x_quantised = false, const RouteJob *job = nullptr, bool *job_done = nullptr)
 {
     if (mode == 0)
-        return launch_a_moe(mb, x, x_f32, rows, placements, max_active, max_count, H, I, flags, stream, nullptr,
-                            direct, bank, routes, job, job_done);
+        return launch_a_moe(mb, x, x_f32, rows, placements, max_active, max_count, H, I, flags, stream, direct,
+                            bank, routes, job, job_done);
     if (!x_quantised)
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
-    // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces; a lone
-    // expert (the one-expert forward) on 32 tokens per workgroup
+    // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces
     const uint32_t piece_rows = moe_piece_rows(1, x_f32, rows);
-    const bool lone = placements == rows, pieces = !lone && max_count > 16;
+    const bool pieces = max_count > 16;
     const ActiveExpert *entries = pieces ? mb.pieces : mb.active;
     if (pieces) {
         max_active = piece_bound(rows, max_active, piece_rows);
         max_count = piece_rows;
     }
-    if (max_count <= 16 && launch_b_fused(mb, entries, nullptr, rows, placements, max_active, max_count, H, I, mb.y,
-                                          nullptr, flags, stream, job, job_done))
-        return ExpertOut{mb.y, 1, 0};
-    if (max_count > 16) launch_b_moe<4, 2>(mb, entries, rows, placements, max_active, H, I, flags, stream);
-    else launch_b_moe<4, 1>(mb, entries, rows, placements, max_active, H, I, flags, stream);
+    if (!launch_b_fused(mb, entries, rows, placements, max_active, max_count, H, I, flags, stream, job, job_done))
+        launch_b_moe<4>(mb, entries, rows, placements, max_active, H, I, flags, stream);
     return ExpertOut{mb.y, 1, 0};
 }
 
@@ -1564,44 +1454,27 @@ void launch_moe_layer(uint32_t mode, const ExpertPtrs *bank, const MoeBuffers &m
     timer_end(t, stream);
 }
 
-void launch_expert_forward(uint32_t mode, const ExpertPtrs *bank, const ExpertPtrs &ep, uint32_t expert,
-                           const MoeBuffers &mb, const void *x, bool x_f32, uint32_t rows, uint32_t H, uint32_t I,
-                           float *out_f32, uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream)
+// One expert on rows 0..rows-1 (the reference's complete-expert measurement, src/lib.rs:4008-6590 "L3"
+// harness; the dense MLP): gate/up with the SwiGLU, then down, as streaming projections
+// (pw_expert.hip). Mode B's output is the rounded expert output, also as F32_RAW.
+void launch_expert_forward(uint32_t mode, const ExpertPtrs &ep, const MoeBuffers &mb, const void *x, bool x_f32,
+                           uint32_t rows, uint32_t H, uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw,
+                           uint32_t *flags, hipStream_t stream)
 {
-    ExpertOut eo{};
-    if (mode == 0) {
-        // mode A takes the expert's schedule entry by value: no plan kernel
-        ActiveExpert one{};
-        one.ep = ep;
-        one.off = 0;
-        one.cnt = rows;
-        for (uint32_t k = 0; k < 16; ++k)
-            one.tok[k] = (uint16_t)k;
-        const DirectOut direct{out_f32, out_bf16, raw};
-        eo = launch_a_moe(mb, x, x_f32, rows, rows, 1, rows, H, I, flags, stream, &one, &direct);
-        if (!eo.y)
-            return;  // the down projection wrote the output
-    } else {
-        // mode B: the whole-K kernels take the expert's entry by value and the down writes the
-        // output rows (the expert output rounded to bf16, which is also the F32_RAW result)
-        if (rows <= 16) {
-            ActiveExpert one{};
-            one.ep = ep;
-            one.off = 0;
-            one.cnt = rows;
-            for (uint32_t k = 0; k < 16; ++k)
-                one.tok[k] = (uint16_t)k;
-            launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
-            if (launch_b_fused(mb, nullptr, &one, rows, rows, 1, rows, H, I, out_f32, out_bf16, flags, stream))
-                return;
-        }
-        hipLaunchKernelGGL(moe_single_plan_kernel, dim3(1), dim3(256), 0, stream, bank, expert, rows, mb.plan,
-                           mb.active_expert, mb.active_offset, mb.active, mb.placement_pos, mb.placement_w);
-        eo = launch_experts(mode, bank, mb, x, x_f32, rows, rows, 1, rows, H, I, flags, stream);
+    const bool codes = mode != 0;
+    raw = raw && !codes;
+    if (codes)
+        launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
+    launch_expert_gateup(ep, codes, x_f32, codes ? mb.xq : x, mb.xs, rows, H, I, mb.hidden, flags, stream);
+    if (codes)
+        launch_quant_group128(mb.hidden, true, rows, I, mb.hq, mb.hs, flags, stream);
+    const uint32_t ks = launch_expert_down(ep, codes, codes ? (const void *)mb.hq : mb.hidden, mb.hs, rows, H, I, mb.y,
+                                           out_f32, out_bf16, raw, flags, stream);
+    if (ks > 1) {
+        const uint32_t n = rows * H;
+        hipLaunchKernelGGL(round_output_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, mb.y, ks, (size_t)n, n,
+                           out_f32, out_bf16, raw ? 1u : 0u, flags);
     }
-    const uint32_t n = rows * H;
-    hipLaunchKernelGGL(round_output_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, eo.y, eo.ks, eo.stride,
-                       n, out_f32, out_bf16, raw ? 1u : 0u, flags);
 }
 
 }  // namespace pw

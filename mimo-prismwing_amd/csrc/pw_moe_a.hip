@@ -17,7 +17,7 @@
 // accumulates in f32. The 128x128 block scale multiplies each block partial in registers.
 // Split-K partials go to a global buffer; the following kernel sums them in split order 0..KS-1
 // (deterministic): moe_a_swiglu_kernel for gate/up (SwiGLU written as three exact bf16 planes for
-// the down projection), the combine (or the single-expert output rounding) for down.
+// the down projection), the combine for down.
 #include "pw_device.h"
 #include "pw_launch.h"
 #include "pw_route_job.h"
@@ -26,8 +26,8 @@ namespace pw {
 
 // JOB: the launch also carries args.job in its first ROUTE_JOB_WGS workgroups (the routed decode
 // step's down; only that instantiation is compiled with it).
-template <int MATS, int NS, int NT, int BPW, bool JOB = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4 : 2))) void moe_a_split_kernel(const SplitArgs args)
+template <int MATS, int NS, int BPW, bool JOB = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void moe_a_split_kernel(const SplitArgs args)
 {
     extern __shared__ uint4 lds_x[];  // [NS * cnt][KC/8 + 1]
     const int tid = threadIdx.x;
@@ -43,10 +43,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
     const uint32_t s = bid % args.KS;
     const uint32_t g = (bid / args.KS) % G;
     const uint32_t a = bid / (args.KS * G);
-    const ActiveExpert ae = args.single ? args.one : load_entry(args.active, a);
+    const ActiveExpert ae = load_entry(args.active, a);
     if (ae.cnt == 0)
         return;
-    if (ae.cnt > 16u * NT || ae.cnt > args.cap) {
+    if (ae.cnt > 16u || ae.cnt > args.cap) {
         if (tid == 0)
             raise_flag(args.flags, FLAG_SCHEDULE);
         return;
@@ -55,15 +55,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
     constexpr uint32_t KC = BPW * 128;
     const uint32_t k0 = s * KC;
     const uint32_t row_base = g * 64 + wave * 16;  // this wave's 16 rows
-
-    // 1. token rows of routed slots 16..31 (lane t holds slot t's row; slots 0..15 come with the
-    //    schedule entry): gate/up gather the token rows, down reads its own slot rows. Issued
-    //    first, so the staging below waits only for it.
-    uint32_t tok = 0;
-    if constexpr (MATS == 2 && NT == 2) {
-        if ((uint32_t)lane >= 16 && (uint32_t)lane < ae.cnt)
-            tok = args.single ? (uint32_t)lane : load_g(args.placement_pos + ae.off + lane);
-    }
 
     // 2. every weight byte of this wave's rows and K split, in flight at once
     const uint8_t *wbase[MATS];
@@ -108,11 +99,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
     // four waves.
     bool bad_row = false;
 #pragma unroll
-    for (uint32_t t = 0; t < 16u * NT; ++t) {
+    for (uint32_t t = 0; t < 16u; ++t) {
         if (t < ae.cnt) {
             uint32_t src = ae.off + t;
             if constexpr (MATS == 2) {
-                src = t < 16 ? (uint32_t)ae.tok[t] : __builtin_amdgcn_readlane(tok, t);
+                src = ae.tok[t];
                 if (src >= args.rows) {
                     bad_row = true;
                     src = args.rows - 1;
@@ -135,20 +126,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
     __syncthreads();
 
     // 4. block partials on the MFMA, block scale in registers
-    f32x4 tot[MATS][NT];
+    f32x4 tot[MATS];
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            tot[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        tot[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < BPW; ++j) {
-        f32x4 acc[MATS][NT];
+        f32x4 acc[MATS];
 #pragma unroll
         for (int m = 0; m < MATS; ++m)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             bf16x8 A[MATS][2];
@@ -158,33 +145,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
                 A[m][1] = fp8x8_to_bf16x8(wv[m][j][h].z, wv[m][j][h].w);
             }
             const uint32_t cu = j * 16 + h * 8 + q * 2;  // column in 16-byte units
+            const bool ok = (uint32_t)r16 < ae.cnt;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const uint32_t t = nt * 16 + r16;
-                const bool ok = t < ae.cnt;
+            for (int p = 0; p < NS; ++p) {
+                uint4 x0 = make_uint4(0, 0, 0, 0), x1 = x0;
+                if (ok) {
+                    const uint4 *xp = lds_x + (p * ae.cnt + r16) * STRIDE + cu;
+                    x0 = xp[0];
+                    x1 = xp[1];
+                }
 #pragma unroll
-                for (int p = 0; p < NS; ++p) {
-                    uint4 x0 = make_uint4(0, 0, 0, 0), x1 = x0;
-                    if (ok) {
-                        const uint4 *xp = lds_x + (p * ae.cnt + t) * STRIDE + cu;
-                        x0 = xp[0];
-                        x1 = xp[1];
-                    }
-#pragma unroll
-                    for (int m = 0; m < MATS; ++m) {
-                        acc[m][nt] = mfma_bf16_16x16x32(A[m][0], bf16x8_from_u4(x0), acc[m][nt]);
-                        acc[m][nt] = mfma_bf16_16x16x32(A[m][1], bf16x8_from_u4(x1), acc[m][nt]);
-                    }
+                for (int m = 0; m < MATS; ++m) {
+                    acc[m] = mfma_bf16_16x16x32(A[m][0], bf16x8_from_u4(x0), acc[m]);
+                    acc[m] = mfma_bf16_16x16x32(A[m][1], bf16x8_from_u4(x1), acc[m]);
                 }
             }
         }
 #pragma unroll
         for (int m = 0; m < MATS; ++m)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    tot[m][nt][i] = __builtin_fmaf(sc[m][j], acc[m][nt][i], tot[m][nt][i]);
+            for (int i = 0; i < 4; ++i)
+                tot[m][i] = __builtin_fmaf(sc[m][j], acc[m][i], tot[m][i]);
     }
 
     // 5. split-K partials: partial[s][m][slot][row]. The splits are summed in split order by the
@@ -192,15 +173,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
     //    cross-workgroup synchronisation, so no device-scope cache maintenance per workgroup.
     const uint32_t P = args.P, R = args.R;
     const uint32_t row4 = row_base + q * 4;
+    if ((uint32_t)r16 < ae.cnt)
 #pragma unroll
-    for (int m = 0; m < MATS; ++m)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const uint32_t t = nt * 16 + r16;
-            if (t < ae.cnt)
-                *(float4 *)(args.partial + (((size_t)s * MATS + m) * P + ae.off + t) * R + row4) =
-                    make_float4(tot[m][nt][0], tot[m][nt][1], tot[m][nt][2], tot[m][nt][3]);
-        }
+        for (int m = 0; m < MATS; ++m)
+            *(float4 *)(args.partial + (((size_t)s * MATS + m) * P + ae.off + r16) * R + row4) =
+                make_float4(tot[m][0], tot[m][1], tot[m][2], tot[m][3]);
 }
 
 // Gate/up over the whole K in one workgroup, SwiGLU fused: the decode fast path when the expert's
@@ -211,7 +188,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 ? 4
 // are added in split order 0..7 -- the same order and the same arithmetic as the split kernel
 // followed by moe_a_swiglu_kernel, so the hidden planes are bit-identical -- and the SwiGLU is
 // written as three exact bf16 planes. No split partials go through memory.
-// RM = 8 (the one-expert forward): a work item is 8 rows of gate and the same 8 rows of up, stacked
+// RM = 8 (one-row experts): a work item is 8 rows of gate and the same 8 rows of up, stacked
 // into one 16-row MFMA operand (lanes 0..7 of a row group read gate rows, 8..15 up rows), so a lone
 // expert spreads over twice the workgroups; output rows 0..7 are gate, 8..15 up, and each gate
 // lane takes its up values from the lane 32 above. The sums are the same as with RM = 16.
@@ -242,9 +219,8 @@ __global__ __launch_bounds__(512) void moe_a_gateup_fused_kernel(const SplitArgs
     // Workgroup i runs on XCD i % 8. XCD x takes the contiguous row groups [x G/8, (x + 1) G/8) of
     // each routed expert (1 MB of gate and 1 MB of up at G = 128), not every eighth 16-row group:
     // the strided form gave each XCD's loads a common set of address bits and ran 4% slower, and
-    // up to 7% slower for some physical placements of the bank. A lone expert (the one-expert
-    // forward, the dense MLP) keeps the strided order, which measured 1 µs faster there. Which
-    // workgroup computes which rows does not change any sum.
+    // up to 7% slower for some physical placements of the bank. Which workgroup computes which rows
+    // does not change any sum.
     uint32_t bid = blockIdx.x;
     if constexpr (JOB) {
         if (route_job_prologue(args.job, lds_x, &bid))
@@ -252,8 +228,8 @@ __global__ __launch_bounds__(512) void moe_a_gateup_fused_kernel(const SplitArgs
     }
     const uint32_t G = args.R / RM;
     const uint32_t a = bid / G, local = bid % G;
-    const uint32_t g = G % 8 == 0 && !args.single ? (local % 8) * (G / 8) + local / 8 : local;
-    const ActiveExpert ae = args.single ? args.one : (args.route_ids ? route_entry(args, a) : load_entry(args.active, a));
+    const uint32_t g = G % 8 == 0 ? (local % 8) * (G / 8) + local / 8 : local;
+    const ActiveExpert ae = args.route_ids ? route_entry(args, a) : load_entry(args.active, a);
     if (ae.cnt == 0)
         return;
     if (ae.cnt > 16u || ae.cnt > args.cap) {
@@ -444,9 +420,8 @@ bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_activ
     if (args.K != 8 * 4 * 128 || args.R % 16 != 0 || (uint32_t)ns * args.cap > 9)
         return false;
     const size_t lds = fused_lds(ns, args.cap, args.K);
-    // a lone expert (the one-expert forward) and one-row experts (a one-token batch) take 8 + 8-row
-    // work items: twice the workgroups
-    const bool half = args.R % 8 == 0 && (args.single || args.cap == 1);
+    // one-row experts (a one-token batch) take 8 + 8-row work items: twice the workgroups
+    const bool half = args.R % 8 == 0 && args.cap == 1;
     const dim3 grid(max_active * (args.R / (half ? 8 : 16)) + (args.job.rows ? ROUTE_JOB_WGS : 0)), block(512);
 #define PW_FUSED_J(NS, RM, J)                                                                                \
     do {                                                                                                      \
@@ -467,153 +442,6 @@ bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_activ
     }
 #undef PW_FUSED
 #undef PW_FUSED_J
-    return true;
-}
-
-// Down over the whole K in one workgroup for one expert's rows, output rounding fused: the
-// one-expert forward's last launch (dense MLP, complete expert). Work item: 16 rows of down.
-// Eight waves split K = I (wave w: blocks [w * BPW, (w + 1) * BPW)), each with all of its weight
-// loads in flight at once; the expert's three bf16 hidden planes (rows 0..cnt-1) go straight into
-// LDS; the eight split sums meet in LDS and are added in split order 0..7, then rounded to bf16 (or
-// kept as raw f32) and written as the output rows: no split partials through memory, no rounding
-// launch.
-template <int BPW>
-__global__ __launch_bounds__(512) void moe_a_down_out_kernel(const SplitArgs args, float *__restrict__ out_f32,
-                                                             uint16_t *__restrict__ out_bf16, uint32_t raw)
-{
-    extern __shared__ uint4 lds_x[];  // [3 * cnt][K/8 + 1]; then the split partials [8][64]
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // split index, wave-uniform
-    const int q = lane >> 4, r16 = lane & 15;
-    const ActiveExpert &ae = args.one;
-    const uint32_t cnt = ae.cnt;
-    if (cnt == 0 || cnt > args.cap) {
-        if (tid == 0 && cnt != 0)
-            raise_flag(args.flags, FLAG_SCHEDULE);
-        return;
-    }
-    const uint32_t K = args.K, R = args.R;
-    constexpr uint32_t KC = BPW * 128;
-    const uint32_t k0 = wave * KC;
-    const uint32_t row0 = blockIdx.x * 16;
-
-    // 1. the hidden rows (three planes, whole K) -> LDS: wave w copies its K split of every row and
-    //    plane (KC / 8 16-byte units per row, at most 64 lanes per instruction) and reads only that
-    constexpr uint32_t PER_SPLIT = KC / 8, LANES = PER_SPLIT < 64 ? PER_SPLIT : 64, CPS = PER_SPLIT / LANES;
-    // (unrolled over the eight possible rows: a loop would make the compiler wait for every
-    // outstanding weight load before its first iteration)
-    const uint32_t stride = K / 8 + 1;
-#pragma unroll
-    for (uint32_t t = 0; t < 8; ++t)
-        if (t < cnt) {
-#pragma unroll
-            for (uint32_t p = 0; p < 3; ++p)
-#pragma unroll
-                for (uint32_t c = 0; c < CPS; ++c)
-                    if ((uint32_t)lane < LANES)
-                        lds_load16(args.x + p * args.x_plane + (size_t)t * K + k0 + (c * 64 + lane) * 8,
-                                   lds_x + (p * cnt + t) * stride + (k0 >> 3) + c * 64);
-        }
-    asm volatile("" ::: "memory");  // the copies stay the oldest memory operations
-
-    // 2. this wave's weight bytes, all in flight at once, and its block scales
-    uint4 wv[BPW][2];
-    const uint8_t *wrow = ae.ep.down_w + (size_t)(row0 + r16) * K + k0 + q * 16;
-#pragma unroll
-    for (int j = 0; j < BPW; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            wv[j][h] = load_global16(wrow + j * 128 + h * 64);
-    const uint32_t blocks = K >> 7;
-    float sc[BPW];
-#pragma unroll
-    for (int j = 0; j < BPW; ++j)
-        sc[j] = load_g(ae.ep.down_s + (row0 >> 7) * blocks + (k0 >> 7) + j);
-
-    // the copies are done once all but the weight loads are; block j's MFMAs start when its weights arrive
-    wait_vmcnt<BPW * 2>();
-
-    // 3. block partials on the MFMA, block scale in registers (as moe_a_split_kernel)
-    f32x4 tot = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bool ok = (uint32_t)r16 < cnt;
-#pragma unroll
-    for (int j = 0; j < BPW; ++j) {
-        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bf16x8 A0 = fp8x8_to_bf16x8(wv[j][h].x, wv[j][h].y);
-            const bf16x8 A1 = fp8x8_to_bf16x8(wv[j][h].z, wv[j][h].w);
-            const uint32_t cu = (k0 >> 3) + j * 16 + h * 8 + q * 2;
-#pragma unroll
-            for (int p = 0; p < 3; ++p) {
-                uint4 x0 = make_uint4(0, 0, 0, 0), x1 = x0;
-                if (ok) {
-                    const uint4 *xp = lds_x + (p * cnt + r16) * stride + cu;
-                    x0 = xp[0];
-                    x1 = xp[1];
-                }
-                acc = mfma_bf16_16x16x32(A0, bf16x8_from_u4(x0), acc);
-                acc = mfma_bf16_16x16x32(A1, bf16x8_from_u4(x1), acc);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            tot[i] = __builtin_fmaf(sc[j], acc[i], tot[i]);
-    }
-
-    // 4. the eight split partials meet in LDS (after every wave is done with the activations),
-    //    summed in split order; lane: rows 4q .. 4q + 3 of the 16, row r16 of the output
-    __syncthreads();
-    f32x4 *red = (f32x4 *)lds_x;  // [8 splits][64 lanes]
-    red[wave * 64 + lane] = tot;
-    __syncthreads();
-    if (wave != 0 || !ok)
-        return;
-    f32x4 sum = red[lane];
-#pragma unroll
-    for (int sp = 1; sp < 8; ++sp) {
-        const f32x4 o = red[sp * 64 + lane];
-        sum[0] += o[0];
-        sum[1] += o[1];
-        sum[2] += o[2];
-        sum[3] += o[3];
-    }
-    bool bad = false;
-    float r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        r[i] = round_bf16(sum[i]);
-        bad |= !finite_f32(r[i]);
-    }
-    const size_t at = (size_t)r16 * R + row0 + q * 4;
-    if (out_f32)
-        *(float4 *)(out_f32 + at) = raw ? make_float4(sum[0], sum[1], sum[2], sum[3]) : make_float4(r[0], r[1], r[2], r[3]);
-    if (out_bf16)
-        *(uint2 *)(out_bf16 + at) = make_uint2((f32_bits(r[0]) >> 16) | (f32_bits(r[1]) & 0xffff0000u),
-                                               (f32_bits(r[2]) >> 16) | (f32_bits(r[3]) & 0xffff0000u));
-    if (bad)
-        raise_flag(args.flags, FLAG_ROUND_NONFINITE);
-}
-
-bool launch_moe_a_down_out(const SplitArgs &args, float *out_f32, uint16_t *out_bf16, bool raw, hipStream_t stream)
-{
-    // eight K splits of one or two 128-column blocks each, output rows in whole 16-row tiles,
-    // the three hidden planes of up to eight rows within LDS
-    const uint32_t K = args.K;
-    if (!args.single || (K != 8 * 128 && K != 16 * 128) || args.R % 16 != 0 || args.one.cnt > 8)
-        return false;
-    const size_t stage = (size_t)3 * args.one.cnt * (K / 8 + 1) * 16, red = (size_t)8 * 64 * 16;
-    const size_t lds = stage > red ? stage : red;
-    const dim3 grid(args.R >> 4), block(512);
-    if (K == 16 * 128) {
-        if (lds > 65536)
-            (void)hipFuncSetAttribute((const void *)moe_a_down_out_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lds);
-        hipLaunchKernelGGL((moe_a_down_out_kernel<2>), grid, block, lds, stream, args, out_f32, out_bf16, raw ? 1u : 0u);
-    } else {
-        hipLaunchKernelGGL((moe_a_down_out_kernel<1>), grid, block, lds, stream, args, out_f32, out_bf16, raw ? 1u : 0u);
-    }
     return true;
 }
 
@@ -908,41 +736,40 @@ SplitPlan plan_split(uint32_t K, int mats, int ns, uint32_t max_cnt)
     return sp;
 }
 
-template <int MATS, int NS, int NT>
-static void launch_split_nt(const SplitArgs &args, const SplitPlan &sp, uint32_t grid, hipStream_t stream)
+template <int MATS, int NS>
+static void launch_split_ns(const SplitArgs &args, const SplitPlan &sp, uint32_t grid, hipStream_t stream)
 {
     switch (sp.bpw) {
     case 8:
         if constexpr (MATS == 1) {
             if (args.job.rows)
-                hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, NT, 8, true>), dim3(grid + ROUTE_JOB_WGS), dim3(256),
+                hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, 8, true>), dim3(grid + ROUTE_JOB_WGS), dim3(256),
                                    sp.lds, stream, args);
             else
-                hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, NT, 8>), dim3(grid), dim3(256), sp.lds, stream, args);
+                hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, 8>), dim3(grid), dim3(256), sp.lds, stream, args);
             break;
         }
         [[fallthrough]];
     case 4:
-        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, NT, 4>), dim3(grid), dim3(256), sp.lds, stream, args);
+        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, 4>), dim3(grid), dim3(256), sp.lds, stream, args);
         break;
     case 2:
-        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, NT, 2>), dim3(grid), dim3(256), sp.lds, stream, args);
+        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, 2>), dim3(grid), dim3(256), sp.lds, stream, args);
         break;
     default:
-        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, NT, 1>), dim3(grid), dim3(256), sp.lds, stream, args);
+        hipLaunchKernelGGL((moe_a_split_kernel<MATS, NS, 1>), dim3(grid), dim3(256), sp.lds, stream, args);
         break;
     }
 }
 
-void launch_moe_a_split(int mats, int ns, int nt, const SplitArgs &args, const SplitPlan &sp,
-                        uint32_t max_active, hipStream_t stream)
+void launch_moe_a_split(int mats, int ns, const SplitArgs &args, const SplitPlan &sp, uint32_t max_active,
+                        hipStream_t stream)
 {
     const uint32_t grid = max_active * (args.R >> 6) * sp.ks;
     if (mats == 2) {
-        if (ns == 3) { if (nt == 2) launch_split_nt<2, 3, 2>(args, sp, grid, stream); else launch_split_nt<2, 3, 1>(args, sp, grid, stream); }
-        else { if (nt == 2) launch_split_nt<2, 1, 2>(args, sp, grid, stream); else launch_split_nt<2, 1, 1>(args, sp, grid, stream); }
+        if (ns == 3) launch_split_ns<2, 3>(args, sp, grid, stream); else launch_split_ns<2, 1>(args, sp, grid, stream);
     } else {
-        if (nt == 2) launch_split_nt<1, 3, 2>(args, sp, grid, stream); else launch_split_nt<1, 3, 1>(args, sp, grid, stream);
+        launch_split_ns<1, 3>(args, sp, grid, stream);
     }
 }
 

@@ -1614,10 +1614,8 @@ int pw_expert_forward_device(pw_runtime *rt, const pw_expert_bank *bank, uint32_
     StreamOrder order(rt, s);
     PW_HIP(order.err);
     PW_TRY(ensure_moe(rt, rows, bank->n_experts, bank->hidden, bank->intermediate));
-    pw::launch_expert_forward(mode, bank->table, bank->host_table[expert], expert, rt->mb, x, x_dtype == PW_DTYPE_F32,
-                              rows,
-                              bank->hidden, bank->intermediate,
-                              out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
+    pw::launch_expert_forward(mode, bank->host_table[expert], rt->mb, x, x_dtype == PW_DTYPE_F32, rows, bank->hidden,
+                              bank->intermediate, out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
                               out_dtype == PW_DTYPE_BF16 ? (uint16_t *)output : nullptr,
                               out_dtype == PW_DTYPE_F32_RAW, rt->d_flags, s);
     PW_HIP(hipGetLastError());

@@ -71,3 +71,48 @@ def test_dense_mlp_mode_a(rt, dense, rows):
     ref32, refbf = O.expert_mode_a(x, expert)
     assert normwise(_run(rt, torch, bank, x, P.MODE_A, P.DTYPE_F32_RAW), ref32) <= 1e-3
     assert normwise(_run(rt, torch, bank, x, P.MODE_A, P.DTYPE_BF16), refbf) <= 8e-3
+
+
+@pytest.mark.parametrize("inter", [128, 2176, 5120, 9216, 16384])
+def test_expert_tile_and_share_edges(rt, inter):
+    """Gate/up tiles of every workgroup size (16 to 2048 tiles of eight gate and eight up rows, a
+    partial last workgroup at 272), waves with no, one and several steps, down in one and in two K
+    shares (intermediate 16384, 17 and 32 rows), at staged-row edges. Mode A on raw f32 against 64
+    bits: two projections' exact products added in f32 chains of at most 48 roundings each (2e-6
+    apiece) and the SwiGLU between them (an ulp or two of each value): 4.5e-6. Mode B equals the same
+    expert as separate projection calls, bit for bit with one share; two shares may move an output
+    over one bf16 rounding step."""
+    import torch
+    from helpers import dequant, fp8_weight, log_uniform_scales, rel_l2, within_one_bf16_ulp
+    hidden = 256
+    rng = np.random.default_rng(inter)
+    mats = []
+    for n, k in ((inter, hidden), (inter, hidden), (hidden, inter)):
+        s = log_uniform_scales(rng, n, k) / 4  # keeps gates in the SwiGLU's curved range
+        mats.append((fp8_weight(rng, n, k, s * 16), s))
+    projs = [rt.bind_projection(w, s) for w, s in mats]
+    bank = rt.expert_bank(*[[p] for p in projs])
+    g, u, d = (dequant(w, s).astype(np.float64) for w, s in mats)
+    x = rng.standard_normal((32, hidden)).astype(np.float32)
+    xd = x.astype(np.float64)
+    h = (xd @ g.T) / (1.0 + np.exp(-(xd @ g.T))) * (xd @ u.T)
+    ref = h @ d.T
+    for rows in (1, 4, 8, 9, 17, 32):
+        xt = torch.from_numpy(x[:rows]).cuda()
+        out = torch.empty((rows, hidden), dtype=torch.float32, device="cuda")
+        stream = torch.cuda.current_stream().cuda_stream
+        rt.expert_forward_device(bank, 0, xt, rows, out, mode=P.MODE_A, x_dtype=P.DTYPE_F32,
+                                 out_dtype=P.DTYPE_F32_RAW, stream=stream)
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), ref[:rows]) <= 4.5e-6, rows
+        rt.expert_forward_device(bank, 0, xt, rows, out, mode=P.MODE_B, x_dtype=P.DTYPE_F32, out_dtype=P.DTYPE_F32,
+                                 stream=stream)
+        torch.cuda.synchronize()
+        assert rt.take_flags() == 0
+        gu = [rt.execute_fp8_linear(x[:rows], p, mode=P.MODE_B).output for p in projs[:2]]
+        want = rt.execute_fp8_linear(O.swiglu_bf16_staged(*gu), projs[2], mode=P.MODE_B).output
+        got = out.cpu().numpy()
+        if inter < 16384 or rows <= 16:
+            assert np.array_equal(got, want), rows
+        else:
+            assert within_one_bf16_ulp(got, want), rows
