@@ -18,7 +18,7 @@ OBJ_DIR = os.path.join(HERE, "_build")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 SOURCES = ["pw_linear.hip", "pw_expert.hip", "pw_bf16.hip", "pw_moe.hip", "pw_moe_a.hip", "pw_moe_b.hip", "pw_prefill.hip", "pw_router.hip",
-           "pw_synth.hip", "pw_checkpoint.cpp",
+           "pw_synth.hip", "pw_host_io.hip", "pw_checkpoint.cpp",
            "pw_runtime.cpp"]
 
 FLAGS = [

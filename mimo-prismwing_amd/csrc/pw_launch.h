@@ -319,6 +319,11 @@ void launch_expert_forward(uint32_t mode, const ExpertPtrs &ep, const MoeBuffers
                            uint32_t rows, uint32_t H, uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw,
                            uint32_t *flags, hipStream_t stream);
 
+// Pinned host block -> device (flags cleared when given), and device -> pinned host block with the
+// error word read out and cleared; both copy whole 16-byte units, so blocks are padded to them.
+void launch_upload(const void *host, void *dev, size_t bytes, uint32_t *flags, hipStream_t stream);
+void launch_download(const void *dev, void *host, size_t bytes, uint32_t *flags, uint32_t *host_flags, hipStream_t stream);
+
 // Seeded synthetic data for benchmarks and tests (counter-based, reproducible on one device).
 void launch_synth_fp8(uint8_t *w, const float *scales, uint64_t rows, uint64_t cols, uint64_t seed,
                       hipStream_t stream);

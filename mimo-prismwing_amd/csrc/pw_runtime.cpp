@@ -63,6 +63,13 @@ namespace {
             return fail(PW_ERR_DEVICE, "%s failed: %s", #call, hipGetErrorString(e_));          \
     } while (0)
 
+#define PW_TRY(expr)                 \
+    do {                             \
+        int s_ = (expr);             \
+        if (s_ != PW_OK)             \
+            return s_;               \
+    } while (0)
+
 double now_ms()
 {
     return std::chrono::duration<double, std::milli>(
@@ -95,6 +102,33 @@ struct DevBuf {
     }
 };
 
+// Pinned host memory of a runtime's host-array calls: grows to the largest call (a routed layer of 128
+// rows of 4096 columns takes 2 MiB each way) and is freed with the runtime.
+struct HostBuf {
+    void *p = nullptr;
+    size_t bytes = 0;
+    ~HostBuf() { release(); }
+    void release()
+    {
+        if (p)
+            (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+    hipError_t ensure(size_t need)
+    {
+        if (need <= bytes)
+            return hipSuccess;
+        release();
+        hipError_t e = hipHostMalloc(&p, need, hipHostMallocDefault);
+        if (e == hipSuccess)
+            bytes = need;
+        else
+            p = nullptr;
+        return e;
+    }
+};
+
 }  // namespace
 
 struct pw_runtime {
@@ -103,7 +137,9 @@ struct pw_runtime {
     hipStream_t stream = nullptr;
     uint32_t *d_flags = nullptr;
     // scratch: host-call staging and mode-B activation codes
-    DevBuf in, out, codes, scales, route_ids, route_w, bank_table;
+    DevBuf in, out, codes, scales;
+    HostBuf host_in, host_out;
+    bool host_pending = false;  // a call left before its wait: its transfers may still be running
     // routed-MoE per-layer scratch
     DevBuf moe_plan, moe_active_expert, moe_active_offset, moe_pos, moe_w, moe_slots, moe_hidden,
         moe_hidden_planes, moe_x_planes, moe_y, moe_xq, moe_xs, moe_hq, moe_hs, lin_planes,
@@ -258,32 +294,88 @@ int check_scales(const float *s, size_t n)
     return PW_OK;
 }
 
+// (no early exit: the loops vectorise)
 bool all_bf16_exact(const float *x, size_t n)
 {
+    uint32_t low = 0;
     for (size_t i = 0; i < n; ++i)
-        if (pw::f32_bits(x[i]) & 0xffffu)
-            return false;
-    return true;
+        low |= pw::f32_bits(x[i]);
+    return (low & 0xffffu) == 0;
 }
 
-// Upload a host f32 activation block, as bf16 when every value is a bf16 value (exact), else
-// as f32 (the kernels then split it into bf16 hi + lo).
-int stage_input(pw_runtime *rt, const float *x, size_t n, bool &is_f32)
+bool all_finite(const float *x, size_t n)
 {
-    is_f32 = !all_bf16_exact(x, n);
-    if (is_f32) {
-        PW_HIP(rt->in.ensure(n * 4));
-        PW_HIP(hipMemcpyAsync(rt->in.p, x, n * 4, hipMemcpyHostToDevice, rt->stream));
-    } else {
-        std::vector<uint16_t> h(n);
-        for (size_t i = 0; i < n; ++i)
-            h[i] = (uint16_t)(pw::f32_bits(x[i]) >> 16);
-        PW_HIP(rt->in.ensure(n * 2));
-        PW_HIP(hipMemcpyAsync(rt->in.p, h.data(), n * 2, hipMemcpyHostToDevice, rt->stream));
-        PW_HIP(hipStreamSynchronize(rt->stream));  // h is released on return
-    }
-    return PW_OK;
+    uint32_t bad = 0;
+    for (size_t i = 0; i < n; ++i)
+        bad |= (pw::f32_bits(x[i]) & 0x7f800000u) == 0x7f800000u;
+    return bad == 0;
 }
+
+// One host-array call's transfers. Its inputs are packed into the runtime's pinned block, 256-byte
+// aligned pieces in the same places on the device, and copied by one launch, which also clears the
+// error word; its outputs come back in one launch with the error word.
+struct HostCall {
+    pw_runtime *rt;
+    size_t used = 0;
+
+    static size_t padded(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+
+    int begin(size_t bytes)
+    {
+        if (rt->host_pending)  // the last call failed between its launches and its wait
+            PW_HIP(hipStreamSynchronize(rt->stream));
+        rt->host_pending = false;
+        PW_HIP(rt->host_in.ensure(bytes));
+        PW_HIP(rt->in.ensure(bytes));
+        return PW_OK;
+    }
+
+    // `bytes` of the block: where to write them, and where they will be on the device
+    void *take(size_t bytes, void *&dev)
+    {
+        void *host = (char *)rt->host_in.p + used;
+        dev = (char *)rt->in.p + used;
+        used += padded(bytes);
+        return host;
+    }
+
+    // an f32 activation block, as bf16 when every value is a bf16 value (exact), else as f32
+    void activations(const float *x, size_t n, bool &is_f32, void *&dev)
+    {
+        is_f32 = !all_bf16_exact(x, n);
+        void *h = take(n * (is_f32 ? 4 : 2), dev);
+        if (is_f32)
+            std::memcpy(h, x, n * 4);
+        else
+            for (size_t i = 0; i < n; ++i)
+                ((uint16_t *)h)[i] = (uint16_t)(pw::f32_bits(x[i]) >> 16);
+    }
+
+    int upload()
+    {
+        rt->host_pending = true;
+        pw::launch_upload(rt->host_in.p, rt->in.p, used, rt->d_flags, rt->stream);
+        PW_HIP(hipGetLastError());
+        return PW_OK;
+    }
+
+    // n outputs in rt->out (padded to 16 bytes) -> output, once the call's work is done; flags: the
+    // error word, finite: every output is
+    int finish(float *output, size_t n, uint32_t &flags, bool &finite_out)
+    {
+        const size_t bytes = padded(n * 4);
+        PW_HIP(rt->host_out.ensure(bytes + 256));
+        uint32_t *host_flags = (uint32_t *)((char *)rt->host_out.p + bytes);
+        pw::launch_download(rt->out.p, rt->host_out.p, n * 4, rt->d_flags, host_flags, rt->stream);
+        PW_HIP(hipGetLastError());
+        PW_HIP(hipStreamSynchronize(rt->stream));
+        rt->host_pending = false;
+        flags = *host_flags;
+        finite_out = all_finite((const float *)rt->host_out.p, n);
+        std::memcpy(output, rt->host_out.p, n * 4);
+        return PW_OK;
+    }
+};
 
 int reset_flags(pw_runtime *rt)
 {
@@ -300,13 +392,6 @@ int read_flags(pw_runtime *rt, uint32_t &flags)
     PW_HIP(hipStreamSynchronize(rt->stream));
     return PW_OK;
 }
-
-#define PW_TRY(expr)                 \
-    do {                             \
-        int s_ = (expr);             \
-        if (s_ != PW_OK)             \
-            return s_;               \
-    } while (0)
 
 // The device schedule's tables for `rows` token rows over E experts.
 int ensure_sched(pw_runtime *rt, uint32_t rows, uint32_t E)
@@ -859,21 +944,23 @@ int pw_fp8_linear(pw_runtime *rt, uint32_t mode, const float *input, uint32_t ro
     if (rows < 1 || rows > 32)
         return fail(PW_ERR_ARGUMENT, "wide row count must be between one and 32");
     const size_t n_in = (size_t)rows * p->columns, n_out = (size_t)rows * p->rows;
-    for (size_t i = 0; i < n_in; ++i)
-        if (!finite(input[i]))
-            return fail(PW_ERR_NONFINITE, "wide FP8 linear input is non-finite");
+    if (!all_finite(input, n_in))
+        return fail(PW_ERR_NONFINITE, "wide FP8 linear input is non-finite");
     PW_HIP(set_device(rt));
     TimerScope timer_scope(rt);
     StreamOrder order(rt, rt->stream);
     PW_HIP(order.err);
-    PW_TRY(reset_flags(rt));
+    HostCall call{rt};
+    PW_TRY(call.begin(HostCall::padded(n_in * 4)));
     bool x_f32;
-    PW_TRY(stage_input(rt, input, n_in, x_f32));
-    PW_HIP(rt->out.ensure(n_out * 4));
-    PW_TRY(enqueue_linear(rt, mode, rt->in.p, x_f32, rows, p, (float *)rt->out.p, nullptr, 1, rt->stream));
-    PW_HIP(hipMemcpyAsync(output, rt->out.p, n_out * 4, hipMemcpyDeviceToHost, rt->stream));
+    void *x;
+    call.activations(input, n_in, x_f32, x);
+    PW_TRY(call.upload());
+    PW_HIP(rt->out.ensure(HostCall::padded(n_out * 4)));
+    PW_TRY(enqueue_linear(rt, mode, x, x_f32, rows, p, (float *)rt->out.p, nullptr, 1, rt->stream));
     uint32_t flags = 0;
-    PW_TRY(read_flags(rt, flags));
+    bool finite_out = true;
+    PW_TRY(call.finish(output, n_out, flags, finite_out));
     if (stats) {
         stats->wall_ms = now_ms() - t0;
         stats->mapped_source_bytes = 0;
@@ -882,9 +969,8 @@ int pw_fp8_linear(pw_runtime *rt, uint32_t mode, const float *input, uint32_t ro
     }
     if (flags)
         return fail(PW_ERR_GPU_FLAGS, "wide FP8 linear kernels set error flags %u", flags);
-    for (size_t i = 0; i < n_out; ++i)
-        if (!finite(output[i]))
-            return fail(PW_ERR_OUTPUT, "wide FP8 linear produced non-finite output");
+    if (!finite_out)
+        return fail(PW_ERR_OUTPUT, "wide FP8 linear produced non-finite output");
     return PW_OK;
 }
 
@@ -1009,21 +1095,23 @@ int pw_bf16_linear(pw_runtime *rt, const float *input, uint32_t rows, const pw_p
     if (rows < 1 || rows > 32)
         return fail(PW_ERR_ARGUMENT, "wide row count must be between one and 32");
     const size_t n_in = (size_t)rows * p->columns, n_out = (size_t)rows * p->rows;
-    for (size_t i = 0; i < n_in; ++i)
-        if (!finite(input[i]))
-            return fail(PW_ERR_NONFINITE, "wide BF16 linear layout mismatch (non-finite input)");
+    if (!all_finite(input, n_in))
+        return fail(PW_ERR_NONFINITE, "wide BF16 linear layout mismatch (non-finite input)");
     PW_HIP(set_device(rt));
     TimerScope timer_scope(rt);
     StreamOrder order(rt, rt->stream);
     PW_HIP(order.err);
-    PW_TRY(reset_flags(rt));
+    HostCall call{rt};
+    PW_TRY(call.begin(HostCall::padded(n_in * 4)));
     bool x_f32;
-    PW_TRY(stage_input(rt, input, n_in, x_f32));
-    PW_HIP(rt->out.ensure(n_out * 4));
-    PW_TRY(enqueue_bf16_linear(rt, rt->in.p, x_f32, rows, p, (float *)rt->out.p, nullptr, 1, rt->stream));
-    PW_HIP(hipMemcpyAsync(output, rt->out.p, n_out * 4, hipMemcpyDeviceToHost, rt->stream));
+    void *x;
+    call.activations(input, n_in, x_f32, x);
+    PW_TRY(call.upload());
+    PW_HIP(rt->out.ensure(HostCall::padded(n_out * 4)));
+    PW_TRY(enqueue_bf16_linear(rt, x, x_f32, rows, p, (float *)rt->out.p, nullptr, 1, rt->stream));
     uint32_t flags = 0;
-    PW_TRY(read_flags(rt, flags));
+    bool finite_out = true;  // a non-finite output raised the error word's round bit
+    PW_TRY(call.finish(output, n_out, flags, finite_out));
     if (stats) {
         stats->wall_ms = now_ms() - t0;
         stats->mapped_source_bytes = 0;
@@ -1123,9 +1211,8 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
         return fail(PW_ERR_SCHEDULE, "wide MoE input or schedule mismatch");
     const uint32_t H = experts[0].gate->columns, I = experts[0].gate->rows;
     const size_t n_in = (size_t)rows * H;
-    for (size_t i = 0; i < n_in; ++i)
-        if (!finite(input[i]))
-            return fail(PW_ERR_NONFINITE, "wide MoE input or schedule mismatch");
+    if (!all_finite(input, n_in))
+        return fail(PW_ERR_NONFINITE, "wide MoE input or schedule mismatch");
     // validation of src/wide_metal_moe.rs:858-938
     size_t total = 0;
     uint32_t max_count = 0;
@@ -1172,32 +1259,31 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
     TimerScope timer_scope(rt);
     StreamOrder order(rt, rt->stream);
     PW_HIP(order.err);
-    PW_TRY(reset_flags(rt));
+    HostCall call{rt};
+    const size_t ids_bytes = ids.size() * 4, table_bytes = table.size() * sizeof(ExpertPtrs);
+    PW_TRY(call.begin(HostCall::padded(n_in * 4) + 2 * HostCall::padded(ids_bytes) + HostCall::padded(table_bytes)));
     bool x_f32;
-    PW_TRY(stage_input(rt, input, n_in, x_f32));
-    PW_HIP(rt->route_ids.ensure(ids.size() * 4));
-    PW_HIP(rt->route_w.ensure(ws.size() * 4));
-    PW_HIP(rt->bank_table.ensure(table.size() * sizeof(ExpertPtrs)));
-    PW_HIP(hipMemcpyAsync(rt->route_ids.p, ids.data(), ids.size() * 4, hipMemcpyHostToDevice, rt->stream));
-    PW_HIP(hipMemcpyAsync(rt->route_w.p, ws.data(), ws.size() * 4, hipMemcpyHostToDevice, rt->stream));
-    PW_HIP(hipMemcpyAsync(rt->bank_table.p, table.data(), table.size() * sizeof(ExpertPtrs),
-                          hipMemcpyHostToDevice, rt->stream));
+    void *x, *d_ids, *d_ws, *d_table;
+    call.activations(input, n_in, x_f32, x);
+    std::memcpy(call.take(ids_bytes, d_ids), ids.data(), ids_bytes);
+    std::memcpy(call.take(ids_bytes, d_ws), ws.data(), ids_bytes);
+    std::memcpy(call.take(table_bytes, d_table), table.data(), table_bytes);
+    PW_TRY(call.upload());
     PW_TRY(ensure_moe(rt, rows, n_experts, H, I));
-    PW_HIP(rt->out.ensure(n_in * 4));
-    const pw::QuantJob qj{rt->in.p, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
+    PW_HIP(rt->out.ensure(HostCall::padded(n_in * 4)));
+    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
     bool quantised = false;
-    pw::launch_moe_schedule((const ExpertPtrs *)rt->bank_table.p, (const uint32_t *)rt->route_ids.p,
-                            (const float *)rt->route_w.p, rows, n_experts,
+    pw::launch_moe_schedule((const ExpertPtrs *)d_table, (const uint32_t *)d_ids, (const float *)d_ws, rows, n_experts,
                             std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, rows),
                             rt->d_flags, rt->stream, nullptr,
                             mode == PW_MODE_B ? &qj : nullptr, mode == PW_MODE_B ? &quantised : nullptr);
-    pw::launch_moe_layer(mode, (const ExpertPtrs *)rt->bank_table.p, rt->mb, rt->in.p, x_f32, rows,
+    pw::launch_moe_layer(mode, (const ExpertPtrs *)d_table, rt->mb, x, x_f32, rows,
                          std::min<uint32_t>(n_experts, rows * 8), max_count, H, I,
                          (float *)rt->out.p, nullptr, false, rt->d_flags, rt->stream, nullptr, quantised);
     PW_HIP(hipGetLastError());
-    PW_HIP(hipMemcpyAsync(output, rt->out.p, n_in * 4, hipMemcpyDeviceToHost, rt->stream));
     uint32_t flags = 0;
-    PW_TRY(read_flags(rt, flags));  // also completes the stream (ids/ws/table stay valid until here)
+    bool finite_out = true;
+    PW_TRY(call.finish(output, n_in, flags, finite_out));
     if (stats) {
         stats->wall_ms = now_ms() - t0;
         stats->unique_experts = (uint32_t)seen.size();
@@ -1208,9 +1294,8 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
     }
     if (flags)
         return fail(PW_ERR_GPU_FLAGS, "wide MoE semantic kernels set error flags %u", flags);
-    for (size_t i = 0; i < n_in; ++i)
-        if (!finite(output[i]))
-            return fail(PW_ERR_OUTPUT, "wide MoE produced non-finite output");
+    if (!finite_out)
+        return fail(PW_ERR_OUTPUT, "wide MoE produced non-finite output");
     return PW_OK;
 }
 

@@ -80,6 +80,37 @@ class WideExpertBinding:
     down: Projection
 
 
+# ExpertBindingC as a record, so that a batch's bindings are filled by columns
+_BINDING = np.dtype([("expert", "<u4"), ("count", "<u4"), ("positions", "<u8"), ("route_weights", "<u8"),
+                     ("gate", "<u8"), ("up", "<u8"), ("down", "<u8")])
+assert _BINDING.itemsize == ctypes.sizeof(_abi.ExpertBindingC)
+
+
+def _expert_bindings(experts):
+    """The C bindings of a batch and what keeps their pointers alive. The positions and weights of all
+    bindings sit in one array each: an array and a pointer object per binding were most of the call's host time."""
+    pos, weights, counts, pos_at, w_at = [], [], [], [], []
+    for b in experts:
+        p, w = b.positions, b.route_weights
+        if type(p) is not list or type(w) is not list:  # any array-like
+            p, w = np.ascontiguousarray(p, dtype=np.uint32), np.ascontiguousarray(w, dtype=np.float32)
+        counts.append(len(p))
+        pos_at.append(len(pos))
+        w_at.append(len(weights))
+        pos += p if type(p) is list else p.reshape(-1).tolist()
+        weights += w if type(w) is list else w.reshape(-1).tolist()
+    pos, weights = np.array(pos, dtype=np.uint32), np.array(weights, dtype=np.float32)
+    rec = np.zeros(len(counts), _BINDING)
+    rec["expert"] = [b.expert & 0xFFFFFFFF for b in experts]
+    rec["count"] = counts
+    rec["positions"] = np.array(pos_at, np.uint64) * 4 + np.uint64(pos.ctypes.data)
+    rec["route_weights"] = np.array(w_at, np.uint64) * 4 + np.uint64(weights.ctypes.data)
+    rec["gate"] = [b.gate.handle or 0 for b in experts]
+    rec["up"] = [b.up.handle or 0 for b in experts]
+    rec["down"] = [b.down.handle or 0 for b in experts]
+    return rec.ctypes.data_as(ctypes.POINTER(_abi.ExpertBindingC)), (rec, pos, weights)
+
+
 class ExpertBank:
     def __init__(self, handle: int, n_experts: int, hidden: int, intermediate: int, keep=None):
         self.handle = handle
@@ -300,15 +331,7 @@ class WideMoeRuntime:
         if x.ndim == 1:
             x = x.reshape(1, -1)
         rows, hidden = x.shape
-        arr = (_abi.ExpertBindingC * len(experts))()
-        keep = []
-        for i, b in enumerate(experts):
-            pos = np.ascontiguousarray(b.positions, dtype=np.uint32)
-            w = np.ascontiguousarray(b.route_weights, dtype=np.float32)
-            keep += [pos, w]
-            arr[i] = _abi.ExpertBindingC(b.expert, len(pos), pos.ctypes.data_as(_abi._u32p),
-                                         w.ctypes.data_as(_abi._f32p), b.gate.handle, b.up.handle,
-                                         b.down.handle)
+        arr, keep = _expert_bindings(experts)
         out = np.zeros((rows, hidden), np.float32)
         st = _abi.MoeStats()
         check(lib().pw_moe_execute(self.handle, mode, int(fused), x.ctypes.data_as(_abi._f32p), rows, arr,

@@ -166,3 +166,30 @@ def test_product_qkv_maps_match_oracle():
         assert P.full_qkv_scale_row(r) == O.full_qkv_scale_row(r)
     for r in list(range(0, 14848, 7)) + [14847, 14848, -1]:
         assert P.swa_qkv_source_row(r) == O.swa_qkv_source_row(r)
+
+
+def test_expert_bindings_by_columns():
+    """The batch's C bindings hold each binding's values, from lists, tuples and arrays of any integer
+    or float type, and from none."""
+    from prismwing_amd.runtime import _expert_bindings
+
+    class Proj:
+        def __init__(self, handle):
+            self.handle = handle
+
+    rng = np.random.default_rng(3)
+    batch = []
+    for e, form in enumerate((list, tuple, np.int64, np.float64, list, np.uint32)):
+        n = int(rng.integers(1, 33))
+        pos, w = rng.integers(0, 128, n), rng.standard_normal(n)
+        p = pos.tolist() if form is list else tuple(pos.tolist()) if form is tuple else pos.astype(form)
+        batch.append(P.WideExpertBinding(1000 - e, p, w.tolist() if form is list else w, Proj(3 * e + 1),
+                                         Proj(None if e == 2 else 3 * e + 2), Proj(2**46 + e)))
+    arr, keep = _expert_bindings(batch)
+    for i, b in enumerate(batch):
+        c = arr[i]
+        assert (c.expert, c.count) == (b.expert, len(b.positions))
+        assert [c.positions[j] for j in range(c.count)] == [int(v) for v in b.positions]
+        assert [c.route_weights[j] for j in range(c.count)] == np.asarray(b.route_weights, np.float32).tolist()
+        assert (c.gate, c.up, c.down) == (b.gate.handle, b.up.handle, b.down.handle)
+    assert len(_expert_bindings([])[1][0]) == 0
