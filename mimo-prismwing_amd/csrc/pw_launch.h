@@ -133,21 +133,15 @@ SplitPlan plan_split(uint32_t K, int mats, int ns, uint32_t max_cnt);
 void launch_moe_a_split(int mats, int ns, const SplitArgs &args, const SplitPlan &sp, uint32_t max_active,
                         hipStream_t stream);
 // gate/up split sums -> SwiGLU -> hidden as three bf16 planes [3][P][I]
-// BF16 wide linear (pw_bf16.hip): w bf16 [R][K] (K a multiple of 128), x bf16 planes [NS][W][K],
-// split-K partials [KS][W][R] f32 summed in split order by the reduce kernel.
-struct Bf16Args {
-    const uint16_t *w;
-    const uint16_t *x;
-    const float *xf;  // f32 activations [W][K], W <= 16, split into the three planes while staging (x unused)
-    size_t x_plane;
-    uint32_t K, R, W, KS;
-    float *partial;
-};
-// 128-column blocks per wave for K (the K split is 128 * that); at most `lds_cap` bytes of LDS
-// for NS planes of W activation rows.
-int bf16_blocks_per_wave(uint32_t K, int planes, uint32_t W, size_t lds_cap);
-void launch_bf16_linear(const Bf16Args &a, int planes, int bpw, float *y32, uint16_t *y16, uint32_t round_f32,
-                        uint32_t *flags, hipStream_t stream);
+// BF16 wide linear (pw_bf16.hip): w bf16 [R][K] (K a multiple of 128), x bf16 or f32 [W][K]; partial:
+// bf16_shares(K, R) x W x R floats when that is above one.
+uint32_t bf16_shares(uint32_t K, uint32_t R);
+void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W, uint32_t K, uint32_t R, float *partial,
+                        float *y32, uint16_t *y16, uint32_t round_f32, uint32_t *flags, hipStream_t stream);
+// ks share sums of n outputs added in share order: f32 rounded to bf16 or raw, bf16 bits; a non-finite
+// rounded value raises FLAG_ROUND_NONFINITE.
+void launch_round_output(const float *y, uint32_t ks, uint32_t n, float *out_f32, uint16_t *out_bf16, bool raw,
+                         uint32_t *flags, hipStream_t stream);
 
 // Gate/up with the SwiGLU fused and no split partials (pw_moe_a.hip), when the routed rows fit the
 // LDS stage; returns false (nothing launched) otherwise.

@@ -1175,6 +1175,13 @@ __global__ __launch_bounds__(256) void round_output_kernel(const float *__restri
 }
 
 // ------------------------------------------------------------------------------- launchers
+void launch_round_output(const float *y, uint32_t ks, uint32_t n, float *out_f32, uint16_t *out_bf16, bool raw,
+                         uint32_t *flags, hipStream_t stream)
+{
+    hipLaunchKernelGGL(round_output_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, y, ks, (size_t)n, n, out_f32,
+                       out_bf16, raw ? 1u : 0u, flags);
+}
+
 bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const float *weights,
                          uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb, uint32_t piece_rows,
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles, const QuantJob *quant,
@@ -1470,11 +1477,8 @@ void launch_expert_forward(uint32_t mode, const ExpertPtrs &ep, const MoeBuffers
         launch_quant_group128(mb.hidden, true, rows, I, mb.hq, mb.hs, flags, stream);
     const uint32_t ks = launch_expert_down(ep, codes, codes ? (const void *)mb.hq : mb.hidden, mb.hs, rows, H, I, mb.y,
                                            out_f32, out_bf16, raw, flags, stream);
-    if (ks > 1) {
-        const uint32_t n = rows * H;
-        hipLaunchKernelGGL(round_output_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, mb.y, ks, (size_t)n, n,
-                           out_f32, out_bf16, raw ? 1u : 0u, flags);
-    }
+    if (ks > 1)
+        launch_round_output(mb.y, ks, rows * H, out_f32, out_bf16, raw, flags, stream);
 }
 
 }  // namespace pw

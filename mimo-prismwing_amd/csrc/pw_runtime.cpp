@@ -1056,30 +1056,11 @@ int pw_bf16_bind_device(pw_runtime *rt, const void *weight, uint32_t rows, uint3
 static int enqueue_bf16_linear(pw_runtime *rt, const void *x, bool x_f32, uint32_t rows, const pw_projection *p,
                                float *y32, uint16_t *y16, uint32_t round_f32, hipStream_t stream)
 {
-    const int planes = x_f32 ? 3 : 1;
-    const uint16_t *xp = (const uint16_t *)x;
-    // f32 rows: up to 16 are split into their planes inside the projection's staging; more go
-    // through a split launch first
-    const bool split_inside = x_f32 && rows <= 16;
-    if (x_f32 && !split_inside) {
-        const size_t n = (size_t)rows * p->columns;
-        PW_HIP(rt->lin_planes.ensure(3 * n * 2));
-        pw::launch_split_planes((const float *)x, (uint32_t)n, (uint16_t *)rt->lin_planes.p, stream);
-        xp = (const uint16_t *)rt->lin_planes.p;
-    }
-    const int bpw = pw::bf16_blocks_per_wave(p->columns, planes, rows, 65536);
-    pw::Bf16Args a{};
-    a.w = (const uint16_t *)p->w;
-    a.x = xp;
-    a.xf = split_inside ? (const float *)x : nullptr;
-    a.x_plane = (size_t)rows * p->columns;
-    a.K = p->columns;
-    a.R = p->rows;
-    a.W = rows;
-    a.KS = p->columns / (128u * bpw);
-    PW_HIP(rt->bf16_partial.ensure((size_t)a.KS * rows * p->rows * 4));
-    a.partial = (float *)rt->bf16_partial.p;
-    pw::launch_bf16_linear(a, planes, bpw, y32, y16, round_f32, rt->d_flags, stream);
+    const uint32_t ks = pw::bf16_shares(p->columns, p->rows);
+    if (ks > 1)
+        PW_HIP(rt->bf16_partial.ensure((size_t)ks * rows * p->rows * 4));
+    pw::launch_bf16_linear((const uint16_t *)p->w, x, x_f32, rows, p->columns, p->rows, (float *)rt->bf16_partial.p, y32,
+                           y16, round_f32, rt->d_flags, stream);
     PW_HIP(hipGetLastError());
     return PW_OK;
 }

@@ -30,11 +30,13 @@ struct WideXBytes {
     static constexpr int value = XT == WX_F32 ? 4 : XT == WX_BF16 ? 2 : 1;
 };
 
-// Columns per step: a block, or half a block where two steps of eight waves would not fit in LDS
-// with whole blocks of f32 rows (24 rows: 196 KB; half blocks 98 KB).
+constexpr int WAVES = 8;  // of a workgroup; they split its share of K
+
+// Columns per step: a block, or half a block where two steps of all waves would take more than 128 KB
+// of LDS (24 f32 rows and eight waves: 196 KB with whole blocks).
 template <int XT, int XR>
 struct WideStep {
-    static constexpr int value = XT == WX_F32 && XR > 16 ? 64 : 128;
+    static constexpr int value = 128 * WideXBytes<XT>::value * XR * 2 * WAVES <= 131072 ? 128 : 64;
 };
 
 // What a workgroup's 16-row tiles are, and what becomes of their sums:
@@ -44,14 +46,16 @@ struct WideStep {
 //              SwiGLU -> hidden rows [W][N] f32 (mode B: bf16-staged).
 //   WK_DOWN    rows of one expert's down matrix, K in KS shares of consecutive workgroups; one share:
 //              the output rows rounded, flagged if not finite; more: share sums [KS][W][N].
-enum WideKind : int { WK_PROJ = 0, WK_GATEUP = 1, WK_DOWN = 2 };
+//   WK_BF16    rows of a bf16 weight [N][K] (mode A activations, no scales), K in KS shares as above;
+//              the output rows, rounded or not, flagged if not finite.
+enum WideKind : int { WK_PROJ = 0, WK_GATEUP = 1, WK_DOWN = 2, WK_BF16 = 3 };
 
 struct WideArgs {
     const ProjTile *tiles;         // WK_PROJ
-    const uint8_t *w0, *w1;        // gate and up, or down [N][K]
+    const uint8_t *w0, *w1;        // gate and up, down [N][K], or the bf16 weight's bytes
     const float *s0, *s1;          // ... and their block scales
-    float *partial;                // WK_DOWN with KS > 1
-    uint32_t KS;                   // WK_DOWN
+    float *partial;                // with KS > 1: share sums [KS][W][N]
+    uint32_t KS;                   // WK_DOWN, WK_BF16
     uint32_t *flags;
     uint32_t n_tiles;
     const void *x;         // activations [W][K]: bf16, f32 or e4m3 codes
@@ -102,17 +106,18 @@ __device__ __forceinline__ void lds_read(const uint32_t (&a)[4], u32x4 (&v)[4])
                  : "memory");
 }
 
-template <int XT, int XR, int RT>
+template <int KIND, int XT, int XR, int RT>
 struct WideStream {
     static constexpr int SC = WideStep<XT, XR>::value;
     static constexpr int XB = WideXBytes<XT>::value;
     static constexpr int NT = (XR + 15) / 16;             // 16-token tiles
     static constexpr int UPR = SC * XB / 16;              // 16-byte units per staged row
     static constexpr int XC = XR * UPR / 64;              // activation copies per step
-    static constexpr int WL = SC / 64;                    // weight loads per tile and step
+    static constexpr int WB = KIND == WK_BF16 ? 2 : 1;    // bytes of a weight
+    static constexpr int WL = SC * WB / 64;               // weight loads per tile and step
     static constexpr int SLOT = XR * UPR;                 // units per step slot
-    static constexpr int RED = 8 * RT * NT * 64;          // split partials, in the slots' place
-    static constexpr int LDS = 16 * SLOT > RED ? 16 * SLOT : RED;
+    static constexpr int RED = WAVES * RT * NT * 64;          // split partials, in the slots' place
+    static constexpr int LDS = 2 * WAVES * SLOT > RED ? 2 * WAVES * SLOT : RED;
     static_assert(XR * UPR % 64 == 0, "whole copies");
     static_assert(LDS * 16 <= 160 * 1024, "a workgroup's LDS");
 
@@ -139,9 +144,9 @@ struct WideStream {
 template <int KIND, int XT, int XR, int RT>
 __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
 {
-    using S = WideStream<XT, XR, RT>;
+    using S = WideStream<KIND, XT, XR, RT>;
     constexpr int NT = S::NT, SC = S::SC, WL = S::WL, XC = S::XC;
-    __shared__ uint4 lds_w[S::LDS];  // per wave two step slots; then the split partials [8][RT * NT][64]
+    __shared__ uint4 lds_w[S::LDS];  // per wave two step slots; then the split partials [WAVES][RT * NT][64]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, r16 = lane & 15;
@@ -149,8 +154,9 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
     const char *x = (const char *)args.x;
     uint4 *slots = lds_w + (size_t)wave * 2 * S::SLOT;
 
-    constexpr int WQ = XT == WX_CODES ? 32 : 16;  // weight bytes of a lane's q within a row's load
-    const uint32_t group = KIND == WK_DOWN ? blockIdx.x / args.KS : blockIdx.x;
+    constexpr int WQ = XT == WX_CODES || KIND == WK_BF16 ? 32 : 16;  // weight bytes of a lane's q in a row
+    constexpr bool SHARES = KIND == WK_DOWN || KIND == WK_BF16;
+    const uint32_t group = SHARES ? blockIdx.x / args.KS : blockIdx.x;
     const uint8_t *wrow[RT];
     const float *ws[RT];
     if constexpr (KIND == WK_PROJ) {
@@ -175,7 +181,10 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const uint32_t t0 = group * RT + r, t = t0 < args.n_tiles ? t0 : args.n_tiles - 1;
-            if constexpr (KIND == WK_GATEUP) {
+            if constexpr (KIND == WK_BF16) {
+                const uint32_t row = t * 16 + r16;
+                wrow[r] = args.w0 + (size_t)(row < args.N ? row : args.N - 1) * K * 2 + q * WQ;
+            } else if constexpr (KIND == WK_GATEUP) {
                 wrow[r] = (r16 < 8 ? args.w0 : args.w1) + (size_t)(t * 8 + (r16 & 7)) * K + q * WQ;
                 ws[r] = (q < 2 ? args.s0 : args.s1) + (size_t)(t * 8 >> 7) * blocks;
             } else {
@@ -186,12 +195,12 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
     }
     // this wave's blocks (of its workgroup's share of K), and its steps
     uint32_t c0 = 0, cn = blocks;
-    if constexpr (KIND == WK_DOWN) {
+    if constexpr (SHARES) {
         const uint32_t share = blockIdx.x % args.KS;
         c0 = share * blocks / args.KS;
         cn = (share + 1) * blocks / args.KS - c0;
     }
-    const uint32_t b0 = c0 + (uint32_t)wave * cn / 8, b1 = c0 + ((uint32_t)wave + 1) * cn / 8;
+    const uint32_t b0 = c0 + (uint32_t)wave * cn / WAVES, b1 = c0 + ((uint32_t)wave + 1) * cn / WAVES;
     const uint32_t steps = (b1 - b0) * (128 / SC);
 
     f32x4 total[RT][NT], acc[RT][NT];
@@ -215,9 +224,10 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
                 sa[s][nt] = load_g(args.x_scales + (size_t)(row < W ? row : W - 1) * blocks + b);
             }
         }
+        if constexpr (KIND != WK_BF16)
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
-            sw[s][r] = load_g(ws[r] + b);
+            for (int r = 0; r < RT; ++r)
+                sw[s][r] = load_g(ws[r] + b);
         asm volatile("" ::: "memory");
         S::copy_x(x, W, K, col, slots + s * S::SLOT, lane);
         asm volatile("" ::: "memory");
@@ -225,7 +235,9 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
         for (int r = 0; r < RT; ++r)
 #pragma unroll
             for (int h = 0; h < WL; ++h)
-                wv[s][r][h] = *(global_u32x4 *)(wrow[r] + col + h * (XT == WX_CODES ? 16 : 64));
+                wv[s][r][h] = *(global_u32x4 *)(wrow[r] + (size_t)col * S::WB +
+                                                (KIND == WK_BF16 ? (h / 2) * 128 + (h % 2) * 16
+                                                                 : h * (XT == WX_CODES ? 16 : 64)));
         asm volatile("" ::: "memory");
     };
     // N loads issued after step s's own may be outstanding
@@ -261,10 +273,15 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
             }
         } else {
 #pragma unroll
-            for (int h = 0; h < WL; ++h) {
+            for (int h = 0; h < SC / 64; ++h) {
                 bf16x8 a[RT][2];
 #pragma unroll
                 for (int r = 0; r < RT; ++r) {
+                    if constexpr (KIND == WK_BF16) {
+                        a[r][0] = __builtin_bit_cast(bf16x8, wv[s][r][2 * h]);
+                        a[r][1] = __builtin_bit_cast(bf16x8, wv[s][r][2 * h + 1]);
+                        continue;
+                    }
                     a[r][0] = fp8x8_to_bf16x8(wv[s][r][h][0], wv[s][r][h][1]);
                     a[r][1] = fp8x8_to_bf16x8(wv[s][r][h][2], wv[s][r][h][3]);
                 }
@@ -318,7 +335,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
                     }
                 }
             }
-            if constexpr (SC == 128 || s == 1) {  // a block is complete
+            if constexpr (KIND != WK_BF16 && (SC == 128 || s == 1)) {  // a block is complete
 #pragma unroll
                 for (int r = 0; r < RT; ++r)
 #pragma unroll
@@ -367,7 +384,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
-            red[(wave * RT * NT + r * NT + nt) * 64 + lane] = total[r][nt];
+            red[(wave * RT * NT + r * NT + nt) * 64 + lane] = KIND == WK_BF16 ? acc[r][nt] : total[r][nt];
     __syncthreads();
     if (wave >= RT * NT)
         return;
@@ -376,7 +393,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
         return;
     f32x4 sum = red[wave * 64 + lane];
 #pragma unroll
-    for (int w = 1; w < 8; ++w) {
+    for (int w = 1; w < WAVES; ++w) {
         const f32x4 o = red[(w * RT * NT + wave) * 64 + lane];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -420,6 +437,29 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
         *(float4 *)(args.y_f32 + (size_t)token * args.N + t * 8 + q * 4) = make_float4(o[0], o[1], o[2], o[3]);
         if (bad)
             raise_flag(args.flags, FLAG_SWIGLU_NONFINITE);
+    } else if constexpr (KIND == WK_BF16) {
+        if (token >= W)
+            return;
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t row = t * 16 + q * 4 + i;
+            if (row >= args.N)
+                continue;
+            const size_t at = (size_t)token * args.N + row;
+            if (args.KS > 1) {
+                args.partial[(size_t)(blockIdx.x % args.KS) * W * args.N + at] = sum[i];
+                continue;
+            }
+            const float r = round_bf16(sum[i]);
+            bad |= !finite_f32(r);
+            if (args.y_f32)
+                args.y_f32[at] = args.round_f32 ? r : sum[i];
+            if (args.y_bf16)
+                args.y_bf16[at] = (uint16_t)(f32_bits(r) >> 16);
+        }
+        if (bad)
+            raise_flag(args.flags, FLAG_ROUND_NONFINITE);
     } else {
         if (token >= W)
             return;
@@ -468,7 +508,7 @@ static inline int pick_rt(int xt, uint32_t W, uint32_t n_tiles)
 template <int KIND, int XT, int XR>
 static void launch_wide_rt(const WideArgs &args, int rt, hipStream_t stream)
 {
-    const dim3 grid((args.n_tiles + rt - 1) / rt * (KIND == WK_DOWN ? args.KS : 1u)), block(512);
+    const dim3 grid((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND == WK_DOWN || KIND == WK_BF16 ? args.KS : 1u)), block(512);
     if (rt == 4)
         hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 4>), grid, block, 0, stream, args);
     else if (rt == 2)

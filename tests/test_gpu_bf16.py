@@ -150,3 +150,25 @@ def test_fail_closed(rt):
     with pytest.raises(P.PwError, match="GPU_FLAGS"):
         rt.execute_bf16_linear(np.ones((1, 256), np.float32), proj_inf)
     assert rt.take_flags() == 0
+
+
+@pytest.mark.parametrize("n,k", [(24, 128), (24, 5120), (1100, 5248), (4104, 1152), (8200, 1152), (2100, 640)])
+def test_tile_step_and_share_edges(rt, n, k):
+    """Workgroups of one, two and four 16-row tiles with partial last tiles and a partial last
+    workgroup, four, two and one K shares (24, 1100 and the other rows), waves with no, one and
+    several steps, at staged-row edges. Raw sums of exact products against 64 bits: chains of at most
+    5248 / 32 + 8 + 3 f32 roundings per element over random terms (2e-6 of the 2-norm)."""
+    import torch
+    from helpers import from_bf16_bits, rel_l2
+    rng = np.random.default_rng(n + k)
+    w = _weights(rng, n, k)
+    proj = rt.bind_bf16(w)
+    wd = from_bf16_bits(w).astype(np.float64)
+    xf = rng.standard_normal((32, k)).astype(np.float32)
+    xb = WL.bf16_round_np(xf)
+    ref_f, ref_b = xf.astype(np.float64) @ wd.T, xb.astype(np.float64) @ wd.T
+    for rows in (1, 4, 5, 8, 9, 16, 17, 24, 32):
+        for x, ref, bf in ((xf, ref_f, False), (xb, ref_b, True)):
+            assert rel_l2(_device(torch, rt, proj, x[:rows], rows, P.DTYPE_F32_RAW, bf), ref[:rows]) <= RAW_TOL, (rows, bf)
+        raw = _device(torch, rt, proj, xb[:rows], rows, P.DTYPE_F32_RAW, True)
+        assert np.array_equal(_device(torch, rt, proj, xb[:rows], rows, P.DTYPE_BF16, True), WL.bf16_round_np(raw)), rows
