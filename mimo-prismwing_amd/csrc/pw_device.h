@@ -430,4 +430,25 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *tmp, uint3
     return r;
 }
 
+// Two exclusive prefix sums over the workgroup at once, with one barrier: every wave adds up the
+// per-wave totals itself. `tmp` holds 32 words of LDS, not reused before the caller's next barrier.
+__device__ __forceinline__ void block_exclusive_scan2(uint32_t v0, uint32_t v1, uint32_t *tmp, uint32_t &x0, uint32_t &x1,
+                                                      uint32_t &total0, uint32_t &total1)
+{
+    const uint32_t lane = threadIdx.x & 63, nw = (blockDim.x + 63) >> 6;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t i0 = wave_inclusive_scan(v0), i1 = wave_inclusive_scan(v1);
+    if (lane == 63) {
+        tmp[wave] = i0;
+        tmp[16 + wave] = i1;
+    }
+    __syncthreads();
+    const uint32_t w0 = lane < nw ? tmp[lane] : 0u, w1 = lane < nw ? tmp[16 + lane] : 0u;
+    const uint32_t s0 = wave_inclusive_scan(w0), s1 = wave_inclusive_scan(w1);
+    x0 = (uint32_t)__builtin_amdgcn_readlane((int)(s0 - w0), (int)wave) + i0 - v0;
+    x1 = (uint32_t)__builtin_amdgcn_readlane((int)(s1 - w1), (int)wave) + i1 - v1;
+    total0 = (uint32_t)__builtin_amdgcn_readlane((int)s0, 63);
+    total1 = (uint32_t)__builtin_amdgcn_readlane((int)s1, 63);
+}
+
 }  // namespace pw

@@ -229,19 +229,20 @@ struct PfTileTable {
 // Bytes of MoeBuffers::sched the schedule of `rows` token rows over E experts needs (0 for the
 // batches scheduled in one workgroup).
 size_t moe_sched_scratch_bytes(uint32_t rows, uint32_t E);
-// Activation rows [rows][K] (f32 or bf16) for the dynamic FP8 quantiser: codes [rows][K] e4m3 and
-// scales [rows][K / 128].
+// Activation rows [rows][K] to prepare for the projections: f32 or bf16 for the dynamic FP8 quantiser
+// (codes [rows][K] e4m3 and scales [rows][K / 128]), or with `planes` f32 rows to split into their
+// three bf16 planes [3][rows][K].
 struct QuantJob {
     const void *x;
     uint32_t f32, rows, K;
     uint8_t *codes;
     float *scales;
+    uint16_t *planes;
 };
-// Returns true when the batch took the long-batch schedule, which also writes the prefill's
-// m-tile table when given tiles and quantises `quant` when given (in the same launch as its plan);
-// false: the caller launches both itself. With `quantised` non-null, a decode batch's one-wave
-// schedule also quantises `quant` (in other workgroups of its launch); *quantised tells whether
-// `quant` was done by either path.
+// Given tiles and `quant`, a schedule of more than eight rows also writes the prefill's m-tile table
+// and prepares `quant` (in other workgroups of the same launch) and returns true; false: the caller
+// launches both itself. With `quantised` non-null, a decode batch's schedule also prepares `quant`;
+// *quantised tells whether it did.
 // piece_rows: the batch's projections take mb.pieces, entries of at most that many slots
 // (moe_piece_rows of the layer that follows; 0: no pieces; batches of at most 128 rows).
 uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows);
@@ -262,7 +263,7 @@ struct OneTokenRoutes {
 void launch_moe_layer(uint32_t mode, const ExpertPtrs *bank, const MoeBuffers &mb, const void *x,
                       bool x_f32, uint32_t rows, uint32_t max_active, uint32_t max_count, uint32_t H,
                       uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw, uint32_t *flags,
-                      hipStream_t stream, const OneTokenRoutes *routes = nullptr, bool x_quantised = false,
+                      hipStream_t stream, const OneTokenRoutes *routes = nullptr, bool x_prepared = false,
                       const RouteJob *job = nullptr);
 
 // Device router (pw_router.hip): x [rows][K] (f32 or bf16) and router weights [E][K] (f32 or bf16)
@@ -303,11 +304,11 @@ void launch_silu_table(uint16_t *table, hipStream_t stream);
 void launch_swiglu_staged(const float *gate, const float *up, uint32_t n, const uint16_t *silu_table, float *out,
                           uint32_t *flags, hipStream_t stream);
 uint32_t prefill_max_tiles(uint32_t rows, uint32_t E);
-// scheduled_long: launch_moe_schedule returned true for this batch, given pb's tile table and the
+// scheduled: launch_moe_schedule returned true for this batch, given pb's tile table and the
 // QuantJob of x into mb.xq / mb.xs (the m-tile table and the activation codes are in place).
 void launch_moe_prefill(const ExpertPtrs *bank, const MoeBuffers &mb, const PrefillBuffers &pb, const void *x,
                         bool x_f32, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, float *out_f32,
-                        uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream, bool scheduled_long);
+                        uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream, bool scheduled);
 
 void launch_expert_forward(uint32_t mode, const ExpertPtrs &ep, const MoeBuffers &mb, const void *x, bool x_f32,
                            uint32_t rows, uint32_t H, uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw,

@@ -111,14 +111,52 @@ static uint32_t piece_bound(uint32_t rows, uint32_t max_active, uint32_t piece_r
     return U + (P - U) / piece_rows;
 }
 
+// Group `group` of qj (128 columns of a row) by 16 lanes: quantised, or split into its planes.
+__device__ __forceinline__ void prepare_group(const QuantJob &qj, uint32_t group, uint32_t lane16, uint32_t *flags)
+{
+    if (group >= qj.rows * (qj.K >> 7))
+        return;  // whole 16-lane groups leave together
+    if (qj.planes) {
+        const size_t base = (size_t)group * 128 + lane16 * 8, plane = (size_t)qj.rows * qj.K;
+        float v[8];
+        load_act8<float>((const float *)qj.x + base, v);
+        uint32_t pk[3][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint16_t h0, m0, l0, h1, m1, l1;
+            split3_bf16(v[2 * e], h0, m0, l0);
+            split3_bf16(v[2 * e + 1], h1, m1, l1);
+            pk[0][e] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+            pk[1][e] = (uint32_t)m0 | ((uint32_t)m1 << 16);
+            pk[2][e] = (uint32_t)l0 | ((uint32_t)l1 << 16);
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+            *(uint4 *)(qj.planes + p * plane + base) = make_uint4(pk[p][0], pk[p][1], pk[p][2], pk[p][3]);
+    } else if (qj.f32) {
+        quant_group128_team<float>((const float *)qj.x, group, lane16, qj.codes, qj.scales, flags);
+    } else {
+        quant_group128_team<uint16_t>((const uint16_t *)qj.x, group, lane16, qj.codes, qj.scales, flags);
+    }
+}
+
+// One workgroup schedules a batch of 9 to 128 rows; the others, when given a QuantJob, prepare the
+// activation rows meanwhile (64 groups of 128 columns each). With a tile table, also the prefill's
+// m-tiles, one per routed expert (at most 128 slots each, a tile's). Latency-bound: the three prefix
+// sums share one barrier (trace, 32 rows of 256 experts: 12.5 us, and 5.1 us for the quantiser's own
+// launch, -> PW_SCHED_US us in all).
 __global__ __launch_bounds__(1024) void moe_schedule_kernel(
     const ExpertPtrs *__restrict__ bank, const uint32_t *__restrict__ ids,
     const float *__restrict__ weights, uint32_t rows, uint32_t E, uint32_t max_active, uint32_t with_prefix,
     MoePlan *plan, uint32_t *__restrict__ active_expert, uint32_t *__restrict__ active_offset,
     ActiveExpert *__restrict__ active, uint32_t *__restrict__ placement_pos, float *__restrict__ placement_w,
     uint32_t *__restrict__ row_slots, ActiveExpert *__restrict__ pieces, uint32_t max_pieces, uint32_t piece_rows,
-    uint32_t *flags)
+    uint32_t *flags, const PfTileTable tt, const QuantJob qj)
 {
+    if (blockIdx.x > 0) {
+        prepare_group(qj, (blockIdx.x - 1) * 64 + (threadIdx.x >> 4), threadIdx.x & 15, flags);
+        return;
+    }
     extern __shared__ uint32_t lds[];
     const uint32_t words = (rows + 31) >> 5;
     uint32_t *mask = lds;                              // [E][words]
@@ -169,9 +207,16 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
                 pref[e * words + w] = (uint16_t)c;
             c += __popc(mask[e * words + w]);
         }
-    uint32_t total, n_active;
-    const uint32_t off = block_exclusive_scan(c, s_scan, &total);
-    const uint32_t act = block_exclusive_scan(c ? 1u : 0u, s_scan, &n_active);
+    // slots and pieces in one word each of the first sum (at most 1024 of either)
+    const uint32_t np = (c + piece_rows - 1) / piece_rows;
+    uint32_t off, act, total, n_active;
+    block_exclusive_scan2(c | (np << 16), c ? 1u : 0u, s_scan, off, act, total, n_active);
+    const uint32_t pbase = off >> 16, n_pieces = total >> 16;
+    off &= 0xffffu;
+    total &= 0xffffu;
+    const uint32_t most = wave_max_u32(c);
+    if ((tid & 63) == 0)
+        atomicMax(&s_max, most);
     if (e < E) {
         offset[e] = off;
         if (c) {
@@ -198,16 +243,19 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
                 dst[3] = u32x4{off, c, tw[0], tw[1]};
                 dst[4] = u32x4{tw[2], tw[3], tw[4], tw[5]};
                 dst[5] = u32x4{tw[6], tw[7], 0u, 0u};
+                if (tt.tiles) {  // PfTileDesc: ExpertPtrs, slot0, cnt, expert, pad
+                    u32x4 *tile = (u32x4 *)(tt.tiles + act);
+                    tile[0] = ep0;
+                    tile[1] = ep1;
+                    tile[2] = ep2;
+                    tile[3] = u32x4{off, c, e, 0u};
+                }
             }
-            atomicMax(&s_max, c);
         }
     }
     if (tid == 0)
         active_offset[n_active] = total;
     if (max_pieces) {  // (uniform) the projections' entries of at most piece_rows slots
-        const uint32_t np = (c + piece_rows - 1) / piece_rows;
-        uint32_t n_pieces;
-        const uint32_t pbase = block_exclusive_scan(np, s_scan, &n_pieces);
         uint32_t w = 0, bits = np ? mask[e * words] : 0u;
         for (uint32_t i = 0; i < np; ++i) {
             uint32_t tw[PIECE_MAX_ROWS / 2] = {};
@@ -267,6 +315,8 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
         plan->n_active = n_active;
         plan->n_placements = total;
         plan->max_count = s_max;
+        if (tt.tiles)
+            *tt.n_tiles = n_active;
         plan->rejected = (s_bad || total != P) ? 1u : 0u;
         if (s_bad || total != P)
             raise_flag(flags, FLAG_SCHEDULE);
@@ -375,12 +425,7 @@ __global__ __launch_bounds__(1024) void moe_sched_plan_kernel(
 {
     if (blockIdx.x > 0) {
         const uint32_t group = (blockIdx.x - 1) * 64 + (threadIdx.x >> 4);
-        if (group < qj.rows * (qj.K >> 7)) {  // whole 16-lane groups leave together
-            if (qj.f32)
-                quant_group128_team((const float *)qj.x, group, threadIdx.x & 15, qj.codes, qj.scales, flags);
-            else
-                quant_group128_team((const uint16_t *)qj.x, group, threadIdx.x & 15, qj.codes, qj.scales, flags);
-        }
+        prepare_group(qj, group, threadIdx.x & 15, flags);
         return;
     }
     __shared__ uint32_t s_scan[48], s_bad, s_max;
@@ -758,12 +803,7 @@ __global__ __launch_bounds__(64) void moe_schedule_wave_kernel(
         // workgroups 1.. quantise the activation rows of qj (four 128-column groups each) while
         // workgroup 0 schedules
         const uint32_t group = (blockIdx.x - 1) * 4 + ((uint32_t)lane >> 4);
-        if (group < qj.rows * (qj.K >> 7)) {
-            if (qj.f32)
-                quant_group128_team<float>((const float *)qj.x, group, lane & 15, qj.codes, qj.scales, flags);
-            else
-                quant_group128_team<uint16_t>((const uint16_t *)qj.x, group, lane & 15, qj.codes, qj.scales, flags);
-        }
+        prepare_group(qj, group, threadIdx.x & 15, flags);
         return;
     }
     const uint32_t P = rows * 8;
@@ -845,12 +885,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     if (blockIdx.x > 0) {
         // 32 128-column groups per workgroup (16 lanes each)
         const uint32_t group = (blockIdx.x - 1) * 32 + (threadIdx.x >> 4);
-        if (group < qj.rows * (qj.K >> 7)) {
-            if (qj.f32)
-                quant_group128_team<float>((const float *)qj.x, group, lane & 15, qj.codes, qj.scales, flags);
-            else
-                quant_group128_team<uint16_t>((const uint16_t *)qj.x, group, lane & 15, qj.codes, qj.scales, flags);
-        }
+        prepare_group(qj, group, threadIdx.x & 15, flags);
         return;
     }
     const uint32_t units = E * 3;  // 16-byte units of the table
@@ -1188,7 +1223,7 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
                          bool *quantised)
 {
     const uint32_t max_pieces = piece_rows ? piece_bound(rows, max_active, piece_rows) : 0u;
-    bool long_batch = false;
+    bool complete = false;
     if (quantised)
         *quantised = false;
     const uint32_t words = (rows + 31) >> 5;
@@ -1216,12 +1251,19 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
         if (quant_wgs)
             *quantised = true;
     }
-    else if (rows <= SCHED_WG_MAX_ROWS)
-        hipLaunchKernelGGL(moe_schedule_kernel, dim3(1), dim3(1024), lds, stream, bank, ids, weights, rows,
+    else if (rows <= SCHED_WG_MAX_ROWS) {
+        const bool prefill = tiles && quant;
+        const PfTileTable tt = prefill ? *tiles : PfTileTable{nullptr, nullptr, 0};
+        const QuantJob qj = quant && (prefill || quantised) ? *quant : QuantJob{};
+        const uint32_t quant_wgs = (qj.rows * (qj.K >> 7) + 63) / 64;
+        complete = prefill;
+        if (quantised && quant)
+            *quantised = true;
+        hipLaunchKernelGGL(moe_schedule_kernel, dim3(1 + quant_wgs), dim3(1024), lds, stream, bank, ids, weights, rows,
                            E, max_active, with_prefix, mb.plan, mb.active_expert, mb.active_offset, mb.active,
                            mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces,
-                           piece_rows ? piece_rows : 1u, flags);
-    else {
+                           piece_rows ? piece_rows : 1u, flags, tt, qj);
+    } else {
         // rows <= 4096 (SCHED_MAX_WORDS words) and E <= 1024 (one plan thread per expert)
         const SchedScratch ss = sched_carve(mb.sched, rows, E, nullptr);
         const uint32_t nwg = (rows + 63) / 64;
@@ -1233,14 +1275,14 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
         hipLaunchKernelGGL(moe_sched_plan_kernel, dim3(1 + quant_wgs), dim3(1024), 0, stream, bank, rows, E,
                            max_active, ss, mb.plan, mb.active_expert, mb.active_offset, mb.active,
                            mb.placement_pos, mb.placement_w, mb.row_slots, flags, tt, qj);
-        long_batch = true;
+        complete = true;
         if (quantised && quant)
             *quantised = true;
         hipLaunchKernelGGL(moe_sched_place_kernel, dim3(nwg), dim3(64), 0, stream, ids, weights, rows, E, max_active,
                            ss, mb.plan, mb.active, mb.placement_pos, mb.placement_w, mb.row_slots);
     }
     timer_end(t, stream);
-    return long_batch;
+    return complete;
 }
 
 // Mode A: gate/up (+SwiGLU) then down, both as split-K expert projections (pw_moe_a.hip).
@@ -1255,8 +1297,8 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
                               uint32_t placements, uint32_t max_active, uint32_t max_count, uint32_t H,
                               uint32_t I, uint32_t *flags, hipStream_t stream, const DirectOut *direct = nullptr,
                               const ExpertPtrs *bank = nullptr,
-                              const OneTokenRoutes *routes = nullptr, const RouteJob *job = nullptr,
-                              bool *job_done = nullptr)
+                              const OneTokenRoutes *routes = nullptr, bool x_prepared = false,
+                              const RouteJob *job = nullptr, bool *job_done = nullptr)
 {
     // A routed batch runs both projections on the schedule's pieces of each expert's slots, so their
     // LDS stages hold piece_rows rows instead of as many as the batch could send one expert (an
@@ -1273,7 +1315,8 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     const uint32_t cnt = pieces ? piece_rows : max_count;
     const uint16_t *xp = (const uint16_t *)x;
     if (x_f32) {
-        launch_split_planes((const float *)x, rows * H, mb.x_planes, stream);
+        if (!x_prepared)
+            launch_split_planes((const float *)x, rows * H, mb.x_planes, stream);
         xp = mb.x_planes;
     }
     SplitArgs ga{};
@@ -1405,12 +1448,12 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
                                 bool x_f32, uint32_t rows, uint32_t placements, uint32_t max_active,
                                 uint32_t max_count, uint32_t H, uint32_t I, uint32_t *flags, hipStream_t stream,
                                 const DirectOut *direct = nullptr, const OneTokenRoutes *routes = nullptr,
-                                bool x_quantised = false, const RouteJob *job = nullptr, bool *job_done = nullptr)
+                                bool x_prepared = false, const RouteJob *job = nullptr, bool *job_done = nullptr)
 {
     if (mode == 0)
         return launch_a_moe(mb, x, x_f32, rows, placements, max_active, max_count, H, I, flags, stream, direct,
-                            bank, routes, job, job_done);
-    if (!x_quantised)
+                            bank, routes, x_prepared, job, job_done);
+    if (!x_prepared)
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
     // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces
     const uint32_t piece_rows = moe_piece_rows(1, x_f32, rows);
@@ -1428,7 +1471,7 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
 void launch_moe_layer(uint32_t mode, const ExpertPtrs *bank, const MoeBuffers &mb, const void *x,
                       bool x_f32, uint32_t rows, uint32_t max_active, uint32_t max_count, uint32_t H,
                       uint32_t I, float *out_f32, uint16_t *out_bf16, bool raw, uint32_t *flags,
-                      hipStream_t stream, const OneTokenRoutes *routes, bool x_quantised, const RouteJob *job)
+                      hipStream_t stream, const OneTokenRoutes *routes, bool x_prepared, const RouteJob *job)
 {
     const DirectOut direct{out_f32, out_bf16, raw};
     // the route weights (job) must be in place before a kernel reads them: the mode A experts carry
@@ -1437,7 +1480,7 @@ void launch_moe_layer(uint32_t mode, const ExpertPtrs *bank, const MoeBuffers &m
     bool job_done = false;
     const ExpertOut eo = launch_experts(mode, bank, mb, x, x_f32, rows, rows * 8, routes ? 8 : max_active,
                                         routes ? 1 : max_count, H, I, flags, stream, rows == 1 ? &direct : nullptr,
-                                        routes, x_quantised, job, &job_done);
+                                        routes, x_prepared, job, &job_done);
     if (job && !job_done)  // no expert launch carried the route weights
         launch_route_weights(*job, stream);
     if (!eo.y)

@@ -770,13 +770,13 @@ static void launch_prefill_projection(const PrefillArgs &a, uint32_t nsub, hipSt
 
 void launch_moe_prefill(const ExpertPtrs *bank, const MoeBuffers &mb, const PrefillBuffers &pb, const void *x,
                         bool x_f32, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, float *out_f32,
-                        uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream, bool scheduled_long)
+                        uint16_t *out_bf16, bool raw, uint32_t *flags, hipStream_t stream, bool scheduled)
 {
     (void)bank;
     const uint32_t P = rows * 8;
     const uint32_t max_active = E < P ? E : P;
     const uint32_t max_tiles = prefill_max_tiles(rows, E);
-    if (!scheduled_long) {
+    if (!scheduled) {
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
         hipLaunchKernelGGL(prefill_tiles_kernel, dim3(1), dim3(1024), 0, stream, mb.plan, mb.active,
                            mb.active_expert, max_active, pb.tiles, max_tiles, pb.n_tiles, flags);

@@ -1252,12 +1252,14 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
     PW_TRY(call.upload());
     PW_TRY(ensure_moe(rt, rows, n_experts, H, I));
     PW_HIP(rt->out.ensure(HostCall::padded(n_in * 4)));
-    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
+    const bool prepare = mode == PW_MODE_B || x_f32;
+    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs,
+                          mode == PW_MODE_A ? rt->mb.x_planes : nullptr};
     bool quantised = false;
     pw::launch_moe_schedule((const ExpertPtrs *)d_table, (const uint32_t *)d_ids, (const float *)d_ws, rows, n_experts,
                             std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, rows),
                             rt->d_flags, rt->stream, nullptr,
-                            mode == PW_MODE_B ? &qj : nullptr, mode == PW_MODE_B ? &quantised : nullptr);
+                            prepare ? &qj : nullptr, prepare ? &quantised : nullptr);
     pw::launch_moe_layer(mode, (const ExpertPtrs *)d_table, rt->mb, x, x_f32, rows,
                          std::min<uint32_t>(n_experts, rows * 8), max_count, H, I,
                          (float *)rt->out.p, nullptr, false, rt->d_flags, rt->stream, nullptr, quantised);
@@ -1391,12 +1393,13 @@ static void launch_routed_layer(const MoeBuffers &mb, const pw_expert_bank *bank
                              flags, s, &routes);
         return;
     }
-    // mode B: a decode batch's schedule launch also quantises the activations
-    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, mb.xq, mb.xs};
+    // the schedule launch also quantises the activations (mode B) or splits f32 ones (mode A)
+    const bool prepare = mode == PW_MODE_B || x_f32;
+    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, mb.xq, mb.xs, mode == PW_MODE_A ? mb.x_planes : nullptr};
     bool quantised = false;
     pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E, max_active, mb,
                             pw::moe_piece_rows(mode, x_f32, rows), flags, s, nullptr,
-                            mode == PW_MODE_B ? &qj : nullptr, mode == PW_MODE_B ? &quantised : nullptr);
+                            prepare ? &qj : nullptr, prepare ? &quantised : nullptr);
     pw::launch_moe_layer(mode, bank->table, mb, x, x_f32, rows, max_active, rows, H, I, out_f32, out_bf16, raw, flags,
                          s, nullptr, quantised);
 }
@@ -1459,12 +1462,14 @@ int pw_moe_layer_routed_device(pw_runtime *rt, const pw_expert_bank *bank, uint3
     pw::timer_end(t, s);
     const bool direct = mode == PW_MODE_A && rows == 1 && pw::moe_a_one_token_direct(H, I);
     PW_HIP(rt->set_ids.ensure((size_t)rows * 8 * 4));
-    // mode B: the schedule launch also quantises the activations
-    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
+    // the schedule launch also quantises the activations (mode B) or splits f32 ones (mode A)
+    const bool prepare = mode == PW_MODE_B || x_f32;
+    const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs,
+                          mode == PW_MODE_A ? rt->mb.x_planes : nullptr};
     if (!direct && pw::launch_route_set_schedule(scores, bias, bank->table, rows, E, max_active,
                                                  (uint32_t *)rt->set_ids.p, rt->mb,
                                                  pw::moe_piece_rows(mode, x_f32, rows), rt->d_flags, s,
-                                                 mode == PW_MODE_B ? &qj : nullptr)) {
+                                                 prepare ? &qj : nullptr)) {
         // the expert sets are scheduled; the routes' order and weights (a serial partition per row)
         // run in extra workgroups of an expert launch (mode A: the down, mode B: the gate/up) while
         // its others stream the experts' weights (or in a launch of their own before the combine)
@@ -1483,7 +1488,7 @@ int pw_moe_layer_routed_device(pw_runtime *rt, const pw_expert_bank *bank, uint3
         pw::launch_moe_layer(mode, bank->table, rt->mb, x, x_f32, rows, max_active, rows, H, I,
                              out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
                              out_dtype == PW_DTYPE_BF16 ? (uint16_t *)output : nullptr, out_dtype == PW_DTYPE_F32_RAW,
-                             rt->d_flags, s, nullptr, mode == PW_MODE_B, &job);
+                             rt->d_flags, s, nullptr, prepare, &job);
     } else if (direct && E <= 256) {
         // one token: the expert set is the direct layer's routes; the routes' order and weights
         // (the partition) run in extra workgroups of its gate/up launch and give the weights in the
@@ -1589,13 +1594,13 @@ int pw_moe_prefill_device(pw_runtime *rt, const pw_expert_bank *bank, const void
     pb.silu = (const uint16_t *)rt->pf_silu.p;
     const uint32_t P = rows * 8;
     const pw::PfTileTable tt{pb.tiles, pb.n_tiles, max_tiles};
-    const pw::QuantJob qj{x, x_dtype == PW_DTYPE_F32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs};
-    const bool scheduled_long = pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E,
+    const pw::QuantJob qj{x, x_dtype == PW_DTYPE_F32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs, nullptr};
+    const bool scheduled = pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E,
                                                         std::min<uint32_t>(E, P), rt->mb, 0, rt->d_flags, s, &tt, &qj);
     pw::launch_moe_prefill(bank->table, rt->mb, pb, x, x_dtype == PW_DTYPE_F32, rows, E, H, I,
                            out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
                            out_dtype == PW_DTYPE_BF16 ? (uint16_t *)output : nullptr,
-                           out_dtype == PW_DTYPE_F32_RAW, rt->d_flags, s, scheduled_long);
+                           out_dtype == PW_DTYPE_F32_RAW, rt->d_flags, s, scheduled);
     PW_HIP(hipGetLastError());
     return PW_OK;
 }
