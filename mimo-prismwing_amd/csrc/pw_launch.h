@@ -132,7 +132,6 @@ struct SplitPlan {
 SplitPlan plan_split(uint32_t K, int mats, int ns, uint32_t max_cnt);
 void launch_moe_a_split(int mats, int ns, const SplitArgs &args, const SplitPlan &sp, uint32_t max_active,
                         hipStream_t stream);
-// gate/up split sums -> SwiGLU -> hidden as three bf16 planes [3][P][I]
 // BF16 wide linear (pw_bf16.hip): w bf16 [R][K] (K a multiple of 128), x bf16 or f32 [W][K]; partial:
 // bf16_shares(K, R) x W x R floats when that is above one.
 uint32_t bf16_shares(uint32_t K, uint32_t R);
@@ -158,6 +157,7 @@ bool launch_moe_a_down_combine1(const SplitArgs &args, const MoePlan *plan, cons
 bool moe_a_one_token_direct(uint32_t H, uint32_t I);
 bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_active, uint16_t *hidden_planes,
                                hipStream_t stream);
+// gate/up split sums -> SwiGLU -> hidden as three bf16 planes [3][P][I]
 void launch_moe_a_swiglu(const float *partial, uint32_t ks, uint32_t P, uint32_t I, uint16_t *hidden_planes,
                          uint32_t *flags, hipStream_t stream);
 

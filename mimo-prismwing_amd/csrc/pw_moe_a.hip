@@ -188,10 +188,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void m
 // are added in split order 0..7 -- the same order and the same arithmetic as the split kernel
 // followed by moe_a_swiglu_kernel, so the hidden planes are bit-identical -- and the SwiGLU is
 // written as three exact bf16 planes. No split partials go through memory.
-// RM = 8 (one-row experts): a work item is 8 rows of gate and the same 8 rows of up, stacked
-// into one 16-row MFMA operand (lanes 0..7 of a row group read gate rows, 8..15 up rows), so a lone
-// expert spreads over twice the workgroups; output rows 0..7 are gate, 8..15 up, and each gate
-// lane takes its up values from the lane 32 above. The sums are the same as with RM = 16.
+// RM = 8 (one-row experts): a work item is 8 rows of gate and the same 8 rows of up, stacked into one
+// 16-row MFMA operand (lanes 0..7 of a row group read gate rows, 8..15 up rows), which doubles the
+// workgroups; output rows 0..7 are gate, 8..15 up, and each gate lane takes its up values from the
+// lane 32 above. The sums are the same as with RM = 16.
+
 // Route a of a one-token batch as a schedule entry: expert route_ids[a] (ids past the bank take its
 // last expert; the down+combine flags them), placement slot a, token row 0.
 __device__ __forceinline__ ActiveExpert route_entry(const SplitArgs &args, uint32_t a)

@@ -1,4 +1,4 @@
-// Mode B routed-expert projections for the decode MoE layer and the one-expert forward: dynamic
+// Mode B gate/up of routed experts for the decode MoE layer: dynamic
 // per-(row, 128-column) e4m3 activations against the block-FP8 weights on the FP8 MFMA, one
 // 128-column block per instruction, total += dot * weight_scale * activation_scale per block
 // (src/wide_metal_moe.rs:404-421, :1080-1166; Metal block_fp8_gemm{count}_sglang_blockscaled
