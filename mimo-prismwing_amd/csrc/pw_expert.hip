@@ -11,8 +11,11 @@ namespace pw {
 // rows: f32 hidden, width 8 49.1 / 48.5 / 51.0, width 16 53.8 / 51.2 / 52.0, width 32
 // 71.5 / 62.2 / 64.5; codes, width 16 52.4 / 53.1 / 56.0, width 32 61.4 / 58.8 / 60.5; K = 2048 one
 // share is best at every width, 16.6 / 17.3 / 18.1 at width 32).
+// Up to 128 tiles follow the projections' rule, so the forward stays the same as its separate calls.
 static uint32_t down_shares(bool codes, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
+    if (n_tiles <= 128)
+        return linear_shares(codes ? WX_CODES : WX_F32, W, K, n_tiles);
     return n_tiles <= 256 && (uint64_t)K * W >= (codes ? 20u : 12u) * 16384u ? 2u : 1u;
 }
 
@@ -63,7 +66,7 @@ uint32_t launch_expert_down(const ExpertPtrs &ep, bool codes, const void *x, con
     args.y_bf16 = out_bf16;
     args.round_f32 = raw ? 0u : 1u;
     args.KS = down_shares(codes, W, I, args.n_tiles);
-    const int rt = args.KS > 1 ? 2 : pick_rt(codes ? WX_CODES : WX_F32, W, args.n_tiles);
+    const int rt = args.KS > 1 && args.n_tiles > 128 ? 2 : pick_rt(codes ? WX_CODES : WX_F32, W, args.n_tiles);
     const int t = timer_begin(K_MOE_DOWN, stream);
     if (codes)
         launch_wide<WK_DOWN, WX_CODES>(args, rt, stream);

@@ -60,12 +60,27 @@ void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream
     hipLaunchKernelGGL(split_planes_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, x, n, planes);
 }
 
+// Shares of K. Few tiles of a long K leave most of the chip idle while each workgroup takes in the
+// batch's rows over the whole K: up to 64 tiles take four shares, up to 128 two, for a second launch
+// that adds them, where the rows are enough to pay for it (us, one / two / four shares: 1000 x 8192,
+// mode A, one f32 row 10.1 / 9.1 / 8.4, 32 f32 rows 19.0 / 14.5 / 11.6, 16 bf16 rows 9.8 / 8.8 / 8.7,
+// one bf16 row 8.2 / 8.6 / 8.5; mode B, 32 rows 16.0 / 12.8 / 11.4; 2000 x 6144, 32 bf16 rows
+// 10.1 / 9.4 / 11.9, 8 f32 rows 9.8 / 9.1 / 9.7; 600 x 5120, one f32 row 7.9 / 8.4 / 8.3, 16 f32 rows
+// 9.8 / 9.6 / 8.7; 3000 x 8192, 16 f32 rows 14.8 / 19.3 / 18.6).
+uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles)
+{
+    const bool pays = xt == WX_F32 ? K >= 6144 || (K >= 5120 && W > 8) : (K >= 8192 && W > 8) || (K >= 6144 && W > 16);
+    return !pays || n_tiles > 128 ? 1u : n_tiles > 64 ? 2u : 4u;
+}
+
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
-                   uint32_t K, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
+                   uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
 {
     WideArgs args{};
     args.tiles = tiles;
     args.n_tiles = n_tiles;
+    args.partial = partial;
+    args.KS = linear_shares(xt, W, K, n_tiles);
     args.x = x;
     args.x_scales = x_scales;
     args.W = W;
@@ -82,6 +97,8 @@ void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void
         launch_wide<WK_PROJ, WX_BF16>(args, rt, stream);
     else
         launch_wide<WK_PROJ, WX_CODES>(args, rt, stream);
+    if (args.KS > 1)
+        launch_round_output(partial, args.KS, W * N, y32, y16, !round_f32, nullptr, stream);
     timer_end(t, stream);
 }
 

@@ -143,7 +143,7 @@ struct pw_runtime {
     // routed-MoE per-layer scratch
     DevBuf moe_plan, moe_active_expert, moe_active_offset, moe_pos, moe_w, moe_slots, moe_hidden,
         moe_hidden_planes, moe_x_planes, moe_y, moe_xq, moe_xs, moe_hq, moe_hs, lin_planes,
-        moe_active, moe_pieces, moe_partial, moe_sched, pf_tiles, pf_silu, router_scores, bf16_partial;
+        moe_active, moe_pieces, moe_partial, moe_sched, pf_tiles, pf_silu, router_scores, share_sums;
     MoeBuffers mb{};
     pw::KernelTimer timer;
     bool silu_ready = false;  // pf_silu holds the complete silu table
@@ -909,6 +909,11 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
                           const pw_projection *p, float *y32, uint16_t *y16, uint32_t round_f32,
                           hipStream_t stream)
 {
+    const pw::WideX xt = mode == PW_MODE_B ? pw::WX_CODES : x_f32 ? pw::WX_F32 : pw::WX_BF16;
+    const uint32_t ks = pw::linear_shares(xt, rows, p->columns, p->n_tiles);
+    if (ks > 1)
+        PW_HIP(rt->share_sums.ensure((size_t)ks * rows * p->rows * 4));
+    float *partial = (float *)rt->share_sums.p;
     if (mode == PW_MODE_A) {
         if ((uintptr_t)x & 15) {
             // rows off 16 bytes (a caller's slice): the projection's copies take an aligned one
@@ -917,15 +922,15 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
             PW_HIP(hipMemcpyAsync(rt->lin_planes.p, x, bytes, hipMemcpyDeviceToDevice, stream));
             x = rt->lin_planes.p;
         }
-        pw::launch_linear(x_f32 ? pw::WX_F32 : pw::WX_BF16, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, y32,
-                          y16, p->rows, round_f32, stream);
+        pw::launch_linear(xt, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, partial, y32, y16, p->rows, round_f32,
+                          stream);
     } else if (mode == PW_MODE_B) {
         PW_HIP(rt->codes.ensure((size_t)rows * p->columns));
         PW_HIP(rt->scales.ensure((size_t)rows * (p->columns / 128) * 4));
         pw::launch_quant_group128(x, x_f32, rows, p->columns, (uint8_t *)rt->codes.p,
                                   (float *)rt->scales.p, rt->d_flags, stream);
-        pw::launch_linear(pw::WX_CODES, p->tiles, p->n_tiles, rt->codes.p, (const float *)rt->scales.p, rows,
-                          p->columns, y32, y16, p->rows, round_f32, stream);
+        pw::launch_linear(xt, p->tiles, p->n_tiles, rt->codes.p, (const float *)rt->scales.p, rows, p->columns, partial,
+                          y32, y16, p->rows, round_f32, stream);
     } else {
         return fail(PW_ERR_ARGUMENT, "unknown mode %u", mode);
     }
@@ -1058,8 +1063,8 @@ static int enqueue_bf16_linear(pw_runtime *rt, const void *x, bool x_f32, uint32
 {
     const uint32_t ks = pw::bf16_shares(p->columns, p->rows);
     if (ks > 1)
-        PW_HIP(rt->bf16_partial.ensure((size_t)ks * rows * p->rows * 4));
-    pw::launch_bf16_linear((const uint16_t *)p->w, x, x_f32, rows, p->columns, p->rows, (float *)rt->bf16_partial.p, y32,
+        PW_HIP(rt->share_sums.ensure((size_t)ks * rows * p->rows * 4));
+    pw::launch_bf16_linear((const uint16_t *)p->w, x, x_f32, rows, p->columns, p->rows, (float *)rt->share_sums.p, y32,
                            y16, round_f32, rt->d_flags, stream);
     PW_HIP(hipGetLastError());
     return PW_OK;

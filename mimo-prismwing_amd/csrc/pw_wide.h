@@ -40,12 +40,13 @@ struct WideStep {
 };
 
 // What a workgroup's 16-row tiles are, and what becomes of their sums:
-//   WK_PROJ    tiles of a projection's table; its output rows.
+//   WK_PROJ    tiles of a projection's table, K in KS shares of consecutive workgroups; one share: its
+//              output rows, rounded or not; more: share sums [KS][W][N].
 //   WK_GATEUP  eight gate rows and the same eight up rows of one expert stacked into one tile (output
 //              rows 0..7 gate, 8..15 up: lane l takes its gate rows' up values from lane l + 32);
 //              SwiGLU -> hidden rows [W][N] f32 (mode B: bf16-staged).
-//   WK_DOWN    rows of one expert's down matrix, K in KS shares of consecutive workgroups; one share:
-//              the output rows rounded, flagged if not finite; more: share sums [KS][W][N].
+//   WK_DOWN    rows of one expert's down matrix, K in KS shares as above; one share: the output rows
+//              rounded, flagged if not finite.
 //   WK_BF16    rows of a bf16 weight [N][K] (mode A activations, no scales), K in KS shares as above;
 //              the output rows, rounded or not, flagged if not finite.
 enum WideKind : int { WK_PROJ = 0, WK_GATEUP = 1, WK_DOWN = 2, WK_BF16 = 3 };
@@ -55,7 +56,7 @@ struct WideArgs {
     const uint8_t *w0, *w1;        // gate and up, down [N][K], or the bf16 weight's bytes
     const float *s0, *s1;          // ... and their block scales
     float *partial;                // with KS > 1: share sums [KS][W][N]
-    uint32_t KS;                   // WK_DOWN, WK_BF16
+    uint32_t KS;                   // all but WK_GATEUP
     uint32_t *flags;
     uint32_t n_tiles;
     const void *x;         // activations [W][K]: bf16, f32 or e4m3 codes
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
     uint4 *slots = lds_w + (size_t)wave * 2 * S::SLOT;
 
     constexpr int WQ = XT == WX_CODES || KIND == WK_BF16 ? 32 : 16;  // weight bytes of a lane's q in a row
-    constexpr bool SHARES = KIND == WK_DOWN || KIND == WK_BF16;
+    constexpr bool SHARES = KIND != WK_GATEUP;
     const uint32_t group = SHARES ? blockIdx.x / args.KS : blockIdx.x;
     const uint8_t *wrow[RT];
     const float *ws[RT];
@@ -409,6 +410,10 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
             if (row >= tile.valid)
                 continue;
             const size_t at = (size_t)token * args.N + tile.out_row + row;
+            if (args.KS > 1) {
+                args.partial[(size_t)(blockIdx.x % args.KS) * W * args.N + at] = sum[i];
+                continue;
+            }
             if (args.y_f32)
                 args.y_f32[at] = args.round_f32 ? round_bf16(sum[i]) : sum[i];
             if (args.y_bf16)
@@ -508,7 +513,7 @@ static inline int pick_rt(int xt, uint32_t W, uint32_t n_tiles)
 template <int KIND, int XT, int XR>
 static void launch_wide_rt(const WideArgs &args, int rt, hipStream_t stream)
 {
-    const dim3 grid((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND == WK_DOWN || KIND == WK_BF16 ? args.KS : 1u)), block(512);
+    const dim3 grid((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND != WK_GATEUP ? args.KS : 1u)), block(512);
     if (rt == 4)
         hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 4>), grid, block, 0, stream, args);
     else if (rt == 2)

@@ -118,12 +118,13 @@ def test_mode_a_f32_row_split_in_staging(rt, n, k):
     assert normwise(one, O.gemm_mode_a(w, s, x)) <= (2e-6 if k <= 512 else 1e-5)
 
 
-@pytest.mark.parametrize("n", [24, 4104, 8200, 12296])
-@pytest.mark.parametrize("k", [128, 1152, 3328])
+@pytest.mark.parametrize("n,k", [(n, k) for n in (24, 4104, 8200, 12296) for k in (128, 1152, 3328)] +
+                         [(1000, 8192), (2000, 6144)])
 def test_projection_tile_and_step_edges(rt, n, k):
     """Every staged-row count (4, 8, 16, 24, 32 rows and one off each), workgroups of one, two and
     four 16-row tiles with a partial last tile and a partial last workgroup, and waves with no, one,
-    two, three and four steps (1, 9 and 26 blocks over eight waves). Mode A against 64 bits: exact
+    two, three and four steps (1, 9 and 26 blocks over eight waves), and K in four and two shares (the last
+    two shapes, by the rows' type and number). Mode A against 64 bits: exact
     products added in f32 in chains of at most 48 roundings (2e-6). Mode B on integers whose sums are
     exact in f32 (weights up to 2, codes up to 8 with one 448 a group, so activation scales are 1,
     block scales powers of two): equal."""
