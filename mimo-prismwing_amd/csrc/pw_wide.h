@@ -336,14 +336,22 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
                     }
                 }
             }
-            if constexpr (KIND != WK_BF16 && (SC == 128 || s == 1)) {  // a block is complete
+            // A block is complete. Blocks are added to the total also where no scale asks for it: a
+            // wave's whole share of K in one accumulator is a chain of 1024 columns at K = 8192, whose
+            // error against 64 bits is 3.6e-7 (f32 rows) and 1.9e-7 (bf16 rows) where block sums have
+            // 1.6e-7 and 1.0e-7, at the same speed.
+            if constexpr (SC == 128 || s == 1) {
 #pragma unroll
                 for (int r = 0; r < RT; ++r)
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            total[r][nt][i] = __builtin_fmaf(sw[s][r], acc[r][nt][i], total[r][nt][i]);
+                        for (int i = 0; i < 4; ++i) {
+                            if constexpr (KIND == WK_BF16)
+                                total[r][nt][i] += acc[r][nt][i];
+                            else
+                                total[r][nt][i] = __builtin_fmaf(sw[s][r], acc[r][nt][i], total[r][nt][i]);
+                        }
                         acc[r][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
                     }
             }
@@ -385,7 +393,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
-            red[(wave * RT * NT + r * NT + nt) * 64 + lane] = KIND == WK_BF16 ? acc[r][nt] : total[r][nt];
+            red[(wave * RT * NT + r * NT + nt) * 64 + lane] = total[r][nt];
     __syncthreads();
     if (wave >= RT * NT)
         return;

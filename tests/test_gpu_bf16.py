@@ -172,3 +172,23 @@ def test_tile_step_and_share_edges(rt, n, k):
             assert rel_l2(_device(torch, rt, proj, x[:rows], rows, P.DTYPE_F32_RAW, bf), ref[:rows]) <= RAW_TOL, (rows, bf)
         raw = _device(torch, rt, proj, xb[:rows], rows, P.DTYPE_F32_RAW, True)
         assert np.array_equal(_device(torch, rt, proj, xb[:rows], rows, P.DTYPE_BF16, True), WL.bf16_round_np(raw)), rows
+
+
+@pytest.mark.parametrize("n", [2064, 24])
+def test_sums_are_folded_every_block(rt, n):
+    """Sums go into the total a 128-column block at a time, so no f32 chain is longer than a block
+    whatever K is. The first block is one 2^24, every other block sums to 2 in steps of 2^-6: added
+    by blocks every partial sum is exact (even integers up to 2^24 + 126, halves of them ...), in a
+    longer chain the steps are lost against 2^24. One K share of 8192 columns (2064 rows) and four."""
+    import torch
+    k = 8192
+    wv = np.full((n, k), 2.0 ** -6, np.float32)
+    wv[:, :128] = 0.0
+    wv[:, 0] = 2.0 ** 24
+    proj = rt.bind_bf16((wv.view(np.uint32) >> 16).astype(np.uint16))
+    for rows in (1, 8, 32):
+        scale = np.ldexp(np.float32(1), -(np.arange(rows) % 4)).astype(np.float32)
+        x = np.repeat(scale[:, None], k, axis=1)
+        for bf in (False, True):
+            got = _device(torch, rt, proj, x, rows, P.DTYPE_F32_RAW, bf)
+            assert np.array_equal(got, np.repeat((scale * np.float32(2 ** 24 + 126))[:, None], n, axis=1)), (rows, bf)
