@@ -21,11 +21,7 @@ namespace pw {
 // 12.8 / 10.2 / 8.5 / 8.6; 2048 x 8192, 8 f32 rows 14.0 / 11.1 / 12.1 / 14.9; 3000 x 8192, one
 // bf16 row 12.2 / 14.7; 1000 x 5120, 16 f32 rows 11.0 / 10.1 / 9.0; 1000 x 4096, one f32 row 7.9 with
 // one share).
-uint32_t bf16_shares(uint32_t K, uint32_t R)
-{
-    const uint32_t n_tiles = (R + 15) / 16;
-    return K < 5120 || n_tiles > 128 ? 1u : n_tiles > 64 ? 2u : 4u;
-}
+static uint32_t bf16_shares(uint32_t K, uint32_t n_tiles) { return K < 5120 ? 1u : tile_shares(n_tiles); }
 
 // Tiles per workgroup (pw_wide.h's pick_rt for one-byte weights): twice the weight bytes per tile keep
 // one tile ahead while the activations are up to 16 bytes a column (32 from 513 to 1024 tiles) (us, one /
@@ -46,7 +42,7 @@ void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W
     args.flags = flags;
     args.n_tiles = (R + 15) / 16;
     args.partial = partial;
-    args.KS = bf16_shares(K, R);
+    args.KS = bf16_shares(K, args.n_tiles);
     args.x = x;
     args.W = W;
     args.K = K;

@@ -132,9 +132,13 @@ struct SplitPlan {
 SplitPlan plan_split(uint32_t K, int mats, int ns, uint32_t max_cnt);
 void launch_moe_a_split(int mats, int ns, const SplitArgs &args, const SplitPlan &sp, uint32_t max_active,
                         hipStream_t stream);
+// K shares of a projection of n_tiles 16-row tiles whose rule asks for them, and the room their sums
+// take at most: 256 tiles in all of 16 rows for 32 activation rows. A runtime holds it from its
+// creation, so a call never allocates for its shares and a captured call's sums stay where they are.
+static inline uint32_t tile_shares(uint32_t n_tiles) { return n_tiles > 128 ? 1u : n_tiles > 64 ? 2u : 4u; }
+constexpr size_t SHARE_SUM_BYTES = (size_t)256 * 16 * 32 * sizeof(float);
 // BF16 wide linear (pw_bf16.hip): w bf16 [R][K] (K a multiple of 128), x bf16 or f32 [W][K]; partial:
-// bf16_shares(K, R) x W x R floats when that is above one.
-uint32_t bf16_shares(uint32_t K, uint32_t R);
+// SHARE_SUM_BYTES.
 void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W, uint32_t K, uint32_t R, float *partial,
                         float *y32, uint16_t *y16, uint32_t round_f32, uint32_t *flags, hipStream_t stream);
 // ks share sums of n outputs added in share order: f32 rounded to bf16 or raw, bf16 bits; a non-finite
@@ -192,8 +196,7 @@ inline void timer_end(int slot, hipStream_t s)
 // f32 [n] -> three bf16 planes [3][n]
 void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream_t stream);
 // Block-FP8 projection (pw_linear.hip): x [W][K] 16-byte aligned, bf16 or f32 (mode A) or e4m3 codes
-// with x_scales [W][K / 128] (mode B); partial: linear_shares(...) x W x N floats when that is above
-// one.
+// with x_scales [W][K / 128] (mode B); partial: SHARE_SUM_BYTES.
 enum WideX : int { WX_BF16 = 0, WX_F32 = 1, WX_CODES = 2 };
 uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles);
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,

@@ -70,7 +70,7 @@ void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream
 uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
     const bool pays = xt == WX_F32 ? K >= 6144 || (K >= 5120 && W > 8) : (K >= 8192 && W > 8) || (K >= 6144 && W > 16);
-    return !pays || n_tiles > 128 ? 1u : n_tiles > 64 ? 2u : 4u;
+    return pays ? tile_shares(n_tiles) : 1u;
 }
 
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,

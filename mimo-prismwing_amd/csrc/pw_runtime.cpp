@@ -592,6 +592,8 @@ int pw_runtime_create(int device, uint32_t flags, pw_runtime **out)
         e = hipMalloc((void **)&rt->d_flags, sizeof(uint32_t));
     if (e == hipSuccess)
         e = hipMemset(rt->d_flags, 0, sizeof(uint32_t));
+    if (e == hipSuccess)
+        e = rt->share_sums.ensure(pw::SHARE_SUM_BYTES);
     if (e != hipSuccess) {
         pw_runtime_destroy(rt);
         return fail(PW_ERR_DEVICE, "runtime setup failed: %s", hipGetErrorString(e));
@@ -910,9 +912,6 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
                           hipStream_t stream)
 {
     const pw::WideX xt = mode == PW_MODE_B ? pw::WX_CODES : x_f32 ? pw::WX_F32 : pw::WX_BF16;
-    const uint32_t ks = pw::linear_shares(xt, rows, p->columns, p->n_tiles);
-    if (ks > 1)
-        PW_HIP(rt->share_sums.ensure((size_t)ks * rows * p->rows * 4));
     float *partial = (float *)rt->share_sums.p;
     if (mode == PW_MODE_A) {
         if ((uintptr_t)x & 15) {
@@ -1061,9 +1060,6 @@ int pw_bf16_bind_device(pw_runtime *rt, const void *weight, uint32_t rows, uint3
 static int enqueue_bf16_linear(pw_runtime *rt, const void *x, bool x_f32, uint32_t rows, const pw_projection *p,
                                float *y32, uint16_t *y16, uint32_t round_f32, hipStream_t stream)
 {
-    const uint32_t ks = pw::bf16_shares(p->columns, p->rows);
-    if (ks > 1)
-        PW_HIP(rt->share_sums.ensure((size_t)ks * rows * p->rows * 4));
     pw::launch_bf16_linear((const uint16_t *)p->w, x, x_f32, rows, p->columns, p->rows, (float *)rt->share_sums.p, y32,
                            y16, round_f32, rt->d_flags, stream);
     PW_HIP(hipGetLastError());

@@ -148,6 +148,53 @@ def test_projection_tile_and_step_edges(rt, n, k):
         assert np.array_equal(run_device(rt, proj_i, xi[:rows], mode=P.MODE_B, x_dtype=P.DTYPE_F32), ref_i[:rows]), rows
 
 
+@pytest.mark.parametrize("weights", ["fp8", "bf16"])
+def test_mode_a_first_call_under_graph_capture(rt, weights):
+    """Mode A and BF16 projections allocate nothing in a call, also where K runs in shares whose sums
+    a second launch adds: a runtime's first call is one under capture, and every replay gives the
+    eager call's bits, with larger eager calls (more rows, more shares' sums) between replays."""
+    torch = _torch()
+    rng = np.random.default_rng(91)
+    n, k, rows = 1000, 8192, 16
+    cap = P.WideMoeRuntime.compile(0)
+
+    def bind(r, n):
+        if weights == "bf16":
+            w = rng.integers(0x3C00, 0x3D00, (n, k)).astype(np.uint16)
+            p = r.bind_bf16(w)
+            call = r.bf16_linear_device
+        else:
+            s = log_uniform_scales(rng, n, k)
+            p = r.bind_projection(fp8_weight(rng, n, k, s), s)
+            call = lambda *a, **kw: r.fp8_linear_device(*a, mode=P.MODE_A, **kw)
+        return lambda x, out, stream: call(p, x, x.shape[0], out, x_dtype=P.DTYPE_BF16, out_dtype=P.DTYPE_F32_RAW,
+                                           stream=stream.cuda_stream)
+
+    state = rng.bit_generator.state
+    eager = bind(rt, n)
+    rng.bit_generator.state = state
+    captured, larger = bind(cap, n), bind(cap, 2000)
+    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).cuda().bfloat16()
+    x32 = torch.from_numpy(rng.standard_normal((32, k)).astype(np.float32)).cuda().bfloat16()
+    want, got = (torch.empty((rows, n), dtype=torch.float32, device="cuda") for _ in range(2))
+    more = torch.empty((32, 2000), dtype=torch.float32, device="cuda")
+    s_cap, s_other = torch.cuda.Stream(), torch.cuda.Stream()
+    eager(x, want, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s_cap, capture_error_mode="thread_local"):
+        captured(x, got, s_cap)
+    for replay in range(3):
+        got.fill_(7)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), f"replay {replay}"
+        larger(x32, more, s_other)
+        torch.cuda.synchronize()
+    assert cap.take_flags() == 0
+
+
 @pytest.mark.parametrize("kind", ["f32", "bf16"])
 def test_mode_a_rows_off_16_bytes(rt, kind):
     """Activation rows that start off 16 bytes give the bits of aligned ones."""
