@@ -36,7 +36,7 @@ void launch_expert_gateup(const ExpertPtrs &ep, bool codes, bool x_f32, const vo
     args.N = I;
     args.y_f32 = hidden;
     const int xt = codes ? WX_CODES : x_f32 ? WX_F32 : WX_BF16;
-    const int rt = pick_rt(xt, W, args.n_tiles);
+    const int rt = pick_rt(xt, W, H, args.n_tiles);
     const int t = timer_begin(K_MOE_GATEUP, stream);
     if (codes)
         launch_wide<WK_GATEUP, WX_CODES>(args, rt, stream);
@@ -66,7 +66,7 @@ uint32_t launch_expert_down(const ExpertPtrs &ep, bool codes, const void *x, con
     args.y_bf16 = out_bf16;
     args.round_f32 = raw ? 0u : 1u;
     args.KS = down_shares(codes, W, I, args.n_tiles);
-    const int rt = args.KS > 1 && args.n_tiles > 128 ? 2 : pick_rt(codes ? WX_CODES : WX_F32, W, args.n_tiles);
+    const int rt = args.KS > 1 && args.n_tiles > 128 ? 2 : pick_rt(codes ? WX_CODES : WX_F32, W, I, args.n_tiles);
     const int t = timer_begin(K_MOE_DOWN, stream);
     if (codes)
         launch_wide<WK_DOWN, WX_CODES>(args, rt, stream);

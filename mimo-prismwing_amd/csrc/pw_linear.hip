@@ -89,7 +89,7 @@ void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void
     args.y_f32 = y32;
     args.y_bf16 = y16;
     args.round_f32 = round_f32;
-    const int rt = pick_rt(xt, W, n_tiles);
+    const int rt = pick_rt(xt, W, K, n_tiles);
     const int t = timer_begin(xt == WX_CODES ? K_LINEAR_B : K_LINEAR_A, stream);
     if (xt == WX_F32)
         launch_wide<WK_PROJ, WX_F32>(args, rt, stream);

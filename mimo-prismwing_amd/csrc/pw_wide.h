@@ -508,9 +508,20 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
 // of up to 32 activation bytes a column two (us of a whole 4096 x 16384 expert, 2048 gate/up tiles:
 // bf16 width 1 40.9 / 44.2 / 47.8, width 16 52.2 / 50.2 / 53.7, width 32 86.2 / 76.4 / 70.8; codes
 // width 24 66.2 / 58.4 / 59.1).
-static inline int pick_rt(int xt, uint32_t W, uint32_t n_tiles)
+// Up to 2048 columns a wave has one or two steps, all in flight at once, so more tiles a workgroup
+// give it nothing to overlap: smaller workgroups keep ahead for longer (us, one / two / four tiles:
+// bf16 width 1, 848 tiles of 1024 columns 6.0 / 6.0 / 6.8, of 2048 8.7 / 8.8 / 9.2; width 8, 1024
+// tiles of 1024 columns 6.8 / 6.4 / 6.8; f32 width 1, 532 tiles of 1024 columns 6.9 / 6.5 / 7.1, of
+// 2048 9.4 / 9.1 / 9.7).
+static inline int pick_rt(int xt, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
     const bool light = xt != WX_F32 && W <= 4, medium = xt != WX_F32 && W <= 8;
+    if (K <= 2048 && n_tiles > 512 && n_tiles <= 1024) {
+        if (light || (medium && n_tiles <= 768))
+            return 1;
+        if (medium || (xt == WX_F32 && W <= 4 && n_tiles <= 768))
+            return 2;
+    }
     if (n_tiles > 1024)
         return medium ? 1 : W * (xt == WX_F32 ? 4 : xt == WX_BF16 ? 2 : 1) <= 32 ? 2 : 4;
     if (n_tiles <= 256 || (light && n_tiles <= 512) || (medium && n_tiles > 512 && n_tiles <= 768))
