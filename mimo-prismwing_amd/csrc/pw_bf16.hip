@@ -23,15 +23,29 @@ namespace pw {
 // one share).
 static uint32_t bf16_shares(uint32_t K, uint32_t n_tiles) { return K < 5120 ? 1u : tile_shares(n_tiles); }
 
-// Tiles per workgroup (pw_wide.h's pick_rt for one-byte weights): twice the weight bytes per tile keep
-// one tile ahead while the activations are up to 16 bytes a column (32 from 513 to 1024 tiles) (us, one /
-// two / four tiles: 6000 x 8192, 8 bf16 rows 21.4 / 23.7 / 33.5, 8 f32 rows 24.0 / 22.0 / 35.2;
-// 16384 x 8192, 8 f32 rows 44.4 / 48.6 / 45.2, 32 bf16 rows 62.1 / 53.9 / 46.1).
-static int bf16_rt(bool x_f32, uint32_t W, uint32_t n_tiles)
+// Tiles per workgroup (pw_wide.h's pick_rt for one-byte weights). Twice the weight bytes per tile keep
+// one tile ahead while the activations are up to 16 bytes a column, and up to 32 from 513 to 2304 tiles
+// (us, one / two / three / four tiles, K = 4096: 1063 tiles, 8 f32 rows 27.6 / 39.6 / 33.0 / 41.4; 2063
+// tiles 47.3 / 66.0 / 50.2 / 62.0; 2500 tiles 73.9 / 72.6 / 72.2 / 71.3). Past that a CU holds one
+// workgroup of three or four tiles, so the launch takes whole generations of 768 or 1024 tiles: the one
+// with the shorter sum of them (1063 tiles, 16 f32 rows 40.9 / 43.5 / 34.9 / 42.8; 2063 tiles
+// 71.9 / 74.9 / 53.6 / 64.2; 2500 tiles 100.8 / 80.5 / 77.2 / 76.7; 532 tiles, 32 f32 rows
+// 34.0 / 31.3 / 20.9 / 25.2; 848 tiles 43.6 / 32.1 / 38.2 / 26.8). At K = 1024 a wave has one step
+// and nothing to overlap: many tiles of 16 to 32 staged bytes a column go by two (1536 tiles, one f32 row
+// 14.2 / 11.5 / - / 14.9, 16 bf16 rows 14.4 / 12.3 / 13.4 / 14.8, 4 bf16 rows 11.2 / 11.5 / - / 14.2).
+static int bf16_rt(bool x_f32, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
-    if (n_tiles <= 256 || W * (x_f32 ? 4 : 2) <= (n_tiles > 512 && n_tiles <= 1024 ? 32u : 16u))
+    const uint32_t bytes = W * (x_f32 ? 4 : 2);
+    if (n_tiles <= 256)
         return 1;
-    return n_tiles <= 512 ? 2 : 4;
+    if (K <= 1024 && n_tiles > 768 && bytes <= 32 && (x_f32 || W > 4))
+        return 2;
+    if (bytes <= (n_tiles > 512 && n_tiles <= 2304 ? 32u : 16u))
+        return 1;
+    if (n_tiles <= 512)
+        return 2;
+    const uint32_t three = (n_tiles + 767) / 768, four = (n_tiles + 1023) / 1024;  // generations
+    return 3 * three < 4 * four ? 3 : 4;
 }
 
 void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W, uint32_t K, uint32_t R, float *partial,
@@ -50,7 +64,7 @@ void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W
     args.y_f32 = y32;
     args.y_bf16 = y16;
     args.round_f32 = round_f32;
-    const int rt = bf16_rt(x_f32, W, args.n_tiles);
+    const int rt = bf16_rt(x_f32, W, K, args.n_tiles);
     const int t = timer_begin(K_BF16_LINEAR, stream);
     if (x_f32)
         launch_wide<WK_BF16, WX_F32>(args, rt, stream);

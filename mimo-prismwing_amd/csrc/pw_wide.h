@@ -535,6 +535,8 @@ static void launch_wide_rt(const WideArgs &args, int rt, hipStream_t stream)
     const dim3 grid((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND != WK_GATEUP ? args.KS : 1u)), block(512);
     if (rt == 4)
         hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 4>), grid, block, 0, stream, args);
+    else if (KIND == WK_BF16 && rt == 3)
+        hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, KIND == WK_BF16 ? 3 : 2>), grid, block, 0, stream, args);
     else if (rt == 2)
         hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 2>), grid, block, 0, stream, args);
     else
