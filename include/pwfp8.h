@@ -185,7 +185,7 @@ int pw_fp8_linear(pw_runtime *rt, uint32_t mode, const float *input, uint32_t ro
 /* Device-resident form: input [rows x columns] of input_dtype, output [rows x proj_rows] of
  * output_dtype (f32 output holds bf16-rounded values when round_output != 0), enqueued on stream.
  * Mode B needs the runtime's scratch for the activation codes, which a larger call than any before
- * reallocates; mode A on rows that start on 16 bytes allocates nothing in a call. rows <= 32. */
+ * reallocates; mode A allocates nothing in a call. rows <= 32. */
 int pw_fp8_linear_device(pw_runtime *rt, uint32_t mode, const void *input, uint32_t input_dtype,
                          uint32_t rows, const pw_projection *proj, void *output,
                          uint32_t output_dtype, uint32_t round_output, void *stream);

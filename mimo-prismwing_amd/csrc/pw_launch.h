@@ -195,7 +195,7 @@ inline void timer_end(int slot, hipStream_t s)
 
 // f32 [n] -> three bf16 planes [3][n]
 void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream_t stream);
-// Block-FP8 projection (pw_linear.hip): x [W][K] 16-byte aligned, bf16 or f32 (mode A) or e4m3 codes
+// Block-FP8 projection (pw_linear.hip): x [W][K] bf16 or f32 (mode A) or 16-byte aligned e4m3 codes
 // with x_scales [W][K / 128] (mode B); partial: SHARE_SUM_BYTES.
 enum WideX : int { WX_BF16 = 0, WX_F32 = 1, WX_CODES = 2 };
 uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles);

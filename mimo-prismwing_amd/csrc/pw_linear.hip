@@ -91,7 +91,12 @@ void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void
     args.round_f32 = round_f32;
     const int rt = pick_rt(xt, W, K, n_tiles);
     const int t = timer_begin(xt == WX_CODES ? K_LINEAR_B : K_LINEAR_A, stream);
-    if (xt == WX_F32)
+    const bool aligned = ((uintptr_t)x & 15) == 0;
+    if (xt == WX_F32 && !aligned)
+        launch_wide_unaligned<WK_PROJ, WX_F32>(args, rt, stream);
+    else if (xt == WX_BF16 && !aligned)
+        launch_wide_unaligned<WK_PROJ, WX_BF16>(args, rt, stream);
+    else if (xt == WX_F32)
         launch_wide<WK_PROJ, WX_F32>(args, rt, stream);
     else if (xt == WX_BF16)
         launch_wide<WK_PROJ, WX_BF16>(args, rt, stream);

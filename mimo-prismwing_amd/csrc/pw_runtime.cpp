@@ -142,7 +142,7 @@ struct pw_runtime {
     bool host_pending = false;  // a call left before its wait: its transfers may still be running
     // routed-MoE per-layer scratch
     DevBuf moe_plan, moe_active_expert, moe_active_offset, moe_pos, moe_w, moe_slots, moe_hidden,
-        moe_hidden_planes, moe_x_planes, moe_y, moe_xq, moe_xs, moe_hq, moe_hs, lin_planes,
+        moe_hidden_planes, moe_x_planes, moe_y, moe_xq, moe_xs, moe_hq, moe_hs,
         moe_active, moe_pieces, moe_partial, moe_sched, pf_tiles, pf_silu, router_scores, share_sums;
     MoeBuffers mb{};
     pw::KernelTimer timer;
@@ -914,13 +914,6 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
     const pw::WideX xt = mode == PW_MODE_B ? pw::WX_CODES : x_f32 ? pw::WX_F32 : pw::WX_BF16;
     float *partial = (float *)rt->share_sums.p;
     if (mode == PW_MODE_A) {
-        if ((uintptr_t)x & 15) {
-            // rows off 16 bytes (a caller's slice): the projection's copies take an aligned one
-            const size_t bytes = (size_t)rows * p->columns * (x_f32 ? 4 : 2);
-            PW_HIP(rt->lin_planes.ensure(bytes));
-            PW_HIP(hipMemcpyAsync(rt->lin_planes.p, x, bytes, hipMemcpyDeviceToDevice, stream));
-            x = rt->lin_planes.p;
-        }
         pw::launch_linear(xt, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, partial, y32, y16, p->rows, round_f32,
                           stream);
     } else if (mode == PW_MODE_B) {

@@ -122,16 +122,14 @@ struct WideStream {
     static_assert(XR * UPR % 64 == 0, "whole copies");
     static_assert(LDS * 16 <= 160 * 1024, "a workgroup's LDS");
 
-    // step columns [col, col + SC) of the activation rows -> LDS (row r's unit u at r * UPR + (u ^ (r & 7)))
-    static __device__ __forceinline__ void copy_x(const char *x, uint32_t W, uint32_t K, uint32_t col, uint4 *slot,
-                                                  int lane)
+    // Step columns [col, col + SC) of the activation rows -> LDS (row r's unit u at r * UPR + (u ^ (r & 7))):
+    // the source of unit c * 64 + lane of the slot.
+    static __device__ __forceinline__ const char *x_unit(const char *x, uint32_t W, uint32_t K, uint32_t col, int c,
+                                                         int lane)
     {
-#pragma unroll
-        for (int c = 0; c < XC; ++c) {
-            const uint32_t p = c * 64 + lane, row = p / UPR, u = (p % UPR) ^ (row & 7);
-            const uint32_t r = row < W ? row : W - 1;  // rows past the batch repeat its last row
-            lds_load16(x + ((size_t)r * K + col) * XB + u * 16, slot + c * 64);
-        }
+        const uint32_t p = c * 64 + lane, row = p / UPR, u = (p % UPR) ^ (row & 7);
+        const uint32_t r = row < W ? row : W - 1;  // rows past the batch repeat its last row
+        return x + ((size_t)r * K + col) * XB + u * 16;
     }
 
     // the row of tile nt that lane r16 reads (a tile of fewer than sixteen staged rows repeats them)
@@ -142,7 +140,11 @@ struct WideStream {
     }
 };
 
-template <int KIND, int XT, int XR, int RT>
+// AL: the activation rows start on 16 bytes. A step's columns of rows that do not (a caller's slice) go
+// through registers while its weights are on their way, so they need no aligned copy in memory (us,
+// aligned / off 16 bytes / with a copy launch before it: 13568 x 4096, 8 f32 rows 15.6 / 16.0 / 17.6, 32
+// 22.1 / 22.3 / 24.2, 8 bf16 rows 13.7 / 14.2 / 15.8, 32 16.7 / 21.5 / 19.2).
+template <int KIND, int XT, int XR, int RT, bool AL = true>
 __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
 {
     using S = WideStream<KIND, XT, XR, RT>;
@@ -230,7 +232,15 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
             for (int r = 0; r < RT; ++r)
                 sw[s][r] = load_g(ws[r] + b);
         asm volatile("" ::: "memory");
-        S::copy_x(x, W, K, col, slots + s * S::SLOT, lane);
+        u32x4 xv[AL ? 1 : XC];
+#pragma unroll
+        for (int c = 0; c < XC; ++c) {
+            const char *src = S::x_unit(x, W, K, col, c, lane);
+            if constexpr (AL)
+                lds_load16(src, slots + s * S::SLOT + c * 64);
+            else
+                __builtin_memcpy(&xv[c], src, 16);
+        }
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int r = 0; r < RT; ++r)
@@ -240,6 +250,12 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
                                                 (KIND == WK_BF16 ? (h / 2) * 128 + (h % 2) * 16
                                                                  : h * (XT == WX_CODES ? 16 : 64)));
         asm volatile("" ::: "memory");
+        if constexpr (!AL) {  // (the wave's LDS operations keep their order)
+#pragma unroll
+            for (int c = 0; c < XC; ++c)
+                slots[s * S::SLOT + c * 64 + lane] = __builtin_bit_cast(uint4, xv[c]);
+            asm volatile("" ::: "memory");
+        }
     };
     // N loads issued after step s's own may be outstanding
     auto compute = [&](auto s_, auto n_) __attribute__((always_inline)) {
@@ -529,10 +545,16 @@ static inline int pick_rt(int xt, uint32_t W, uint32_t K, uint32_t n_tiles)
     return n_tiles <= 512 ? 2 : 4;
 }
 
+template <int KIND>
+static dim3 wide_grid(const WideArgs &args, int rt)
+{
+    return dim3((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND != WK_GATEUP ? args.KS : 1u));
+}
+
 template <int KIND, int XT, int XR>
 static void launch_wide_rt(const WideArgs &args, int rt, hipStream_t stream)
 {
-    const dim3 grid((args.n_tiles + rt - 1) / (uint32_t)rt * (KIND != WK_GATEUP ? args.KS : 1u)), block(512);
+    const dim3 grid = wide_grid<KIND>(args, rt), block(512);
     if (rt == 4)
         hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 4>), grid, block, 0, stream, args);
     else if (KIND == WK_BF16 && rt == 3)
@@ -558,6 +580,29 @@ static void launch_wide(const WideArgs &args, int rt, hipStream_t stream)
         launch_wide_rt<KIND, XT, XT == WX_F32 ? 24 : 32>(args, rt, stream);
     else
         launch_wide_rt<KIND, XT, 32>(args, rt, stream);
+}
+
+// Rows off 16 bytes: eight, sixteen or 32 staged rows, one or four tiles.
+template <int KIND, int XT, int XR>
+static void launch_unaligned_xr(const WideArgs &args, int rt, hipStream_t stream)
+{
+    const dim3 grid = wide_grid<KIND>(args, rt), block(512);
+    if (rt == 1)
+        hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 1, false>), grid, block, 0, stream, args);
+    else
+        hipLaunchKernelGGL((wide_kernel<KIND, XT, XR, 4, false>), grid, block, 0, stream, args);
+}
+
+template <int KIND, int XT>
+static void launch_wide_unaligned(const WideArgs &args, int rt, hipStream_t stream)
+{
+    rt = rt == 1 ? 1 : 4;
+    if (args.W <= 8)
+        launch_unaligned_xr<KIND, XT, 8>(args, rt, stream);
+    else if (args.W <= 16)
+        launch_unaligned_xr<KIND, XT, 16>(args, rt, stream);
+    else
+        launch_unaligned_xr<KIND, XT, 32>(args, rt, stream);
 }
 
 }  // namespace pw

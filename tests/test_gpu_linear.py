@@ -148,10 +148,10 @@ def test_projection_tile_and_step_edges(rt, n, k):
         assert np.array_equal(run_device(rt, proj_i, xi[:rows], mode=P.MODE_B, x_dtype=P.DTYPE_F32), ref_i[:rows]), rows
 
 
-@pytest.mark.parametrize("weights", ["fp8", "bf16"])
-def test_mode_a_first_call_under_graph_capture(rt, weights):
+@pytest.mark.parametrize("weights,off", [("fp8", 0), ("fp8", 1), ("bf16", 0)])
+def test_mode_a_first_call_under_graph_capture(rt, weights, off):
     """Mode A and BF16 projections allocate nothing in a call, also where K runs in shares whose sums
-    a second launch adds: a runtime's first call is one under capture, and every replay gives the
+    a second launch adds or the rows start off 16 bytes: a runtime's first call is one under capture, and every replay gives the
     eager call's bits, with larger eager calls (more rows, more shares' sums) between replays."""
     torch = _torch()
     rng = np.random.default_rng(91)
@@ -174,7 +174,8 @@ def test_mode_a_first_call_under_graph_capture(rt, weights):
     eager = bind(rt, n)
     rng.bit_generator.state = state
     captured, larger = bind(cap, n), bind(cap, 2000)
-    x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).cuda().bfloat16()
+    x = torch.empty(rows * k + off, dtype=torch.bfloat16, device="cuda")[off:].view(rows, k)
+    x.copy_(torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)))
     x32 = torch.from_numpy(rng.standard_normal((32, k)).astype(np.float32)).cuda().bfloat16()
     want, got = (torch.empty((rows, n), dtype=torch.float32, device="cuda") for _ in range(2))
     more = torch.empty((32, 2000), dtype=torch.float32, device="cuda")
@@ -215,6 +216,31 @@ def test_mode_a_rows_off_16_bytes(rt, kind):
         torch.cuda.synchronize()
         outs.append(out)
     assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+@pytest.mark.parametrize("n,k", [(4104, 1152), (1000, 8192)])
+def test_mode_a_rows_off_16_bytes_edges(rt, kind, n, k):
+    """The same with four tiles a workgroup (a partial last one) and in four K shares, up to eight
+    rows and more, starting one and three values off."""
+    torch = _torch()
+    rng = np.random.default_rng(77)
+    s = log_uniform_scales(rng, n, k)
+    proj = rt.bind_projection(fp8_weight(rng, n, k, s), s)
+    dt, pt = (torch.float32, P.DTYPE_F32) if kind == "f32" else (torch.bfloat16, P.DTYPE_BF16)
+    for rows in (1, 5, 9, 32):
+        x = torch.from_numpy(rng.standard_normal((rows, k)).astype(np.float32)).to(dt).cuda()
+        outs = []
+        for off in (0, 1, 3):
+            t = torch.empty(rows * k + off, dtype=dt, device="cuda")[off:].view(rows, k)
+            t.copy_(x)
+            out = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+            rt.fp8_linear_device(proj, t, rows, out, mode=P.MODE_A, x_dtype=pt, out_dtype=P.DTYPE_F32_RAW,
+                                 stream=torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            outs.append(out)
+        assert torch.equal(outs[0].view(torch.int32), outs[1].view(torch.int32)), rows
+        assert torch.equal(outs[0].view(torch.int32), outs[2].view(torch.int32)), rows
 
 
 def test_real_checkpoint_gemv_fixture(rt, golden_dir):
