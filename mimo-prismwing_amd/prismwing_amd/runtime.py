@@ -7,6 +7,7 @@ raw device addresses) and enqueue on the runtime's HIP stream.
 from __future__ import annotations
 
 import ctypes
+import operator
 from dataclasses import dataclass
 from typing import Iterable, Optional, Sequence
 
@@ -86,13 +87,17 @@ _BINDING = np.dtype([("expert", "<u4"), ("count", "<u4"), ("positions", "<u8"), 
 assert _BINDING.itemsize == ctypes.sizeof(_abi.ExpertBindingC)
 
 
+def _flat_list(v):
+    return type(v) is list and (not v or isinstance(v[0], (int, float, np.generic)))
+
+
 def _expert_bindings(experts):
     """The C bindings of a batch and what keeps their pointers alive. The positions and weights of all
     bindings sit in one array each: an array and a pointer object per binding were most of the call's host time."""
     pos, weights, counts, pos_at, w_at = [], [], [], [], []
     for b in experts:
         p, w = b.positions, b.route_weights
-        if type(p) is not list or type(w) is not list:  # any array-like
+        if not _flat_list(p) or not _flat_list(w):  # any array-like
             p, w = np.ascontiguousarray(p, dtype=np.uint32), np.ascontiguousarray(w, dtype=np.float32)
         counts.append(len(p))
         pos_at.append(len(pos))
@@ -101,7 +106,7 @@ def _expert_bindings(experts):
         weights += w if type(w) is list else w.reshape(-1).tolist()
     pos, weights = np.array(pos, dtype=np.uint32), np.array(weights, dtype=np.float32)
     rec = np.zeros(len(counts), _BINDING)
-    rec["expert"] = [b.expert & 0xFFFFFFFF for b in experts]
+    rec["expert"] = [operator.index(b.expert) & 0xFFFFFFFF for b in experts]
     rec["count"] = counts
     rec["positions"] = np.array(pos_at, np.uint64) * 4 + np.uint64(pos.ctypes.data)
     rec["route_weights"] = np.array(w_at, np.uint64) * 4 + np.uint64(weights.ctypes.data)

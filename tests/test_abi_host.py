@@ -193,3 +193,30 @@ def test_expert_bindings_by_columns():
         assert [c.route_weights[j] for j in range(c.count)] == np.asarray(b.route_weights, np.float32).tolist()
         assert (c.gate, c.up, c.down) == (b.gate.handle, b.up.handle, b.down.handle)
     assert len(_expert_bindings([])[1][0]) == 0
+
+
+def test_expert_bindings_take_any_integer_id_and_nested_rows():
+    """Expert ids of any integer type (numpy's narrow ones do not hold the 32-bit mask), negative ones
+    wrapped to 32 bits; positions and weights as nested or one-element sequences, read in order; ids
+    that are no integers refused."""
+    from prismwing_amd.runtime import _expert_bindings
+
+    class Proj:
+        handle = 1
+
+    def bind(expert, pos, w):
+        return P.WideExpertBinding(expert, pos, w, Proj(), Proj(), Proj())
+
+    ids = [np.int8(5), np.uint8(200), np.int16(300), np.int32(7), np.uint32(8), np.int64(9), np.uint64(10), True, -1]
+    batch = [bind(e, [i], [0.5]) for i, e in enumerate(ids)]
+    batch.append(bind(3, [[4], [2]], [[0.25], [0.75]]))
+    batch.append(bind(3, [np.int32(6), np.int64(1)], [np.float32(0.1), 0.2]))
+    batch.append(bind(3, [np.array([5])], [np.array([0.125])]))
+    arr, keep = _expert_bindings(batch)
+    assert [arr[i].expert for i in range(len(ids))] == [5, 200, 300, 7, 8, 9, 10, 1, 0xFFFFFFFF]
+    got = [([c.positions[j] for j in range(c.count)], [c.route_weights[j] for j in range(c.count)])
+           for c in (arr[i] for i in range(len(batch)))]
+    assert got[:len(ids)] == [([i], [0.5]) for i in range(len(ids))]
+    assert got[len(ids):] == [([4, 2], [0.25, 0.75]), ([6, 1], np.float32([0.1, 0.2]).tolist()), ([5], [0.125])]
+    with pytest.raises(TypeError):
+        _expert_bindings([bind(1.0, [0], [1.0])])
