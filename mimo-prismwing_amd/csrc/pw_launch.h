@@ -250,7 +250,7 @@ struct QuantJob {
 // *quantised tells whether it did.
 // piece_rows: the batch's projections take mb.pieces, entries of at most that many slots
 // (moe_piece_rows of the layer that follows; 0: no pieces; batches of at most 128 rows).
-uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows);
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t max_count);
 bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const float *weights,
                          uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb, uint32_t piece_rows,
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles = nullptr,

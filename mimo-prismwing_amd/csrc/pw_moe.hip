@@ -94,21 +94,24 @@ __device__ __forceinline__ void place_route_row(const RouteRow &rr, uint32_t p, 
 }
 
 // The schedule of a decode batch also cuts every routed expert's slots into entries of at most this many
-// rows, with their token rows, for the projections (see launch_a_moe and launch_b_fused).
-uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows)
+// rows, with their token rows, where the projections take such entries (see launch_a_moe and
+// launch_experts); 0 where none of the batch's experts has more rows than one entry holds (max_count at
+// most), so that no schedule writes a table that nothing reads.
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t max_count)
 {
-    if (mode != 0)
-        return rows <= 8 ? 4u : 8u;  // mode B takes pieces for experts of more than 16 rows only
-    return x_f32 ? 3u : 4u;
+    if (mode != 0)  // mode B takes pieces for experts of more than 16 rows only
+        return max_count > 16 ? 8u : 0u;
+    const uint32_t piece = x_f32 ? 3u : 4u;
+    return max_count > piece ? piece : 0u;
 }
 constexpr uint32_t PIECE_MAX_ROWS = 8;
 
 // At most this many entries of piece_rows rows: one per routed expert and one for every further
-// piece_rows of its slots.
+// piece_rows of its slots; none for no pieces.
 static uint32_t piece_bound(uint32_t rows, uint32_t max_active, uint32_t piece_rows)
 {
     const uint32_t P = rows * 8, U = max_active < P ? max_active : P;
-    return U + (P - U) / piece_rows;
+    return piece_rows ? U + (P - U) / piece_rows : 0u;
 }
 
 // Group `group` of qj (128 columns of a row) by 16 lanes: quantised, or split into its planes.
@@ -208,7 +211,7 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
             c += __popc(mask[e * words + w]);
         }
     // slots and pieces in one word each of the first sum (at most 1024 of either)
-    const uint32_t np = (c + piece_rows - 1) / piece_rows;
+    const uint32_t np = max_pieces ? (c + piece_rows - 1) / piece_rows : 0u;
     uint32_t off, act, total, n_active;
     block_exclusive_scan2(c | (np << 16), c ? 1u : 0u, s_scan, off, act, total, n_active);
     const uint32_t pbase = off >> 16, n_pieces = total >> 16;
@@ -742,29 +745,31 @@ __device__ __forceinline__ void schedule_wave_body(
     // the projections' entries: each routed expert's slots in pieces of at most piece_rows (up to
     // four here), so their LDS stages are sized for that many rows (see launch_a_moe); a piece
     // carries its slots' token rows (of an expert's at most eight)
-    const uint32_t np = (c_a + piece_rows - 1) / piece_rows;  // 0 past the routed experts
-    const uint32_t pincl = wave_inclusive_scan(np);
-    const uint32_t pbase = pincl - np, npieces = __builtin_amdgcn_readlane(pincl, 63);
-    for (uint32_t i = 0; i < np; ++i) {
-        if (pbase + i < max_pieces) {
-            const uint32_t left = c_a - i * piece_rows;
-            const uint32_t pc = left < piece_rows ? left : piece_rows;
-            const uint16_t *tk = tok_of + a * 16 + i * piece_rows;
-            u32x4 *dst = (u32x4 *)(pieces + pbase + i);
-            dst[0] = ep0;
-            dst[1] = ep1;
-            dst[2] = ep2;
-            dst[3] = u32x4{off_a + i * piece_rows, pc, (uint32_t)tk[0] | ((uint32_t)tk[1] << 16),
-                           (uint32_t)tk[2] | ((uint32_t)tk[3] << 16)};
-            dst[4] = u32x4{0u, 0u, 0u, 0u};
-            dst[5] = u32x4{0u, 0u, 0u, 0u};
+    if (max_pieces) {  // (uniform)
+        const uint32_t np = (c_a + piece_rows - 1) / piece_rows;  // 0 past the routed experts
+        const uint32_t pincl = wave_inclusive_scan(np);
+        const uint32_t pbase = pincl - np, npieces = __builtin_amdgcn_readlane(pincl, 63);
+        for (uint32_t i = 0; i < np; ++i) {
+            if (pbase + i < max_pieces) {
+                const uint32_t left = c_a - i * piece_rows;
+                const uint32_t pc = left < piece_rows ? left : piece_rows;
+                const uint16_t *tk = tok_of + a * 16 + i * piece_rows;
+                u32x4 *dst = (u32x4 *)(pieces + pbase + i);
+                dst[0] = ep0;
+                dst[1] = ep1;
+                dst[2] = ep2;
+                dst[3] = u32x4{off_a + i * piece_rows, pc, (uint32_t)tk[0] | ((uint32_t)tk[1] << 16),
+                               (uint32_t)tk[2] | ((uint32_t)tk[3] << 16)};
+                dst[4] = u32x4{0u, 0u, 0u, 0u};
+                dst[5] = u32x4{0u, 0u, 0u, 0u};
+            }
         }
-    }
-    for (uint32_t d = npieces + (uint32_t)lane; d < max_pieces; d += 64) {
-        u32x4 *dst = (u32x4 *)(pieces + d);
+        for (uint32_t d = npieces + (uint32_t)lane; d < max_pieces; d += 64) {
+            u32x4 *dst = (u32x4 *)(pieces + d);
 #pragma unroll
-        for (int i = 0; i < 6; ++i)
-            dst[i] = u32x4{0u, 0u, 0u, 0u};
+            for (int i = 0; i < 6; ++i)
+                dst[i] = u32x4{0u, 0u, 0u, 0u};
+        }
     }
     if ((uint32_t)lane < P) {
         if (bad) {
@@ -915,12 +920,12 @@ bool launch_route_set_schedule(const float *scores, const float *bias, const Exp
     const size_t table = (size_t)E * sizeof(ExpertPtrs);  // <= 12 KB
     const QuantJob qj = quant ? *quant : QuantJob{};
     const uint32_t quant_wgs = (qj.rows * (qj.K >> 7) + 31) / 32;
+    const uint32_t max_pieces = piece_bound(rows, max_active, piece_rows);
     const int t = timer_begin(K_ROUTE_SCHEDULE, stream);
 #define PW_RSS(NC)                                                                                                 \
     hipLaunchKernelGGL(route_set_schedule_kernel<NC>, dim3(1 + quant_wgs), dim3(512), table, stream, scores, bias,  \
                        bank, rows, E, max_active, set_ids, mb.plan, mb.active_expert, mb.active_offset, mb.active,  \
-                       mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, piece_bound(rows, max_active, piece_rows),         \
-                       piece_rows, flags, qj)
+                       mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces, piece_rows, flags, qj)
     if (E <= 64) PW_RSS(1);
     else if (E <= 128) PW_RSS(2);
     else PW_RSS(4);
@@ -1222,7 +1227,7 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles, const QuantJob *quant,
                          bool *quantised)
 {
-    const uint32_t max_pieces = piece_rows ? piece_bound(rows, max_active, piece_rows) : 0u;
+    const uint32_t max_pieces = piece_bound(rows, max_active, piece_rows);
     bool complete = false;
     if (quantised)
         *quantised = false;
@@ -1247,7 +1252,7 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
         hipLaunchKernelGGL(moe_schedule_wave_kernel, dim3(1 + quant_wgs), dim3(64), table, stream, bank, ids, weights,
                            rows, E, max_active, mb.plan, mb.active_expert, mb.active_offset, mb.active,
                            mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces,
-                           piece_rows ? piece_rows : 1u, flags, qj);
+                           piece_rows, flags, qj);
         if (quant_wgs)
             *quantised = true;
     }
@@ -1262,7 +1267,7 @@ bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const floa
         hipLaunchKernelGGL(moe_schedule_kernel, dim3(1 + quant_wgs), dim3(1024), lds, stream, bank, ids, weights, rows,
                            E, max_active, with_prefix, mb.plan, mb.active_expert, mb.active_offset, mb.active,
                            mb.placement_pos, mb.placement_w, mb.row_slots, mb.pieces, max_pieces,
-                           piece_rows ? piece_rows : 1u, flags, tt, qj);
+                           piece_rows, flags, tt, qj);
     } else {
         // rows <= 4096 (SCHED_MAX_WORDS words) and E <= 1024 (one plan thread per expert)
         const SchedScratch ss = sched_carve(mb.sched, rows, E, nullptr);
@@ -1309,8 +1314,8 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
     // with four bf16 rows or three f32 ones (three planes each). 19 f32 rows with skewed routes: the
     // layer 542 -> 388 us against stages of 19 rows (split-K gate/up with partials through memory,
     // down in four K splits).
-    const uint32_t piece_rows = moe_piece_rows(0, x_f32, rows);
-    const bool pieces = max_count > piece_rows;
+    const uint32_t piece_rows = moe_piece_rows(0, x_f32, max_count);
+    const bool pieces = piece_rows != 0;
     const uint32_t entries = pieces ? piece_bound(rows, max_active, piece_rows) : max_active;
     const uint32_t cnt = pieces ? piece_rows : max_count;
     const uint16_t *xp = (const uint16_t *)x;
@@ -1456,8 +1461,8 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
     if (!x_prepared)
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
     // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces
-    const uint32_t piece_rows = moe_piece_rows(1, x_f32, rows);
-    const bool pieces = max_count > 16;
+    const uint32_t piece_rows = moe_piece_rows(1, x_f32, max_count);
+    const bool pieces = piece_rows != 0;
     const ActiveExpert *entries = pieces ? mb.pieces : mb.active;
     if (pieces) {
         max_active = piece_bound(rows, max_active, piece_rows);

@@ -1251,7 +1251,7 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
                           mode == PW_MODE_A ? rt->mb.x_planes : nullptr};
     bool quantised = false;
     pw::launch_moe_schedule((const ExpertPtrs *)d_table, (const uint32_t *)d_ids, (const float *)d_ws, rows, n_experts,
-                            std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, rows),
+                            std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, max_count),
                             rt->d_flags, rt->stream, nullptr,
                             prepare ? &qj : nullptr, prepare ? &quantised : nullptr);
     pw::launch_moe_layer(mode, (const ExpertPtrs *)d_table, rt->mb, x, x_f32, rows,
