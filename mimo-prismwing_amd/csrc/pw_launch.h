@@ -50,6 +50,9 @@ struct KernelTimer {
     }
 };
 
+// Rows that an entry of a decode projection holds at most (the tokens of one MFMA).
+constexpr uint32_t MOE_ENTRY_ROWS = 16;
+
 // Per-layer device scratch of the routed-MoE launch, sized for `max_rows` token rows.
 struct MoeBuffers {
     MoePlan *plan;
@@ -146,8 +149,6 @@ void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W
 void launch_round_output(const float *y, uint32_t ks, uint32_t n, float *out_f32, uint16_t *out_bf16, bool raw,
                          uint32_t *flags, hipStream_t stream);
 
-// Gate/up with the SwiGLU fused and no split partials (pw_moe_a.hip), when the routed rows fit the
-// LDS stage; returns false (nothing launched) otherwise.
 // Down and combine of a one-token decode batch in one launch (mode A, I = 2048, eight routed
 // experts; args are the down projection's, whose rows are the eight placement slots): the same
 // arithmetic as the split-K down followed by the combine; false when the batch does not fit it.
@@ -159,6 +160,9 @@ bool launch_moe_a_down_combine1(const SplitArgs &args, const MoePlan *plan, cons
 // Whether a one-token mode A layer of hidden H and intermediate I runs as the fused gate/up and the
 // one-token down+combine (both reading the token's routes directly, no schedule launch).
 bool moe_a_one_token_direct(uint32_t H, uint32_t I);
+// Gate/up with the SwiGLU fused and no split partials (pw_moe_a.hip), for K columns, R rows and cap
+// routed rows of ns planes an entry that it fits; false (nothing launched) otherwise.
+bool moe_a_gateup_fits(int ns, uint32_t K, uint32_t R, uint32_t cap);
 bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_active, uint16_t *hidden_planes,
                                hipStream_t stream);
 // gate/up split sums -> SwiGLU -> hidden as three bf16 planes [3][P][I]
@@ -250,7 +254,8 @@ struct QuantJob {
 // *quantised tells whether it did.
 // piece_rows: the batch's projections take mb.pieces, entries of at most that many slots
 // (moe_piece_rows of the layer that follows; 0: no pieces; batches of at most 128 rows).
-uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t max_count);
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows, uint32_t max_active, uint32_t max_count, uint32_t H,
+                        uint32_t I);
 bool launch_moe_schedule(const ExpertPtrs *bank, const uint32_t *ids, const float *weights,
                          uint32_t rows, uint32_t E, uint32_t max_active, const MoeBuffers &mb, uint32_t piece_rows,
                          uint32_t *flags, hipStream_t stream, const PfTileTable *tiles = nullptr,

@@ -96,15 +96,33 @@ __device__ __forceinline__ void place_route_row(const RouteRow &rr, uint32_t p, 
 // The schedule of a decode batch also cuts every routed expert's slots into entries of at most this many
 // rows, with their token rows, where the projections take such entries (see launch_a_moe and
 // launch_experts); 0 where none of the batch's experts has more rows than one entry holds (max_count at
-// most), so that no schedule writes a table that nothing reads.
-uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t max_count)
+// most), so that no schedule writes a table that nothing reads. An entry reads its expert's weights for
+// itself, so entries follow the rows per expert (slots over the experts that can be routed):
+//   - Mode A, up to 1.6 rows an expert, where the fused gate/up takes the shape: small LDS stages, so
+//     that more workgroups share a CU, are worth the few experts that are read twice.
+//   - Mode A beyond that: eight rows, and sixteen (the MFMA's tokens) from four rows an expert on, from
+//     seven where the fused gate/up takes the rows of eight.
+//   - Mode B: sixteen rows.
+// Layer, us, three or four rows an entry (mode A) or eight (mode B) / this rule / one entry of up to 32
+// rows (two tiles of tokens) an expert: 4096 x 2048, mode A, bf16 rows, 32 over 16 experts
+// 244 / 133 / 142, 16 over 32 experts 183 / 154 / 180, 9 over 256 experts 262 / 261 / 302, f32 rows, 32
+// over 32 experts 338 / 189 / 262; mode B, 32 over 16 experts 170 / 130 / 122; 1024 x 512, bf16 rows, 32
+// over 32 experts 36.3 / 29.1 / 31.0. The last split stays ahead in banks of 8 and 16 experts only (mode B
+// above; 1024 x 512, mode A, 24 bf16 rows over 16 experts 33.7 / 28.2 / 25.2).
+uint32_t moe_piece_rows(uint32_t mode, bool x_f32, uint32_t rows, uint32_t max_active, uint32_t max_count, uint32_t H,
+                        uint32_t I)
 {
-    if (mode != 0)  // mode B takes pieces for experts of more than 16 rows only
-        return max_count > 16 ? 8u : 0u;
-    const uint32_t piece = x_f32 ? 3u : 4u;
+    const uint32_t P = rows * 8, U = max_active < P ? max_active : P;
+    uint32_t piece = MOE_ENTRY_ROWS;
+    if (mode == 0) {
+        const bool fused = moe_a_gateup_fits(x_f32 ? 3 : 1, H, I, x_f32 ? 3 : 8);
+        if (fused && 5 * P < 8 * U)
+            piece = x_f32 ? 3 : rows <= 8 ? 4 : 6;
+        else if (P < (fused && !x_f32 ? 7 : 4) * U)
+            piece = 8;
+    }
     return max_count > piece ? piece : 0u;
 }
-constexpr uint32_t PIECE_MAX_ROWS = 8;
 
 // At most this many entries of piece_rows rows: one per routed expert and one for every further
 // piece_rows of its slots; none for no pieces.
@@ -261,9 +279,9 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
     if (max_pieces) {  // (uniform) the projections' entries of at most piece_rows slots
         uint32_t w = 0, bits = np ? mask[e * words] : 0u;
         for (uint32_t i = 0; i < np; ++i) {
-            uint32_t tw[PIECE_MAX_ROWS / 2] = {};
+            uint32_t tw[MOE_ENTRY_ROWS / 2] = {};
 #pragma unroll
-            for (uint32_t k = 0; k < PIECE_MAX_ROWS; ++k) {
+            for (uint32_t k = 0; k < MOE_ENTRY_ROWS; ++k) {
                 if (k < piece_rows) {
                     while (!bits && w + 1 < words)
                         bits = mask[e * words + ++w];
@@ -279,8 +297,8 @@ __global__ __launch_bounds__(1024) void moe_schedule_kernel(
                 dst[1] = ep1;
                 dst[2] = ep2;
                 dst[3] = u32x4{off + i * piece_rows, left < piece_rows ? left : piece_rows, tw[0], tw[1]};
-                dst[4] = u32x4{tw[2], tw[3], 0u, 0u};
-                dst[5] = u32x4{0u, 0u, 0u, 0u};
+                dst[4] = u32x4{tw[2], tw[3], tw[4], tw[5]};
+                dst[5] = u32x4{tw[6], tw[7], 0u, 0u};
             }
         }
         for (uint32_t a = n_pieces + tid; a < max_pieces; a += nthr) {
@@ -1307,14 +1325,14 @@ static ExpertOut launch_a_moe(const MoeBuffers &mb, const void *x, bool x_f32, u
 {
     // A routed batch runs both projections on the schedule's pieces of each expert's slots, so their
     // LDS stages hold piece_rows rows instead of as many as the batch could send one expert (an
-    // expert with more rows reads its weights once per piece, from the caches; every slot's
-    // arithmetic is unchanged). Uniform and skewed routes give most experts one to three rows. The
-    // down's stage of four rows (25 KB at hidden 4096) leaves its 98 VGPRs to set its occupancy,
-    // four workgroups per CU (width 8: 90 -> 83 us); the fused gate/up fits two workgroups per CU
-    // with four bf16 rows or three f32 ones (three planes each). 19 f32 rows with skewed routes: the
-    // layer 542 -> 388 us against stages of 19 rows (split-K gate/up with partials through memory,
-    // down in four K splits).
-    const uint32_t piece_rows = moe_piece_rows(0, x_f32, max_count);
+    // expert with more rows reads its weights once per piece, from the caches). Where routes give
+    // most experts one row (moe_piece_rows), the down's stage of four rows (25 KB at hidden 4096)
+    // leaves its 98 VGPRs to set its occupancy, four workgroups per CU (width 8: 90 -> 83 us), and the
+    // fused gate/up fits two workgroups per CU with up to eight bf16 rows or three f32 ones (three
+    // planes each). 19 f32 rows with skewed routes over 256 experts: the layer 542 -> 388 us against
+    // stages of 19 rows. A slot's arithmetic is the same in pieces of up to ten rows; in larger ones the
+    // down's stage takes half the columns, so twice the K splits.
+    const uint32_t piece_rows = moe_piece_rows(0, x_f32, rows, max_active, max_count, H, I);
     const bool pieces = piece_rows != 0;
     const uint32_t entries = pieces ? piece_bound(rows, max_active, piece_rows) : max_active;
     const uint32_t cnt = pieces ? piece_rows : max_count;
@@ -1461,7 +1479,7 @@ static ExpertOut launch_experts(uint32_t mode, const ExpertPtrs *bank, const Moe
     if (!x_prepared)
         launch_quant_group128(x, x_f32, rows, H, mb.xq, mb.xs, flags, stream);
     // experts of more than sixteen rows (one MFMA's tokens) run as the schedule's pieces
-    const uint32_t piece_rows = moe_piece_rows(1, x_f32, max_count);
+    const uint32_t piece_rows = moe_piece_rows(1, x_f32, rows, max_active, max_count, H, I);
     const bool pieces = piece_rows != 0;
     const ActiveExpert *entries = pieces ? mb.pieces : mb.active;
     if (pieces) {

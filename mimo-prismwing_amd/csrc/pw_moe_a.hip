@@ -413,12 +413,17 @@ static size_t fused_lds(int ns, uint32_t cnt, uint32_t K)
     return stage > red ? stage : red;
 }
 
+// four 128-column blocks per wave and split (the split kernel's gate/up stream), eight splits
+// (up to eight bf16 rows or three f32 ones, 74 KB: two workgroups per CU)
+bool moe_a_gateup_fits(int ns, uint32_t K, uint32_t R, uint32_t cap)
+{
+    return K == 8 * 4 * 128 && R % 16 == 0 && (uint32_t)ns * cap <= 9;
+}
+
 bool launch_moe_a_gateup_fused(int ns, const SplitArgs &args, uint32_t max_active, uint16_t *hidden_planes,
                                hipStream_t stream)
 {
-    // four 128-column blocks per wave and split (the split kernel's gate/up stream), eight splits
-    // (up to eight bf16 rows or three f32 ones, 74 KB: two workgroups per CU)
-    if (args.K != 8 * 4 * 128 || args.R % 16 != 0 || (uint32_t)ns * args.cap > 9)
+    if (!moe_a_gateup_fits(ns, args.K, args.R, args.cap))
         return false;
     const size_t lds = fused_lds(ns, args.cap, args.K);
     // one-row experts (a one-token batch) take 8 + 8-row work items: twice the workgroups

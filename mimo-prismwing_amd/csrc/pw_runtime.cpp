@@ -1250,12 +1250,12 @@ int pw_moe_execute(pw_runtime *rt, uint32_t mode, uint32_t fused_gate_up, const 
     const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, rt->mb.xq, rt->mb.xs,
                           mode == PW_MODE_A ? rt->mb.x_planes : nullptr};
     bool quantised = false;
+    const uint32_t max_active = std::min<uint32_t>(n_experts, rows * 8);
     pw::launch_moe_schedule((const ExpertPtrs *)d_table, (const uint32_t *)d_ids, (const float *)d_ws, rows, n_experts,
-                            std::min<uint32_t>(n_experts, rows * 8), rt->mb, pw::moe_piece_rows(mode, x_f32, max_count),
+                            max_active, rt->mb, pw::moe_piece_rows(mode, x_f32, rows, max_active, max_count, H, I),
                             rt->d_flags, rt->stream, nullptr,
                             prepare ? &qj : nullptr, prepare ? &quantised : nullptr);
-    pw::launch_moe_layer(mode, (const ExpertPtrs *)d_table, rt->mb, x, x_f32, rows,
-                         std::min<uint32_t>(n_experts, rows * 8), max_count, H, I,
+    pw::launch_moe_layer(mode, (const ExpertPtrs *)d_table, rt->mb, x, x_f32, rows, max_active, max_count, H, I,
                          (float *)rt->out.p, nullptr, false, rt->d_flags, rt->stream, nullptr, quantised);
     PW_HIP(hipGetLastError());
     uint32_t flags = 0;
@@ -1392,7 +1392,7 @@ static void launch_routed_layer(const MoeBuffers &mb, const pw_expert_bank *bank
     const pw::QuantJob qj{x, x_f32 ? 1u : 0u, rows, H, mb.xq, mb.xs, mode == PW_MODE_A ? mb.x_planes : nullptr};
     bool quantised = false;
     pw::launch_moe_schedule(bank->table, route_ids, route_weights, rows, E, max_active, mb,
-                            pw::moe_piece_rows(mode, x_f32, rows), flags, s, nullptr,
+                            pw::moe_piece_rows(mode, x_f32, rows, max_active, rows, H, I), flags, s, nullptr,
                             prepare ? &qj : nullptr, prepare ? &quantised : nullptr);
     pw::launch_moe_layer(mode, bank->table, mb, x, x_f32, rows, max_active, rows, H, I, out_f32, out_bf16, raw, flags,
                          s, nullptr, quantised);
@@ -1462,7 +1462,7 @@ int pw_moe_layer_routed_device(pw_runtime *rt, const pw_expert_bank *bank, uint3
                           mode == PW_MODE_A ? rt->mb.x_planes : nullptr};
     if (!direct && pw::launch_route_set_schedule(scores, bias, bank->table, rows, E, max_active,
                                                  (uint32_t *)rt->set_ids.p, rt->mb,
-                                                 pw::moe_piece_rows(mode, x_f32, rows), rt->d_flags, s,
+                                                 pw::moe_piece_rows(mode, x_f32, rows, max_active, rows, H, I), rt->d_flags, s,
                                                  prepare ? &qj : nullptr)) {
         // the expert sets are scheduled; the routes' order and weights (a serial partition per row)
         // run in extra workgroups of an expert launch (mode A: the down, mode B: the gate/up) while

@@ -355,6 +355,45 @@ def test_wide_batch_pieces_equal_small_batches(rt, full_bank, mode, x_f32, rows)
         assert np.array_equal(layer(at).view(np.uint32), whole[at].view(np.uint32)), (p, rows)
 
 
+@pytest.mark.parametrize("hidden,inter,n", [(512, 256, 8), (512, 256, 32), (4096, 128, 8), (4096, 128, 40)])
+@pytest.mark.parametrize("rows", [8, 9, 17, 32])
+def test_entries_of_several_rows_match_oracle(rt, hidden, inter, n, rows):
+    """Banks of few experts give an expert many rows: entries of eight and sixteen rows, full ones and
+    remainders (expert 0 has every row, expert 1 every second one), the gate/up fused (hidden 4096, up
+    to three f32 or eight bf16 rows) and split over K, the down in wide and in half columns (more than
+    ten rows). Modes A (f32 and bf16 rows, raw sums) and B against the oracle. Mode A within 2e-7 C: at
+    most 48 roundings a sum, each 2^-24 of a partial sum of about C / sqrt(512) or less, for gate/up and
+    down (a wrong row is about 1e-3 C off)."""
+    import torch
+    rng = np.random.default_rng([hidden, n, rows])
+    experts = make_experts(rng, n, hidden, inter)
+    projs = {e: (rt.bind_projection(v[0], v[1]), rt.bind_projection(v[2], v[3]), rt.bind_projection(v[4], v[5]))
+             for e, v in experts.items()}
+    bank = rt.expert_bank(*[[projs[e][i] for e in range(n)] for i in range(3)])
+    sel = np.empty((rows, 8), np.uint32)
+    for p in range(rows):
+        first = [0] if n > 8 and p % 2 else [0, 1]
+        rest = rng.permutation(np.arange(1 if n == 8 and len(first) == 1 else 2, n))[:8 - len(first)]
+        sel[p] = rng.permutation(np.concatenate([first, rest]))
+    w = rng.uniform(0.01, 0.3, (rows, 8)).astype(np.float32)
+    xb = bf16_normal(rng, (rows, hidden))
+    ids, wts = torch.from_numpy(sel.astype(np.int32)).cuda(), torch.from_numpy(w).cuda()
+    for mode, x_f32 in ((P.MODE_A, False), (P.MODE_A, True), (P.MODE_B, False)):
+        x = rng.standard_normal((rows, hidden)).astype(np.float32) if x_f32 else xb
+        xt = torch.from_numpy(x).cuda() if x_f32 else torch.from_numpy(WL.bf16_bits_np(x).view(np.int16)).cuda()
+        raw = torch.empty((rows, hidden), dtype=torch.float32, device="cuda")
+        rt.moe_layer_device(bank, xt, rows, ids, wts, raw, mode=mode, x_dtype=P.DTYPE_F32 if x_f32 else P.DTYPE_BF16,
+                            out_dtype=P.DTYPE_F32_RAW, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rt.take_flags() == 0
+        _, ref = O.moe_layer("a" if mode == P.MODE_A else "b", x, experts, n, sel, w, raw=True)
+        if mode == P.MODE_A:
+            d = np.abs(raw.cpu().numpy().astype(np.float64) - ref)
+            assert np.all(d <= 2e-7 * moe_condition(x, experts, sel, w)), (x_f32, float(d.max()))
+        else:
+            assert normwise(raw.cpu().numpy(), ref) <= 2e-2 and rel_l2(raw.cpu().numpy(), ref) <= 5e-3
+
+
 @pytest.mark.parametrize("x_f32", [False, True])
 def test_one_token_equals_two_copies(rt, full_bank, x_f32):
     """Each token's result depends only on its own row and routes: a two-row batch holding the
