@@ -19,8 +19,8 @@ import pytest
 
 import oracle as O
 import prismwing_amd as P
-from helpers import (STAGED_CASES, STAGES, _unit_codes, bf16_normal, bf16_round, closed_form_mode_b, decode_table,
-                     fp8_weight, log_uniform_scales, staged_swiglu_independent, to_bf16_bits)
+from helpers import (STAGED_CASES, STAGES, _unit_codes, bf16_normal, bf16_round, closed_form_mode_b, decode_table, dequant,
+                     fp8_weight, log_uniform_scales, rel_l2, staged_swiglu_independent, to_bf16_bits)
 
 pytestmark = pytest.mark.gpu
 
@@ -366,9 +366,8 @@ def _expert_forward(rt, bank, e, x, out_dtype):
 @pytest.mark.parametrize("rows", [1, 8, 16, 17])
 def test_closed_form_mode_b_expert_forward_production_bit_exact(rt, closed_form_production, rows):
     """The one-expert forward in mode B at the production expert shape (hidden 4096, intermediate
-    2048): up to 16 rows run as whole-K workgroups (gate/up of 8 + 8 stacked rows, the down writing
-    the output rows), 17 rows take the split kernels. Bit for bit the oracle's layer, f32 (also as
-    F32_RAW, which in mode B is the rounded expert output) and bf16."""
+    2048) with 8, 16 and 32 staged rows, two 16-token tiles at 17 rows. Bit for bit the oracle's
+    layer, f32 (also as F32_RAW, which in mode B is the rounded expert output) and bf16."""
     experts, x, _, _, _, bank = closed_form_production
     e = 5
     xr = x[:rows]
@@ -381,7 +380,7 @@ def test_closed_form_mode_b_expert_forward_production_bit_exact(rt, closed_form_
 def test_closed_form_mode_b_device_layer_production_rows_bit_exact(rt, closed_form_production, rows):
     """The mode-B decode layer at the production expert shape with one row (one-row experts: 8 + 8
     stacked gate/up rows per workgroup), sixteen rows (sixteen rows per expert in LDS) and seventeen
-    (the split kernels), top-8 of 8 experts; bit for bit the oracle's layer."""
+    (pieces of sixteen rows and of one), top-8 of 8 experts; bit for bit the oracle's layer."""
     experts, x, sel, w, _, bank = closed_form_production
     x, sel, w = x[:rows], sel[:rows], w[:rows]
     want, want_raw = O.moe_layer("b", x, experts, 8, sel, w, raw=True)
@@ -391,22 +390,73 @@ def test_closed_form_mode_b_device_layer_production_rows_bit_exact(rt, closed_fo
 
 @pytest.fixture(scope="module")
 def closed_form_dense(rt):
-    experts, x, sel, w = closed_form_mode_b(0x50570600, 8, 1, hidden=1024, inter=16384, top_k=1, down_block_step=8)
+    experts, x, sel, w = closed_form_mode_b(0x50570600, 16, 1, hidden=1024, inter=16384, top_k=1, down_block_step=8)
     projs, bank = _bank_from(rt, experts, 1)
     return experts, x, projs, bank
 
 
-@pytest.mark.parametrize("rows", [1, 8])
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
 def test_closed_form_mode_b_dense_mlp_bit_exact(rt, closed_form_dense, rows):
     """The dense layer-0 MLP's intermediate 16384 as a one-expert bank in mode B (hidden 1024 keeps
-    the fixture small): the down's K of 16384 runs as four K shares whose sums are added in share
-    order by the output rounding (the down weights hold codes in every eighth 128-column block, four
-    blocks per share, which keeps every sum exact). Bit for bit the oracle's layer, f32 and bf16."""
+    the fixture small): the down's K of 16384 runs in one share for up to eight rows and in four for
+    more, whose sums the output rounding adds in share order (the down weights hold codes in every
+    eighth 128-column block, four blocks per share, which keeps every sum exact). Bit for bit the
+    oracle's layer, f32 and bf16."""
     experts, x, _, bank = closed_form_dense
     xr = x[:rows]
     want = O.moe_layer("b", xr, experts, 1, np.zeros((rows, 1), np.uint32), np.ones((rows, 1), np.float32))
     for dt in (P.DTYPE_F32, P.DTYPE_BF16):
         _same_bits(_expert_forward(rt, bank, 0, xr, dt), want)
+
+
+@pytest.fixture(scope="module")
+def closed_form_two_shares(rt):
+    experts, x, sel, w = closed_form_mode_b(0x50570700, 32, 1, hidden=2176, inter=16384, top_k=1, down_block_step=8)
+    projs, bank = _bank_from(rt, experts, 1)
+    return experts, x, projs, bank
+
+
+@pytest.mark.parametrize("rows", [19, 20, 24, 32])
+def test_closed_form_mode_b_two_share_down_bit_exact(rt, closed_form_two_shares, rows):
+    """136 output tiles: from 20 rows on the mode B down runs in two K shares of 32-row workgroups whose
+    sums the output rounding adds, with 19 rows in one. Bit for bit the oracle's layer, f32 and bf16."""
+    experts, x, _, bank = closed_form_two_shares
+    xr = x[:rows]
+    want = O.moe_layer("b", xr, experts, 1, np.zeros((rows, 1), np.uint32), np.ones((rows, 1), np.float32))
+    for dt in (P.DTYPE_F32, P.DTYPE_BF16):
+        _same_bits(_expert_forward(rt, bank, 0, xr, dt), want)
+
+
+@pytest.mark.parametrize("rows", [11, 12, 16, 32])
+def test_mode_a_two_share_down(rt, closed_form_two_shares, rows):
+    """The same expert in mode A (two shares from 12 rows on), raw f32 against 64 bits. Gate/up sums are
+    exact; the down's f32 chains have at most 48 roundings (2e-6 of the 2-norm)."""
+    torch = _torch()
+    experts, x, _, bank = closed_form_two_shares
+    gw, gs, uw, us, dw, ds = experts[0]
+    xd = x[:rows].astype(np.float64)
+    g = xd @ dequant(gw, gs).T
+    ref = (g / (1.0 + np.exp(-g)) * (xd @ dequant(uw, us).T)) @ dequant(dw, ds).T
+    out = torch.empty((rows, x.shape[1]), dtype=torch.float32, device="cuda")
+    rt.expert_forward_device(bank, 0, torch.from_numpy(x[:rows]).cuda(), rows, out, mode=P.MODE_A,
+                             x_dtype=P.DTYPE_F32, out_dtype=P.DTYPE_F32_RAW, stream=_stream())
+    torch.cuda.synchronize()
+    assert rt.take_flags() == 0
+    assert rel_l2(out.cpu().numpy(), ref) <= 2e-6
+
+
+@pytest.mark.parametrize("seed,hidden,inter", [(0x50570800, 1024, 128), (0x50570900, 2048, 512),
+                                               (0x50570A00, 1024, 1536)])
+def test_closed_form_mode_b_gateup_shapes_bit_exact(rt, seed, hidden, inter):
+    """Mode B decode layers whose hidden the whole-K gate/up takes (one and two blocks a wave) and whose
+    intermediate is no power of two times 1024, at one, nine and seventeen rows of every expert. Bit for
+    bit the oracle's layer."""
+    experts, x, sel, w = closed_form_mode_b(seed, 17, 8, hidden=hidden, inter=inter)
+    _, bank = _bank_from(rt, experts, 8)
+    for rows in (1, 9, 17):
+        want, want_raw = O.moe_layer("b", x[:rows], experts, 8, sel[:rows], w[:rows], raw=True)
+        _same_bits(_device_layer(rt, bank, x[:rows], sel[:rows], w[:rows], P.DTYPE_F32_RAW), want_raw)
+        _same_bits(_device_layer(rt, bank, x[:rows], sel[:rows], w[:rows], P.DTYPE_BF16), want)
 
 
 # ------------------------------------------------------------------ layer vs separate calls

@@ -1,5 +1,6 @@
 """The test helpers' vectorised e4m3 encoder agrees with the oracle's literal search."""
 import numpy as np
+import pytest
 
 import oracle as O
 from helpers import closed_form_mode_b, decode_table, encode_e4m3, exact_in_f32, fp8_blocks_exact
@@ -87,7 +88,17 @@ def test_closed_form_production_shape_meets_its_preconditions():
 def test_closed_form_dense_intermediate_meets_its_preconditions():
     """The intermediate-16384 closed form of the dense-MLP test (hidden 1024, one expert, down codes
     in every eighth 128-column block) at the GPU test's seed and size."""
-    experts, x, sel, w = closed_form_mode_b(0x50570600, 8, 1, hidden=1024, inter=16384, top_k=1, check=True,
+    experts, x, sel, w = closed_form_mode_b(0x50570600, 16, 1, hidden=1024, inter=16384, top_k=1, check=True,
                                             down_block_step=8)
     out = O.moe_layer("b", x[:1], experts, 1, sel[:1], np.ones((1, 1), np.float32))
     assert np.all(np.isfinite(out)) and np.any(out)
+
+
+@pytest.mark.parametrize("seed,rows,n,kw", [
+    (0x50570700, 32, 1, {"hidden": 2176, "inter": 16384, "top_k": 1, "down_block_step": 8}),
+    (0x50570800, 17, 8, {"hidden": 1024, "inter": 128}), (0x50570900, 17, 8, {"hidden": 2048, "inter": 512}),
+    (0x50570A00, 17, 8, {"hidden": 1024, "inter": 1536})])
+def test_closed_form_shapes_meet_their_preconditions(seed, rows, n, kw):
+    """The closed forms of the two-share down and of the whole-K gate/up's shapes, seeds and sizes as in
+    the GPU tests."""
+    closed_form_mode_b(seed, rows, n, check=True, **kw)
