@@ -420,8 +420,19 @@ int ensure_sched(pw_runtime *rt, uint32_t rows, uint32_t E)
     return PW_OK;
 }
 
+// Split-K partials of the mode A projections of `rows` token rows, for the widest split a launch can
+// pick (entries of at most MOE_ENTRY_ROWS rows).
+size_t moe_partial_bytes(uint32_t rows, uint32_t H, uint32_t I)
+{
+    const size_t P = (size_t)rows * 8;
+    const uint32_t cnt = std::min<uint32_t>(rows, pw::MOE_ENTRY_ROWS);
+    const size_t ks_gu = std::max(pw::plan_split(H, 2, 1, cnt).ks, pw::plan_split(H, 2, 3, cnt).ks);
+    const size_t ks_d = pw::plan_split(I, 1, 3, cnt).ks;
+    return std::max(ks_gu * 2 * P * I, ks_d * P * H) * 4;
+}
+
 // Routed-MoE scratch for `rows` token rows. mode_a_split: also the mode A buffers (activation
-// and hidden bf16 planes, split-K partial sums), which the decode paths (rows <= 128) use.
+// and hidden bf16 planes, split-K partial sums), which the routed decode layers (rows <= 128) use.
 int ensure_moe(pw_runtime *rt, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, bool mode_a_split = true)
 {
     const size_t P = (size_t)rows * 8;
@@ -438,12 +449,8 @@ int ensure_moe(pw_runtime *rt, uint32_t rows, uint32_t E, uint32_t H, uint32_t I
     PW_HIP(rt->moe_xs.ensure((size_t)rows * (H / 128) * 4));
     PW_HIP(rt->moe_hq.ensure(P * I));
     PW_HIP(rt->moe_hs.ensure(P * (I / 128) * 4));
-    // split-K partials of the mode A projections, sized for the widest split the launch can pick
-    const uint32_t cnt = std::min<uint32_t>(rows, 32);
-    const size_t ks_gu = std::max(pw::plan_split(H, 2, 1, cnt).ks, pw::plan_split(H, 2, 3, cnt).ks);
-    const size_t ks_d = pw::plan_split(I, 1, 3, cnt).ks;
     if (mode_a_split)
-        PW_HIP(rt->moe_partial.ensure(std::max(ks_gu * 2 * P * I, ks_d * P * H) * 4));
+        PW_HIP(rt->moe_partial.ensure(moe_partial_bytes(rows, H, I)));
     MoeBuffers &mb = rt->mb;
     mb.partial = (float *)rt->moe_partial.p;
     mb.hidden = (float *)rt->moe_hidden.p;
@@ -528,9 +535,6 @@ size_t carve_moe(char *base, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, 
         return p;
     };
     const size_t P = (size_t)rows * 8;
-    const uint32_t cnt = std::min<uint32_t>(rows, 32);
-    const size_t ks_gu = std::max(pw::plan_split(H, 2, 1, cnt).ks, pw::plan_split(H, 2, 3, cnt).ks);
-    const size_t ks_d = pw::plan_split(I, 1, 3, cnt).ks;
     mb = MoeBuffers{};
     mb.plan = (pw::MoePlan *)take(sizeof(pw::MoePlan));
     mb.active_expert = (uint32_t *)take((E + 1) * 4);
@@ -548,7 +552,7 @@ size_t carve_moe(char *base, uint32_t rows, uint32_t E, uint32_t H, uint32_t I, 
     mb.xs = (float *)take((size_t)rows * (H / 128) * 4);
     mb.hq = (uint8_t *)take(P * I);
     mb.hs = (float *)take(P * (I / 128) * 4);
-    mb.partial = (float *)take(std::max(ks_gu * 2 * P * I, ks_d * P * H) * 4);
+    mb.partial = (float *)take(moe_partial_bytes(rows, H, I));
     mb.sched = nullptr;  // decode batches are scheduled by one wave, without these tables
     mb.max_rows = rows;
     mb.experts = E;
@@ -1678,7 +1682,7 @@ int pw_expert_forward_device(pw_runtime *rt, const pw_expert_bank *bank, uint32_
     hipStream_t s = stream ? (hipStream_t)stream : rt->stream;
     StreamOrder order(rt, s);
     PW_HIP(order.err);
-    PW_TRY(ensure_moe(rt, rows, bank->n_experts, bank->hidden, bank->intermediate));
+    PW_TRY(ensure_moe(rt, rows, bank->n_experts, bank->hidden, bank->intermediate, false));
     pw::launch_expert_forward(mode, bank->host_table[expert], rt->mb, x, x_dtype == PW_DTYPE_F32, rows, bank->hidden,
                               bank->intermediate, out_dtype != PW_DTYPE_BF16 ? (float *)output : nullptr,
                               out_dtype == PW_DTYPE_BF16 ? (uint16_t *)output : nullptr,

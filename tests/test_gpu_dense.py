@@ -111,3 +111,22 @@ def test_expert_tile_and_share_edges(rt, inter):
         gu = [rt.execute_fp8_linear(x[:rows], p, mode=P.MODE_B).output for p in projs[:2]]
         want = rt.execute_fp8_linear(O.swiglu_bf16_staged(*gu), projs[2], mode=P.MODE_B).output
         assert np.array_equal(out.cpu().numpy(), want), rows
+
+
+def test_one_expert_scratch(rt, dense):
+    """The forward's scratch: its hidden values, codes and share sums for 8 x 32 slots (26 MB at
+    4096 x 16384), without the routed layer's split sums and planes (half a GB here)."""
+    import torch
+    _, _, mats = dense
+    r = P.WideMoeRuntime.compile(0)
+    projs = [r.bind_projection_device(*mats[k][:2], *((H, I) if k == "down" else (I, H))) for k in ("gate", "up", "down")]
+    bank = r.expert_bank(*[[p] for p in projs])
+    x = torch.randn((32, H), device="cuda")
+    out = torch.empty((32, H), device="cuda")
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for mode in (P.MODE_A, P.MODE_B):
+        r.expert_forward_device(bank, 0, x, 32, out, mode=mode, x_dtype=P.DTYPE_F32, out_dtype=P.DTYPE_F32)
+        torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 64 << 20
+    assert r.take_flags() == 0
