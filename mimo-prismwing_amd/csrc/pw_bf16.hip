@@ -20,8 +20,15 @@ namespace pw {
 // (us, one / two / four / eight shares: 512 x 8192, one f32 row 12.1 / 9.9 / 8.9 / 8.9, 16 bf16 rows
 // 12.8 / 10.2 / 8.5 / 8.6; 2048 x 8192, 8 f32 rows 14.0 / 11.1 / 12.1 / 14.9; 3000 x 8192, one
 // bf16 row 12.2 / 14.7; 1000 x 5120, 16 f32 rows 11.0 / 10.1 / 9.0; 1000 x 4096, one f32 row 7.9 with
-// one share).
-static uint32_t bf16_shares(uint32_t K, uint32_t n_tiles) { return K < 5120 ? 1u : tile_shares(n_tiles); }
+// one share). From 32 bytes of f32 and 48 of bf16 rows a column on, shares pay from K = 4096 (one / two /
+// four, weights in the memory-side cache | from HBM: 1000 x 4096, 8 f32 rows 7.3 / 7.0 / 6.6 |
+// 8.6 / 8.2 / 7.2, 32 f32 rows 10.6 / 8.8 / 7.6 | 14.9 / 11.5 / 8.9, 32 bf16 rows 7.9 / 7.2 / 6.7 |
+// 10.3 / 8.9 / 7.5; 2000 x 4096, 32 bf16 rows 8.2 / 7.7 / 9.6 | 10.7 / 9.6 / 11.1; 1000 x 2048, 32 bf16 rows
+// 5.4 / 6.6 / 6.6 | 5.9 / 7.3 / 6.4).
+static uint32_t bf16_shares(bool x_f32, uint32_t W, uint32_t K, uint32_t n_tiles)
+{
+    return K >= (W >= (x_f32 ? 8u : 24u) ? 4096u : 5120u) ? tile_shares(n_tiles) : 1u;
+}
 
 // Tiles per workgroup (pw_wide.h's pick_rt for one-byte weights). Twice the weight bytes per tile keep
 // one tile ahead while the activations are up to 16 bytes a column, and up to 32 from 513 to 2304 tiles
@@ -56,7 +63,7 @@ void launch_bf16_linear(const uint16_t *w, const void *x, bool x_f32, uint32_t W
     args.flags = flags;
     args.n_tiles = (R + 15) / 16;
     args.partial = partial;
-    args.KS = bf16_shares(K, args.n_tiles);
+    args.KS = bf16_shares(x_f32, W, K, args.n_tiles);
     args.x = x;
     args.W = W;
     args.K = K;

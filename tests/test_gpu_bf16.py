@@ -153,10 +153,11 @@ def test_fail_closed(rt):
 
 
 @pytest.mark.parametrize("n,k", [(24, 128), (24, 5120), (1100, 5248), (4104, 1152), (8200, 1152), (2100, 640),
-                                 (12296, 1024), (16392, 640)])
+                                 (12296, 1024), (16392, 640), (1000, 4096), (2040, 4224)])
 def test_tile_step_and_share_edges(rt, n, k):
     """Workgroups of one to four 16-row tiles with partial last tiles and a partial last
-    workgroup, four, two and one K shares (24, 1100 and the other rows), waves with no, one and
+    workgroup, four, two and one K shares (24, 1100 and the other rows; 1000 and 2040
+    rows by the batch's), waves with no, one and
     several steps, at staged-row edges. Raw sums of exact products against 64 bits: chains of at most
     5248 / 32 + 8 + 3 f32 roundings per element over random terms (2e-6 of the 2-norm)."""
     import torch
