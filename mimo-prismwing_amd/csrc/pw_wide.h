@@ -515,32 +515,34 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
 
 // Tiles per workgroup. One generation of workgroups over the 256 CUs reads the activations least and
 // has no second start: one tile up to 256 tiles, two up to 512, then four. Where a row's activations
-// are few bytes beside the weights, several small workgroups per CU beat half a chip of larger ones:
-// up to four rows of bf16 or codes keep one tile up to 768 tiles, eight rows from 513 to 768 (us,
-// K = 4096, one / two / four tiles: bf16 width 1, 257 tiles 7.0 / 8.3 / 12.5, 532 tiles
-// 10.9 / 12.6 / 12.7, 848 tiles 14.8 / 14.3 / 13.7; f32 width 16, 257 tiles 14.8 / 11.2 / 15.4, 512
-// tiles 17.4 / 12.2 / 16.8, 532 tiles 23.5 / 20.4 / 16.7). Past 1024 tiles four tiles are several
-// generations of one workgroup per CU, each with its own start: light batches take one tile, batches
-// of up to 32 activation bytes a column two (us of a whole 4096 x 16384 expert, 2048 gate/up tiles:
-// bf16 width 1 40.9 / 44.2 / 47.8, width 16 52.2 / 50.2 / 53.7, width 32 86.2 / 76.4 / 70.8; codes
-// width 24 66.2 / 58.4 / 59.1).
+// are few bytes beside the weights, several small workgroups per CU beat half a chip of larger ones, and
+// keep more loads in flight where the weights come from HBM: up to four rows of bf16 or codes take one
+// tile, but from 769 to 1024 tiles three and four rows two, and of 6144 columns and more four; eight
+// rows one from 513 to 768 (us, K = 4096, one / two / four tiles, weights in the memory-side cache |
+// from HBM: bf16 width 1, 938 tiles 13.1 / 12.8 / 12.3 | 14.3 / 14.4 / 16.5, 1024 tiles
+// 13.3 / 13.4 / 13.0 | 14.7 / 15.2 / 17.9; width 4, 848 tiles 12.5 / 12.3 / 12.0 | 14.4 / 14.2 / 15.5; of
+// 8192 columns, 769 tiles, width 4 19.9 / 21.5 / 19.1 | 22.5 / 24.4 / 22.7; f32 width 16, 257 tiles
+// 14.8 / 11.2 / 15.4, 512 tiles 17.4 / 12.2 / 16.8, 532 tiles 23.5 / 20.4 / 16.7). Past 1024 tiles
+// four tiles are several generations of one workgroup per CU, each with its own start: up to eight rows
+// take one tile, batches of up to 32 activation bytes a column two (us of a whole 4096 x 16384 expert,
+// 2048 gate/up tiles: bf16 width 1 40.9 / 44.2 / 47.8, width 16 52.2 / 50.2 / 53.7, width 32
+// 86.2 / 76.4 / 70.8; codes width 24 66.2 / 58.4 / 59.1).
 // Up to 2048 columns a wave has one or two steps, all in flight at once, so more tiles a workgroup
 // give it nothing to overlap: smaller workgroups keep ahead for longer (us, one / two / four tiles:
-// bf16 width 1, 848 tiles of 1024 columns 6.0 / 6.0 / 6.8, of 2048 8.7 / 8.8 / 9.2; width 8, 1024
-// tiles of 1024 columns 6.8 / 6.4 / 6.8; f32 width 1, 532 tiles of 1024 columns 6.9 / 6.5 / 7.1, of
-// 2048 9.4 / 9.1 / 9.7).
+// width 8, 1024 tiles of 1024 columns 6.8 / 6.4 / 6.8; f32 width 1, 532 tiles of 1024 columns
+// 6.9 / 6.5 / 7.1, of 2048 9.4 / 9.1 / 9.7).
 static inline int pick_rt(int xt, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
     const bool light = xt != WX_F32 && W <= 4, medium = xt != WX_F32 && W <= 8;
-    if (K <= 2048 && n_tiles > 512 && n_tiles <= 1024) {
-        if (light || (medium && n_tiles <= 768))
-            return 1;
-        if (medium || (xt == WX_F32 && W <= 4 && n_tiles <= 768))
-            return 2;
-    }
+    if (light && (n_tiles <= 256 || n_tiles > 1024))
+        return 1;
+    if (light && n_tiles > 768)
+        return K <= 2048 ? 1 : K >= 6144 ? 4 : W <= 2 ? 1 : 2;
+    if (K <= 2048 && n_tiles > 512 && n_tiles <= 1024 && (medium ? n_tiles > 768 : xt == WX_F32 && W <= 4 && n_tiles <= 768))
+        return 2;
     if (n_tiles > 1024)
         return medium ? 1 : W * (xt == WX_F32 ? 4 : xt == WX_BF16 ? 2 : 1) <= 32 ? 2 : 4;
-    if (n_tiles <= 256 || (light && n_tiles <= 512) || (medium && n_tiles > 512 && n_tiles <= 768))
+    if (light || n_tiles <= 256 || (medium && n_tiles > 512 && n_tiles <= 768))
         return 1;
     return n_tiles <= 512 ? 2 : 4;
 }
