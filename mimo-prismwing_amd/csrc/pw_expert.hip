@@ -11,7 +11,8 @@ namespace pw {
 // rows: f32 hidden, width 8 49.1 / 48.5 / 51.0, width 16 53.8 / 51.2 / 52.0, width 32
 // 71.5 / 62.2 / 64.5; codes, width 16 52.4 / 53.1 / 56.0, width 32 61.4 / 58.8 / 60.5; K = 2048 one
 // share is best at every width, 16.6 / 17.3 / 18.1 at width 32).
-// Up to 128 tiles follow the projections' rule, so the forward stays the same as its separate calls.
+// Up to 128 tiles follow the projections' rule, so that mode B's forward stays the same as its separate
+// calls, bit for bit.
 static uint32_t down_shares(bool codes, uint32_t W, uint32_t K, uint32_t n_tiles)
 {
     if (n_tiles <= 128)

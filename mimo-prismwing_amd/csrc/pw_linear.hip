@@ -73,6 +73,20 @@ uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles)
     return pays ? tile_shares(n_tiles) : 1u;
 }
 
+// Sixteen waves a workgroup instead of eight. With one tile a CU a wave of eight computes four blocks one
+// after another at K = 4096, two of them in flight, and splitting f32 rows into planes costs most of a
+// block; sixteen waves have two blocks each. For up to four f32 rows, and for one or two bf16 ones of 8192
+// columns, where a wave has whole pairs of blocks (us, eight / sixteen waves, weights in the memory-side
+// cache | from HBM: 2048 x 4096, one f32 row 6.0 / 5.8 | 7.5 / 6.6; 4096 x 4096, four f32 rows
+// 6.5 / 6.2 | 8.1 / 7.7; 3000 x 8192, one f32 row 9.6 / 9.3 | 11.7 / 10.7, one bf16 row 7.2 / 7.3 |
+// 9.4 / 8.6; 3000 x 5120, one f32 row 6.8 / 7.2 | 8.7 / 8.7, 1000 x 6144 7.1 / 7.4 | 7.9 / 7.7; 2048 x 4096,
+// one bf16 row 4.8 / 4.9 | 6.1 / 6.1).
+static bool sixteen_waves(WideX xt, uint32_t W, uint32_t K, uint32_t KS, uint32_t n_tiles)
+{
+    return n_tiles <= 256 && K % (KS * 4096) == 0 &&
+           (xt == WX_F32 ? W <= 4 : xt == WX_BF16 && W <= 2 && K / KS >= 8192);
+}
+
 void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
                    uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
 {
@@ -92,7 +106,12 @@ void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void
     const int rt = pick_rt(xt, W, K, n_tiles);
     const int t = timer_begin(xt == WX_CODES ? K_LINEAR_B : K_LINEAR_A, stream);
     const bool aligned = ((uintptr_t)x & 15) == 0;
-    if (xt == WX_F32 && !aligned)
+    if (rt == 1 && sixteen_waves(xt, W, K, args.KS, n_tiles)) {
+        if (aligned)
+            launch_wide_16<WK_PROJ, true>(xt, args, stream);
+        else
+            launch_wide_16<WK_PROJ, false>(xt, args, stream);
+    } else if (xt == WX_F32 && !aligned)
         launch_wide_unaligned<WK_PROJ, WX_F32>(args, rt, stream);
     else if (xt == WX_BF16 && !aligned)
         launch_wide_unaligned<WK_PROJ, WX_BF16>(args, rt, stream);

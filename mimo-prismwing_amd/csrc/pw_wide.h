@@ -30,7 +30,7 @@ struct WideXBytes {
     static constexpr int value = XT == WX_F32 ? 4 : XT == WX_BF16 ? 2 : 1;
 };
 
-constexpr int WAVES = 8;  // of a workgroup; they split its share of K
+constexpr int WAVES = 8;  // of a workgroup (but launch_wide_16's); they split its share of K
 
 // Columns per step: a block, or half a block where two steps of all waves would take more than 128 KB
 // of LDS (24 f32 rows and eight waves: 196 KB with whole blocks).
@@ -107,7 +107,7 @@ __device__ __forceinline__ void lds_read(const uint32_t (&a)[4], u32x4 (&v)[4])
                  : "memory");
 }
 
-template <int KIND, int XT, int XR, int RT>
+template <int KIND, int XT, int XR, int RT, int WV>
 struct WideStream {
     static constexpr int SC = WideStep<XT, XR>::value;
     static constexpr int XB = WideXBytes<XT>::value;
@@ -117,8 +117,8 @@ struct WideStream {
     static constexpr int WB = KIND == WK_BF16 ? 2 : 1;    // bytes of a weight
     static constexpr int WL = SC * WB / 64;               // weight loads per tile and step
     static constexpr int SLOT = XR * UPR;                 // units per step slot
-    static constexpr int RED = WAVES * RT * NT * 64;          // split partials, in the slots' place
-    static constexpr int LDS = 2 * WAVES * SLOT > RED ? 2 * WAVES * SLOT : RED;
+    static constexpr int RED = WV * RT * NT * 64;         // split partials, in the slots' place
+    static constexpr int LDS = 2 * WV * SLOT > RED ? 2 * WV * SLOT : RED;
     static_assert(XR * UPR % 64 == 0, "whole copies");
     static_assert(LDS * 16 <= 160 * 1024, "a workgroup's LDS");
 
@@ -144,12 +144,12 @@ struct WideStream {
 // through registers while its weights are on their way, so they need no aligned copy in memory (us,
 // aligned / off 16 bytes / with a copy launch before it: 13568 x 4096, 8 f32 rows 15.6 / 16.0 / 17.6, 32
 // 22.1 / 22.3 / 24.2, 8 bf16 rows 13.7 / 14.2 / 15.8, 32 16.7 / 21.5 / 19.2).
-template <int KIND, int XT, int XR, int RT, bool AL = true>
-__global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
+template <int KIND, int XT, int XR, int RT, bool AL = true, int WV = WAVES>
+__global__ __launch_bounds__(64 * WV, WV / 4) void wide_kernel(const WideArgs args)
 {
-    using S = WideStream<KIND, XT, XR, RT>;
+    using S = WideStream<KIND, XT, XR, RT, WV>;
     constexpr int NT = S::NT, SC = S::SC, WL = S::WL, XC = S::XC;
-    __shared__ uint4 lds_w[S::LDS];  // per wave two step slots; then the split partials [WAVES][RT * NT][64]
+    __shared__ uint4 lds_w[S::LDS];  // per wave two step slots; then the split partials [WV][RT * NT][64]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, r16 = lane & 15;
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
         c0 = share * blocks / args.KS;
         cn = (share + 1) * blocks / args.KS - c0;
     }
-    const uint32_t b0 = c0 + (uint32_t)wave * cn / WAVES, b1 = c0 + ((uint32_t)wave + 1) * cn / WAVES;
+    const uint32_t b0 = c0 + (uint32_t)wave * cn / WV, b1 = c0 + ((uint32_t)wave + 1) * cn / WV;
     const uint32_t steps = (b1 - b0) * (128 / SC);
 
     f32x4 total[RT][NT], acc[RT][NT];
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideArgs args)
         return;
     f32x4 sum = red[wave * 64 + lane];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) {
+    for (int w = 1; w < WV; ++w) {
         const f32x4 o = red[(w * RT * NT + wave) * 64 + lane];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -582,6 +582,17 @@ static void launch_wide(const WideArgs &args, int rt, hipStream_t stream)
         launch_wide_rt<KIND, XT, XT == WX_F32 ? 24 : 32>(args, rt, stream);
     else
         launch_wide_rt<KIND, XT, 32>(args, rt, stream);
+}
+
+// One tile of up to four rows on sixteen waves.
+template <int KIND, bool AL>
+static void launch_wide_16(int xt, const WideArgs &args, hipStream_t stream)
+{
+    const dim3 grid = wide_grid<KIND>(args, 1), block(1024);
+    if (xt == WX_F32)
+        hipLaunchKernelGGL((wide_kernel<KIND, WX_F32, 4, 1, AL, 16>), grid, block, 0, stream, args);
+    else
+        hipLaunchKernelGGL((wide_kernel<KIND, WX_BF16, 4, 1, AL, 16>), grid, block, 0, stream, args);
 }
 
 // Rows off 16 bytes: eight, sixteen or 32 staged rows, one or four tiles.

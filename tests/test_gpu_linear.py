@@ -119,12 +119,13 @@ def test_mode_a_f32_row_split_in_staging(rt, n, k):
 
 
 @pytest.mark.parametrize("n,k", [(n, k) for n in (24, 4104, 8200, 12296) for k in (128, 1152, 3328)] +
-                         [(1000, 8192), (2000, 6144)])
+                         [(1000, 8192), (2000, 6144), (24, 4096), (4096, 4096), (2100, 8192), (2040, 8192), (16376, 4096)])
 def test_projection_tile_and_step_edges(rt, n, k):
     """Every staged-row count (4, 8, 16, 24, 32 rows and one off each), workgroups of one, two and
     four 16-row tiles with a partial last tile and a partial last workgroup, and waves with no, one,
-    two, three and four steps (1, 9 and 26 blocks over eight waves), and K in four and two shares (the last
-    two shapes, by the rows' type and number). Mode A against 64 bits: exact
+    two, three and four steps (1, 9 and 26 blocks over eight waves), K in four and two shares (1000 x 8192,
+    2000 x 6144, by the rows' type and number), sixteen waves of two and four steps for up to four
+    f32 rows (one share; 2040 x 8192 two), and 1024 tiles by the rows' number. Mode A against 64 bits: exact
     products added in f32 in chains of at most 48 roundings (2e-6). Mode B on integers whose sums are
     exact in f32 (weights up to 2, codes up to 8 with one 448 a group, so activation scales are 1,
     block scales powers of two): equal."""
@@ -219,10 +220,10 @@ def test_mode_a_rows_off_16_bytes(rt, kind):
 
 
 @pytest.mark.parametrize("kind", ["f32", "bf16"])
-@pytest.mark.parametrize("n,k", [(4104, 1152), (1000, 8192)])
+@pytest.mark.parametrize("n,k", [(4104, 1152), (1000, 8192), (2100, 8192)])
 def test_mode_a_rows_off_16_bytes_edges(rt, kind, n, k):
-    """The same with four tiles a workgroup (a partial last one) and in four K shares, up to eight
-    rows and more, starting one and three values off."""
+    """The same with four tiles a workgroup (a partial last one), in four K shares and on sixteen waves, up
+    to eight rows and more, starting one and three values off."""
     torch = _torch()
     rng = np.random.default_rng(77)
     s = log_uniform_scales(rng, n, k)
