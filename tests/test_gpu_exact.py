@@ -500,7 +500,7 @@ def test_mode_a_hidden_through_identity_down(rt, hidden, inter, rows):
     (g / (1 + e^-g)) * u unrounded: the three bf16 planes must carry it exactly. Gate/up sums are
     exact (e4m3 activations and weights in [1, 2), power-of-two scales), so the only difference
     from the oracle is the exp (a few f32 steps); dropping the lowest plane moves values by up to
-    2^-16 relative. Hidden 4096 takes the whole-K fused gate/up kernel, 256 the split-K one."""
+    2^-16 relative (the streaming kernel splits the f32 hidden rows into them)."""
     torch = _torch()
     rng = np.random.default_rng(hidden + rows)
     gw, uw = _unit_codes(rng, (inter, hidden), 0.3), _unit_codes(rng, (inter, hidden), 0.3)

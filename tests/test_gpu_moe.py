@@ -265,66 +265,74 @@ def test_decode_layer_is_deterministic(rt, full_bank):
 
 
 def test_whole_k_gateup_matches_split_k(rt, full_bank):
-    """At hidden 4096 a batch of up to 8 bf16 rows takes the whole-K gate/up kernel (SwiGLU fused, no
-    split partials in memory); 9 rows take the split-K kernel plus the SwiGLU kernel. Each token's
-    result depends only on its own row and routes, and both paths add the same eight K-split sums
-    in the same order, so the first 8 rows of a 9-row batch equal the 8-row batch bit for bit."""
+    """At hidden 4096 entries of up to three f32 rows take the whole-K gate/up kernel (SwiGLU fused, no
+    split partials in memory); ten rows over 32 experts run on entries of eight, which take the split-K
+    kernel plus the SwiGLU kernel. Each token's result depends only on its own row and routes, and both
+    paths add the same eight K-split sums in the same order, so pairs of rows, whose experts have at most
+    two, equal the ten-row batch bit for bit; that batch against the oracle."""
     import torch
-    x = WL.activations(9, WL.SEED_BASE + 80)
-    rw, bias = WL.router_inputs(WL.SEED_BASE + 3)
-    _, _, sel, w, _ = O.route(x, rw, bias)
+    n, rows = 32, 10
+    bank = rt.expert_bank(*[full_bank.projections[i:3 * n:3] for i in range(3)])
+    x = np.random.default_rng(80).standard_normal((rows, 4096)).astype(np.float32)
+    sel, w = random_routes(np.random.default_rng(81), rows, n)
     stream = torch.cuda.current_stream().cuda_stream
-    outs = []
-    for rows in (8, 9):
-        xt = torch.from_numpy(WL.bf16_bits_np(x[:rows]).view(np.int16)).cuda()
-        ids = torch.from_numpy(sel[:rows].astype(np.int32)).cuda()
-        wts = torch.from_numpy(w[:rows]).cuda()
-        raw = torch.empty((rows, 4096), dtype=torch.float32, device="cuda")
-        rt.moe_layer_device(full_bank.bank, xt, rows, ids, wts, raw, mode=P.MODE_A, out_dtype=P.DTYPE_F32_RAW,
-                            stream=stream)
+
+    def layer(at):
+        ids, wts = torch.from_numpy(sel[at].astype(np.int32)).cuda(), torch.from_numpy(w[at]).cuda()
+        raw = torch.empty((len(at), 4096), dtype=torch.float32, device="cuda")
+        rt.moe_layer_device(bank, torch.from_numpy(x[at]).cuda(), len(at), ids, wts, raw, mode=P.MODE_A,
+                            x_dtype=P.DTYPE_F32, out_dtype=P.DTYPE_F32_RAW, stream=stream)
         torch.cuda.synchronize()
         assert rt.take_flags() == 0
-        outs.append(raw.cpu().numpy())
-    assert np.array_equal(outs[0].view(np.uint32), outs[1][:8].view(np.uint32))
-    used = sorted(set(sel.reshape(-1).tolist()))
-    experts = {e: full_bank.expert_host(e) for e in used}
-    _, ref_raw = O.moe_layer("a", x, experts, 256, sel, w, raw=True)
-    check_mode_a(outs[1], ref_raw, moe_condition(x, experts, sel, w), raw=True)
+        return raw.cpu().numpy()
+
+    whole = layer(np.arange(rows))
+    for p in range(0, rows, 2):
+        at = np.array([p, p + 1])
+        assert np.array_equal(layer(at).view(np.uint32), whole[at].view(np.uint32)), p
+    experts = {e: full_bank.expert_host(e) for e in sorted(set(sel.reshape(-1).tolist()))}
+    _, ref_raw = O.moe_layer("a", x, experts, n, sel, w, raw=True)
+    check_mode_a(whole, ref_raw, moe_condition(x, experts, sel, w), raw=True)
 
 
 @pytest.mark.parametrize("width", [5, 6, 8])
 def test_pieces_match_one_workgroup_schedule(rt, full_bank, width):
-    """A decode batch of 5 to 8 rows runs both projections on pieces of at most four slots of an
-    expert (its one-wave schedule cuts them). With every token on the same eight experts (width
-    slots each: pieces of 4 + 1, 4 + 2, 4 + 4), the first rows of a 9-row batch (one-workgroup
-    schedule, no pieces) equal the smaller batch bit for bit."""
+    """A decode batch of 5 to 8 bf16 rows over many experts runs both projections on pieces of at most four
+    slots of an expert (its one-wave schedule cuts them), one of nine on pieces of six (its one-workgroup
+    schedule), one of two on none. With every token on the same eight experts (width slots each: pieces of
+    4 + 1, 4 + 2, 4 + 4; nine rows 6 + 3), the batches agree bit for
+    bit."""
     import torch
     x = WL.activations(9, WL.SEED_BASE + 130)
     sel = np.tile(np.array([17, 3, 250, 99, 128, 64, 5, 200], np.uint32), (9, 1))
     w = np.random.default_rng(5).uniform(0.01, 0.3, (9, 8)).astype(np.float32)
     stream = torch.cuda.current_stream().cuda_stream
-    outs = []
-    for rows in (width, 9):
-        xt = torch.from_numpy(WL.bf16_bits_np(x[:rows]).view(np.int16)).cuda()
-        ids = torch.from_numpy(sel[:rows].astype(np.int32)).cuda()
-        wts = torch.from_numpy(w[:rows]).cuda()
-        raw = torch.empty((rows, 4096), dtype=torch.float32, device="cuda")
-        rt.moe_layer_device(full_bank.bank, xt, rows, ids, wts, raw, mode=P.MODE_A, out_dtype=P.DTYPE_F32_RAW,
+
+    def layer(at):
+        xt = torch.from_numpy(WL.bf16_bits_np(x[at]).view(np.int16)).cuda()
+        ids, wts = torch.from_numpy(sel[at].astype(np.int32)).cuda(), torch.from_numpy(w[at]).cuda()
+        raw = torch.empty((len(at), 4096), dtype=torch.float32, device="cuda")
+        rt.moe_layer_device(full_bank.bank, xt, len(at), ids, wts, raw, mode=P.MODE_A, out_dtype=P.DTYPE_F32_RAW,
                             stream=stream)
         torch.cuda.synchronize()
         assert rt.take_flags() == 0
-        outs.append(raw.cpu().numpy())
-    assert np.array_equal(outs[0].view(np.uint32), outs[1][:width].view(np.uint32))
+        return raw.cpu().numpy()
+
+    out = layer(np.arange(width))
+    assert np.array_equal(out.view(np.uint32), layer(np.arange(9))[:width].view(np.uint32))
+    for p in range(width):
+        at = np.array([p, (p + 1) % width])
+        assert np.array_equal(layer(at).view(np.uint32), out[at].view(np.uint32)), p
     experts = {e: full_bank.expert_host(e) for e in sorted(set(sel.reshape(-1).tolist()))}
     _, ref_raw = O.moe_layer("a", x[:width], experts, 256, sel[:width], w[:width], raw=True)
-    check_mode_a(outs[0], ref_raw, moe_condition(x[:width], experts, sel[:width], w[:width]), raw=True)
+    check_mode_a(out, ref_raw, moe_condition(x[:width], experts, sel[:width], w[:width]), raw=True)
 
 
 @pytest.mark.parametrize("mode,x_f32", [(P.MODE_A, False), (P.MODE_A, True), (P.MODE_B, False)])
 @pytest.mark.parametrize("rows", [9, 17, 32])
 def test_wide_batch_pieces_equal_small_batches(rt, full_bank, mode, x_f32, rows):
-    """A batch of 9 to 32 rows runs the experts on pieces of their slots (three or four rows in mode A;
-    eight in mode B, for more than sixteen rows). Experts with every row (full pieces and a
+    """A batch of 9 to 32 rows over many experts runs them on pieces of their slots (three f32 or six bf16
+    rows in mode A; sixteen in mode B, for more than sixteen rows). Experts with every row (full pieces and a
     remainder), with some rows and with one: each row equals, bit for bit, its result in a two-row
     batch, whose experts need no pieces."""
     import torch
