@@ -87,26 +87,37 @@ _BINDING = np.dtype([("expert", "<u4"), ("count", "<u4"), ("positions", "<u8"), 
 assert _BINDING.itemsize == ctypes.sizeof(_abi.ExpertBindingC)
 
 
-def _flat_list(v):
-    return type(v) is list and (not v or isinstance(v[0], (int, float, np.generic)))
-
-
-def _expert_bindings(experts):
-    """The C bindings of a batch and what keeps their pointers alive. The positions and weights of all
-    bindings sit in one array each: an array and a pointer object per binding were most of the call's host time."""
+def _joined(experts, flat):
+    """Positions and weights of all bindings in one array each, and every binding's count and offsets.
+    flat: lists are taken to hold numbers; else every sequence goes through numpy by itself."""
     pos, weights, counts, pos_at, w_at = [], [], [], [], []
     for b in experts:
         p, w = b.positions, b.route_weights
-        if not _flat_list(p) or not _flat_list(w):  # any array-like
+        if not flat or type(p) is not list or type(w) is not list:  # any array-like
             p, w = np.ascontiguousarray(p, dtype=np.uint32), np.ascontiguousarray(w, dtype=np.float32)
         counts.append(len(p))
         pos_at.append(len(pos))
         w_at.append(len(weights))
         pos += p if type(p) is list else p.reshape(-1).tolist()
         weights += w if type(w) is list else w.reshape(-1).tolist()
-    pos, weights = np.array(pos, dtype=np.uint32), np.array(weights, dtype=np.float32)
+    return np.array(pos, dtype=np.uint32), np.array(weights, dtype=np.float32), counts, pos_at, w_at
+
+
+def _expert_bindings(experts):
+    """The C bindings of a batch and what keeps their pointers alive. The positions and weights of all
+    bindings sit in one array each: an array and a pointer object per binding were most of the call's host
+    time, and so is a look at every list's elements: nested lists show in the joined arrays."""
+    try:
+        pos, weights, counts, pos_at, w_at = _joined(experts, True)
+        flat = pos.ndim == 1 and weights.ndim == 1
+    except (TypeError, ValueError):
+        flat = False
+    if not flat:
+        pos, weights, counts, pos_at, w_at = _joined(experts, False)
+    ids = [b.expert for b in experts]
+    column = np.array(ids)
     rec = np.zeros(len(counts), _BINDING)
-    rec["expert"] = [operator.index(b.expert) & 0xFFFFFFFF for b in experts]
+    rec["expert"] = column if column.dtype.kind == "i" else [operator.index(e) & 0xFFFFFFFF for e in ids]
     rec["count"] = counts
     rec["positions"] = np.array(pos_at, np.uint64) * 4 + np.uint64(pos.ctypes.data)
     rec["route_weights"] = np.array(w_at, np.uint64) * 4 + np.uint64(weights.ctypes.data)

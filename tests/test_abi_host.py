@@ -218,5 +218,9 @@ def test_expert_bindings_take_any_integer_id_and_nested_rows():
            for c in (arr[i] for i in range(len(batch)))]
     assert got[:len(ids)] == [([i], [0.5]) for i in range(len(ids))]
     assert got[len(ids):] == [([4, 2], [0.25, 0.75]), ([6, 1], np.float32([0.1, 0.2]).tolist()), ([5], [0.125])]
-    with pytest.raises(TypeError):
-        _expert_bindings([bind(1.0, [0], [1.0])])
+    wide = _expert_bindings([bind(2 ** 33 + 7, [[1, 2], [3, 4]], [0.5, 0.25]), bind(3, [9], [1.0])])[0]
+    assert wide[0].expert == 7 and [wide[0].positions[j] for j in range(wide[0].count)] == [1, 2]
+    assert wide[1].positions[0] == 9
+    for bad in (1.0, "3", None):
+        with pytest.raises(TypeError):
+            _expert_bindings([bind(bad, [0], [1.0]), bind(2, [1], [1.0])])
