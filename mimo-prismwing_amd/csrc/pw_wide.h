@@ -4,12 +4,12 @@
 // What bounds it: the weights' bytes once, and beside them the activations, which every workgroup
 // reads again from L2. A workgroup of 16 weight rows reads W rows of activations for its 16 rows of
 // weights: at 13 f32 rows 52 bytes a column (78 as three bf16 planes) against 16. Here a workgroup
-// takes 16 RT weight rows over the whole K (pick_rt), its eight waves split K, and each wave streams
-// its blocks two steps deep with no barrier: the step's activation columns go by coalesced
-// direct-to-LDS copies to the wave's own LDS region, the step's weights to registers, and step
-// j + 2 is issued as soon as step j is computed. f32 rows are read as f32 and split in registers,
-// once per step for all RT tiles. The split sums meet in LDS and are added in split order 0..7, so
-// results are deterministic.
+// takes 16 RT weight rows over the whole K (pick_rt), its eight waves (launch_wide_16: sixteen) split K,
+// and each wave streams its blocks two steps deep with no barrier: the step's activation columns go by
+// coalesced direct-to-LDS copies to the wave's own LDS region, the step's weights to registers, and step
+// j + 2 is issued as soon as step j is computed. f32 rows are read as f32 and split in registers, once per
+// step for all RT tiles. The split sums meet in LDS and are added in split order, so results are
+// deterministic.
 //
 // Measured against one 16-row tile per workgroup with the activations read inside the MFMA loop (us,
 // weights in the memory-side cache): 13800 x 4096 (56.5 MB) with 13 f32 rows, mode A, 46.8 -> 15.7
