@@ -203,8 +203,9 @@ void launch_split_planes(const float *x, uint32_t n, uint16_t *planes, hipStream
 // with x_scales [W][K / 128] (mode B); partial: SHARE_SUM_BYTES.
 enum WideX : int { WX_BF16 = 0, WX_F32 = 1, WX_CODES = 2 };
 uint32_t linear_shares(WideX xt, uint32_t W, uint32_t K, uint32_t n_tiles);
-void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
-                   uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream);
+// Weights: a tile table, or without one (tiles null) the tensor w [N][K] with block scales s.
+void launch_linear(WideX xt, const uint8_t *w, const float *s, const ProjTile *tiles, uint32_t n_tiles, const void *x,
+                   const float *x_scales, uint32_t W, uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream);
 // One expert on W rows (pw_expert.hip). Gate/up with the SwiGLU: x [W][H] e4m3 codes with x_scales
 // (mode B, hidden bf16-staged), f32 or bf16 (mode A) -> hidden [W][I] f32. Down: x [W][I] codes or f32
 // -> the output rows [W][H] (raw: f32 sums unrounded), or with the K shares it returns above one the

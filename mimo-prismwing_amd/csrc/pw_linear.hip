@@ -87,10 +87,12 @@ static bool sixteen_waves(WideX xt, uint32_t W, uint32_t K, uint32_t KS, uint32_
            (xt == WX_F32 ? W <= 4 : xt == WX_BF16 && W <= 2 && K / KS >= 8192);
 }
 
-void launch_linear(WideX xt, const ProjTile *tiles, uint32_t n_tiles, const void *x, const float *x_scales, uint32_t W,
-                   uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
+void launch_linear(WideX xt, const uint8_t *w, const float *s, const ProjTile *tiles, uint32_t n_tiles, const void *x,
+                   const float *x_scales, uint32_t W, uint32_t K, float *partial, float *y32, uint16_t *y16, uint32_t N, uint32_t round_f32, hipStream_t stream)
 {
     WideArgs args{};
+    args.w0 = w;
+    args.s0 = s;
     args.tiles = tiles;
     args.n_tiles = n_tiles;
     args.partial = partial;

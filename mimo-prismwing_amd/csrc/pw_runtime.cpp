@@ -221,7 +221,7 @@ struct pw_projection {
     float *s = nullptr;         // device scale base
     bool owns = false;
     uint32_t rows = 0, columns = 0;
-    ProjTile *tiles = nullptr;  // device tile table
+    ProjTile *tiles = nullptr;  // device tile table; null: one tensor in its own row order
     uint32_t n_tiles = 0;
     uint64_t weight_bytes = 0, scale_bytes = 0;
 };
@@ -255,6 +255,9 @@ void add_segment_tiles(std::vector<ProjTile> &tiles, const uint8_t *w, const flo
         tiles.push_back(t);
     }
 }
+
+// Tiles of one tensor in its own row order: tile t is rows [16 t, 16 t + 16), with no table.
+uint32_t plain_tiles(uint32_t rows) { return rows / 16 + (rows % 16 != 0); }
 
 int upload_tiles(pw_projection *p, const std::vector<ProjTile> &tiles)
 {
@@ -759,10 +762,13 @@ int pw_projection_bind(pw_runtime *rt, const pw_projection_desc *d, int scan_cod
         pw_projection_release(p);
         return fail(PW_ERR_DEVICE, "weight upload failed: %s", hipGetErrorString(e));
     }
-    std::vector<ProjTile> tiles;
     if (d->layout == PW_LAYOUT_PLAIN) {
-        add_segment_tiles(tiles, p->w, p->s, cols, 0, rows, 0, 0);
-    } else if (d->layout == PW_LAYOUT_FULL_QKV_TP4) {
+        p->n_tiles = plain_tiles(rows);
+        *out = p;
+        return PW_OK;
+    }
+    std::vector<ProjTile> tiles;
+    if (d->layout == PW_LAYOUT_FULL_QKV_TP4) {
         // shards of [Q 3072 | K 192 | V 128], 27 scale rows each (24 Q, 2 K incl. a 64-row
         // partial block, 1 V); outputs deinterleaved as all Q, all K, all V
         for (uint32_t s = 0; s < 4; ++s) {
@@ -872,13 +878,7 @@ int pw_projection_bind_device(pw_runtime *rt, const void *weight, const float *s
     p->columns = columns;
     p->weight_bytes = (uint64_t)rows * columns;
     p->scale_bytes = (uint64_t)((rows + 127) / 128) * (columns / 128) * 4;
-    std::vector<ProjTile> tiles;
-    add_segment_tiles(tiles, p->w, p->s, columns, 0, rows, 0, 0);
-    int st = upload_tiles(p, tiles);
-    if (st != PW_OK) {
-        pw_projection_release(p);
-        return st;
-    }
+    p->n_tiles = plain_tiles(rows);
     *out = p;
     return PW_OK;
 }
@@ -918,14 +918,14 @@ static int enqueue_linear(pw_runtime *rt, uint32_t mode, const void *x, bool x_f
     const pw::WideX xt = mode == PW_MODE_B ? pw::WX_CODES : x_f32 ? pw::WX_F32 : pw::WX_BF16;
     float *partial = (float *)rt->share_sums.p;
     if (mode == PW_MODE_A) {
-        pw::launch_linear(xt, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, partial, y32, y16, p->rows, round_f32,
+        pw::launch_linear(xt, p->w, p->s, p->tiles, p->n_tiles, x, nullptr, rows, p->columns, partial, y32, y16, p->rows, round_f32,
                           stream);
     } else if (mode == PW_MODE_B) {
         PW_HIP(rt->codes.ensure((size_t)rows * p->columns));
         PW_HIP(rt->scales.ensure((size_t)rows * (p->columns / 128) * 4));
         pw::launch_quant_group128(x, x_f32, rows, p->columns, (uint8_t *)rt->codes.p,
                                   (float *)rt->scales.p, rt->d_flags, stream);
-        pw::launch_linear(xt, p->tiles, p->n_tiles, rt->codes.p, (const float *)rt->scales.p, rows, p->columns, partial,
+        pw::launch_linear(xt, p->w, p->s, p->tiles, p->n_tiles, rt->codes.p, (const float *)rt->scales.p, rows, p->columns, partial,
                           y32, y16, p->rows, round_f32, stream);
     } else {
         return fail(PW_ERR_ARGUMENT, "unknown mode %u", mode);

@@ -52,8 +52,8 @@ struct WideStep {
 enum WideKind : int { WK_PROJ = 0, WK_GATEUP = 1, WK_DOWN = 2, WK_BF16 = 3 };
 
 struct WideArgs {
-    const ProjTile *tiles;         // WK_PROJ
-    const uint8_t *w0, *w1;        // gate and up, down [N][K], or the bf16 weight's bytes
+    const ProjTile *tiles;         // WK_PROJ; null: the tensor w0 [N][K]
+    const uint8_t *w0, *w1;        // gate and up, down or a projection [N][K], or the bf16 weight's bytes
     const float *s0, *s1;          // ... and their block scales
     float *partial;                // with KS > 1: share sums [KS][W][N]
     uint32_t KS;                   // all but WK_GATEUP
@@ -162,7 +162,10 @@ __global__ __launch_bounds__(64 * WV, WV / 4) void wide_kernel(const WideArgs ar
     const uint32_t group = SHARES ? blockIdx.x / args.KS : blockIdx.x;
     const uint8_t *wrow[RT];
     const float *ws[RT];
-    if constexpr (KIND == WK_PROJ) {
+    // One tensor's tiles are formed from the arguments: a descriptor is a trip to memory of its own ahead of
+    // the first weight (weights from HBM, us, with / without: 2048 x 4096, one bf16 row 6.1 / 5.75,
+    // 13568 x 4096 14.0 / 13.6, one f32 row of 2048 x 4096 6.7 / 6.3).
+    if (KIND == WK_PROJ && args.tiles) {
         // the tiles' descriptors in one round trip: all of them are taken before any address is formed
         const uint8_t *wt[RT];
         uint32_t valid[RT];
@@ -190,8 +193,9 @@ __global__ __launch_bounds__(64 * WV, WV / 4) void wide_kernel(const WideArgs ar
             } else if constexpr (KIND == WK_GATEUP) {
                 wrow[r] = (r16 < 8 ? args.w0 : args.w1) + (size_t)(t * 8 + (r16 & 7)) * K + q * WQ;
                 ws[r] = (q < 2 ? args.s0 : args.s1) + (size_t)(t * 8 >> 7) * blocks;
-            } else {
-                wrow[r] = args.w0 + (size_t)(t * 16 + r16) * K + q * WQ;
+            } else {  // (a projection's last tile may be partial: its rows repeat the last one, never stored)
+                const uint32_t row = t * 16 + r16;
+                wrow[r] = args.w0 + (size_t)(KIND != WK_PROJ || row < args.N ? row : args.N - 1) * K + q * WQ;
                 ws[r] = args.s0 + (size_t)(t * 16 >> 7) * blocks;
             }
         }
@@ -427,13 +431,14 @@ __global__ __launch_bounds__(64 * WV, WV / 4) void wide_kernel(const WideArgs ar
     if constexpr (KIND == WK_PROJ) {
         if (token >= W)
             return;
-        const ProjTile tile = args.tiles[t];
+        const uint32_t out_row = args.tiles ? args.tiles[t].out_row : t * 16;
+        const uint32_t valid = args.tiles ? args.tiles[t].valid : args.N - t * 16;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t row = q * 4 + i;
-            if (row >= tile.valid)
+            if (row >= valid)
                 continue;
-            const size_t at = (size_t)token * args.N + tile.out_row + row;
+            const size_t at = (size_t)token * args.N + out_row + row;
             if (args.KS > 1) {
                 args.partial[(size_t)(blockIdx.x % args.KS) * W * args.N + at] = sum[i];
                 continue;
